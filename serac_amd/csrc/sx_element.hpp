@@ -4,7 +4,7 @@
 // one workgroup-resident pass:
 //   gather L -> LDS                           (fn/element_restriction.cpp:443-454)
 //   sum-factorized interpolate (3 stages)     (fn/detail/hexahedron_H1.inl:169-228)
-//   quadrature point: qfunction + parent/physical maps (+ dual tangents)
+//   quadrature point: qfunction + parent/physical maps (+ its closed-form tangent)
 //                     or stored-tangent chain rule for J.v
 //   sum-factorized integrate (3 stages)       (fn/detail/hexahedron_H1.inl:230-280)
 //   scatter-add LDS -> L                      (fn/element_restriction.cpp:456-467)
@@ -261,6 +261,21 @@ __device__ __forceinline__ void trilinear_jacobian(const double* X, double x0, d
   }
 }
 
+// The value v as the compiler cannot connect it with its origin: what is
+// computed from it afterwards is not merged with earlier expressions.
+__device__ __forceinline__ void opaque(double& v) { asm volatile("" : "+v"(v)); }
+
+// grad_x = grad_xi inv(J)
+template <int NC>
+__device__ __forceinline__ void physical_gradient(const double* gp, const double* Ji, double* g)
+{
+#pragma unroll
+  for (int c = 0; c < NC; c++)
+#pragma unroll
+    for (int k = 0; k < 3; k++)
+      g[c * 3 + k] = gp[c * 3 + 0] * Ji[0 * 3 + k] + gp[c * 3 + 1] * Ji[1 * 3 + k] + gp[c * 3 + 2] * Ji[2 * 3 + k];
+}
+
 // Quadrature-point stage of the residual / linearization: parent-space
 // (value, grad) in, parent-space (source, flux) out, following
 // fn/finite_element.hpp:246-322: grad_x = grad_xi inv(J); source *= detJ;
@@ -270,11 +285,7 @@ __device__ __forceinline__ void qpoint_eval(const double* prm, const double* Ji,
                                             const double* gp, double* src, double* fp, double* st)
 {
   double g[3 * NC], s[NC], f[3 * NC];
-#pragma unroll
-  for (int c = 0; c < NC; c++)
-#pragma unroll
-    for (int k = 0; k < 3; k++)
-      g[c * 3 + k] = gp[c * 3 + 0] * Ji[0 * 3 + k] + gp[c * 3 + 1] * Ji[1 * 3 + k] + gp[c * 3 + 2] * Ji[2 * 3 + k];
+  physical_gradient<NC>(gp, Ji, g);
 #pragma unroll
   for (int c = 0; c < NC; c++) s[c] = 0.0;
   if constexpr (QF::STATE > 0)
@@ -288,53 +299,6 @@ __device__ __forceinline__ void qpoint_eval(const double* prm, const double* Ji,
     for (int j = 0; j < 3; j++)
       fp[c * 3 + j] = (f[c * 3 + 0] * Ji[j * 3 + 0] + f[c * 3 + 1] * Ji[j * 3 + 1] + f[c * 3 + 2] * Ji[j * 3 + 2]) * dJ;
   }
-}
-
-// One forward-mode pass seeded at input s (the inputs are [value(NC)] then
-// [parent grad (NC x 3)] when FULL, else only the parent grad); returns the
-// derivative of [source(NC)] [parent flux (NC x 3)] (or only the flux).
-template <class QF, int NC, bool FULL>
-__device__ __forceinline__ void qpoint_tangent_column(const double* prm, const double* Ji, double dJ,
-                                                      const double* val, const double* gp, const double* st0,
-                                                      int s, double* col)
-{
-  constexpr int VOFF = FULL ? NC : 0;
-  d1            v[NC], g[3 * NC], sr[NC], f[3 * NC];
-#pragma unroll
-  for (int c = 0; c < NC; c++) v[c] = d1(val[c], (FULL && s == c) ? 1.0 : 0.0);
-#pragma unroll
-  for (int c = 0; c < NC; c++)
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-      double gv = gp[c * 3 + 0] * Ji[0 * 3 + k] + gp[c * 3 + 1] * Ji[1 * 3 + k] + gp[c * 3 + 2] * Ji[2 * 3 + k];
-      // seeded parent-gradient entry (c, j) contributes Ji[j][k] to d grad_x(c, k)
-      double gd = 0.0;
-#pragma unroll
-      for (int j = 0; j < 3; j++)
-        if (s == VOFF + c * 3 + j) gd = Ji[j * 3 + k];
-      g[c * 3 + k] = d1(gv, gd);
-    }
-#pragma unroll
-  for (int c = 0; c < NC; c++) sr[c] = d1(0.0);
-  if constexpr (QF::STATE > 0) {
-    // every pass starts from the point's state before this evaluation
-    double st[QF::STATE];
-#pragma unroll
-    for (int k = 0; k < QF::STATE; k++) st[k] = st0[k];
-    QF::eval(prm, v, g, sr, f, st);
-  } else {
-    QF::eval(prm, v, g, sr, f);
-  }
-  if constexpr (FULL) {
-#pragma unroll
-    for (int c = 0; c < NC; c++) col[c] = sr[c].d * dJ;
-  }
-#pragma unroll
-  for (int c = 0; c < NC; c++)
-#pragma unroll
-    for (int j = 0; j < 3; j++)
-      col[VOFF + c * 3 + j] =
-          (f[c * 3 + 0].d * Ji[j * 3 + 0] + f[c * 3 + 1].d * Ji[j * 3 + 1] + f[c * 3 + 2].d * Ji[j * 3 + 2]) * dJ;
 }
 
 // Directional derivative of the quadrature-point stage with respect to the
@@ -499,8 +463,16 @@ __device__ __forceinline__ void store_tangent_entry(void* base, int q, int k, do
 // ---------------------------------------------------------------------------
 // residual (MODE_RESIDUAL) and linearization (MODE_LINEARIZE, tangent in S)
 // ---------------------------------------------------------------------------
+// Waves per SIMD the register allocation aims at: the J2 linearization would
+// take 278 registers (one wave); held to two waves it spills nothing.
+template <int MODE, class QF>
+constexpr int element_waves()
+{
+  return MODE == MODE_LINEARIZE && QF::STATE > 0 ? 2 : 1;
+}
+
 template <int N, int NC, int MODE, class QF, int LAYOUT, typename S>
-__global__ void __launch_bounds__(256) k_element(const ElemLaunch P)
+__global__ void __launch_bounds__(256, (element_waves<MODE, QF>())) k_element(const ElemLaunch P)
 {
   constexpr int  NQ      = N * N * N;
   constexpr int  EB      = 256 / NQ;
@@ -709,17 +681,19 @@ __global__ void __launch_bounds__(256) k_element(const ElemLaunch P)
       qpoint_shape_dir<QF, NC>(P.params, J, dgps, val, gp, st, src, fp);
     } else {
     if constexpr (MODE == MODE_LINEARIZE) {
-      // columns s = 0..M-1 give entries idx(r, s), r < rows(s), in increasing
-      // storage order; every column starts from the state before this call
-      void*                          Dp = static_cast<char*>(P.D) + size_t(slot) * Lay::stride * sizeof(S);
+      // the entries come in increasing storage order; the state is the one before this call
+      void*                        Dp = static_cast<char*>(P.D) + size_t(slot) * Lay::stride * sizeof(S);
       typename StoreTraits<S>::raw pend[Lay::VEC];
+      double                       g[3 * NC];
+      physical_gradient<NC>(gp, Ji, g);
+      QF::tangent(P.params, g, Ji, dJ, st, [&](int rr, int s, double v) {
+        store_tangent_entry<S, DS, NQ>(Dp, li, Shape::idx(rr, s), v, pend);
+      });
+      if constexpr (NST > 0) {
+        // eval() below starts over from its inputs: sharing the trial state with the tangent kept it in registers
+        // across all 81 entries
 #pragma unroll
-      for (int s = 0; s < M; s++) {
-        double col[M];
-        qpoint_tangent_column<QF, NC, FULL>(P.params, Ji, dJ, val, gp, st, s, col);
-#pragma unroll
-        for (int rr = 0; rr < Shape::rows(s); rr++)
-          store_tangent_entry<S, DS, NQ>(Dp, li, Shape::idx(rr, s), col[rr], pend);
+        for (int k = 0; k < 3 * NC; k++) opaque(gp[k]);
       }
     }
     qpoint_eval<QF, NC>(P.params, Ji, dJ, val, gp, src, fp, st);
