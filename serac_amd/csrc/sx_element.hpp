@@ -1370,27 +1370,45 @@ __global__ void __launch_bounds__(256) k_diagonal(const ElemLaunch P)
 // fn/domain_integral_kernels.hpp:327-361, and Gradient::assemble,
 // fn/functional.hpp:569-667, which scatters K_e through lookup tables):
 //   K_e[(c,i)][(c',j)] = sum_q [w phi_i, w grad phi_i]_c . D(q) . [phi_j, grad phi_j]_c'
-// One workgroup per element: the element's tangent is staged in LDS as FP64
-// ([q][DS]), lane i owns test node i and loops over trial nodes j and
-// quadrature points; each entry is added at its CSR position, found by binary
-// search in the row's sorted columns.  Plain read-modify-write when the launch
-// covers one element colour (deterministic), atomics otherwise.
-template <int N, int NC, int LAYOUT, typename S, bool STAGE>
-__global__ void __launch_bounds__(128) k_assemble(const ElemLaunch P)
-{
-  constexpr int NQ = N * N * N;
-  using Shape      = TanShape<LAYOUT, NC>;
-  constexpr bool VAL = Shape::VAL;
-  constexpr int  DS  = Shape::DS;
-  constexpr int  VO  = Shape::VO;
-  constexpr int  TAB = 4 * N * N + N;
-  using Lay          = TangentLayout<S, DS, NQ>;
-  __shared__ double stab[TAB];
-  extern __shared__ double sD[];  // [q][DS]
+// For each pair (c, c') this is a product of an NQ x (slots NQ) matrix of test
+// functions with an (slots NQ) x NQ matrix of D times the trial functions, so
+// it runs on the FP64 matrix cores: a wave owns a 16 x 16 tile of node pairs
+// for every (c, c'), and each mfma_f64_16x16x4 takes four points for one slot
+// (lane l: test node l % 16, trial node l % 16, point l / 16 of the four).
+// Both factors are formed in registers from the 1D tables and the point's
+// tangent entries (staged in LDS where they fit in 48 KB, which leaves one
+// wait on memory per element instead of one per four points); the test factor serves all c', the trial factor all c.
+// The lane's results (nodes 4 r + l / 16 by l % 16) are added at their CSR
+// positions: a row holds NC columns per neighbour node, so one binary search
+// per node pair over the neighbours gives the positions of all NC x NC
+// entries.  Plain read-modify-write when the launch covers one element colour
+// (deterministic), atomics otherwise.
+// Neo-Hookean p = 2 on 14x12x13 elements: eight colour launches of 1008 us each
+// with one lane per test node looping over trial nodes and points (and a
+// search per entry) before, 36 us each now (a wave and the waits of one element).
+template <int N>
+struct AssembleTiles {
+  static constexpr int T      = (N * N * N + 15) / 16;           // tiles per direction of the node pairs
+  static constexpr int WAVES  = T * T < 4 ? T * T : 4;           // waves (tiles) per workgroup
+  static constexpr int GROUPS = (T * T + WAVES - 1) / WAVES;     // workgroups per element
+};
 
-  const int     li   = threadIdx.x;
-  const int64_t slot = P.slot_begin + blockIdx.x;
-  for (int k = li; k < TAB; k += blockDim.x) stab[k] = P.tables[k];
+template <int N, int NC, int LAYOUT, typename S, bool STAGE>
+__global__ void __launch_bounds__(64 * AssembleTiles<N>::WAVES, 2) k_assemble(const ElemLaunch P)
+{
+  typedef double d4 __attribute__((ext_vector_type(4)));
+  constexpr int  NQ = N * N * N;
+  using Shape       = TanShape<LAYOUT, NC>;
+  using Tiles       = AssembleTiles<N>;
+  using Lay         = TangentLayout<S, Shape::DS, NQ>;
+  constexpr bool VAL = Shape::VAL;
+  constexpr int  NS  = VAL ? 4 : 3;  // slots per component: [value], gradient
+  constexpr int  TAB = 4 * N * N;
+  constexpr int  DS  = Shape::DS;
+  __shared__ double        stab[TAB];
+  extern __shared__ double sD[];  // [q][DS]
+  const int64_t slot = P.slot_begin + blockIdx.x / Tiles::GROUPS;
+
   using raw       = typename StoreTraits<S>::raw;
   const raw* Dsrc = reinterpret_cast<const raw*>(static_cast<const char*>(P.D) + size_t(slot) * Lay::stride * sizeof(S));
   auto       Dat  = [&](int k, int q) -> double {
@@ -1400,78 +1418,127 @@ __global__ void __launch_bounds__(128) k_assemble(const ElemLaunch P)
     else
       return double(v);
   };
-  if constexpr (STAGE)
-    for (int t = li; t < NQ * DS; t += blockDim.x) sD[t] = Dat(t % DS, t / DS);
+  if constexpr (STAGE) {
+    // group by group, a group's points side by side in memory
+#pragma unroll 4
+    for (int t = threadIdx.x; t < NQ * DS; t += blockDim.x) {
+      constexpr int V  = Lay::VEC;
+      const int     gq = t / V, k = t < Lay::G * V * NQ ? (gq / NQ) * V + t % V : Lay::G * V + (t - Lay::G * V * NQ) / NQ;
+      const int     q  = t < Lay::G * V * NQ ? gq % NQ : (t - Lay::G * V * NQ) % NQ;
+      sD[q * DS + k]   = Dat(k, q);
+    }
+  }
+  for (int k = threadIdx.x; k < TAB; k += blockDim.x) stab[k] = P.tables[k];
   __syncthreads();
-  if (li >= NQ) return;
-  const double* tB  = stab;
-  const double* tG  = stab + N * N;
-  const double* tBw = stab + 2 * N * N;
-  const double* tGw = stab + 3 * N * N;
-  const int     ix = li % N, iy = (li / N) % N, iz = li / (N * N);
-  const int64_t node_i = P.map[size_t(slot) * NQ + li];
 
-  for (int jn = 0; jn < NQ; jn++) {
-    const int jx = jn % N, jy = (jn / N) % N, jz = jn / (N * N);
-    double    acc[NC][NC];
+  const int     tile = int(blockIdx.x % Tiles::GROUPS) * Tiles::WAVES + int(threadIdx.x >> 6);
+  if (tile >= Tiles::T * Tiles::T) return;
+  const int l  = threadIdx.x & 63;
+  const int i  = (tile / Tiles::T) * 16 + (l & 15);  // the lane's test node in the products
+  const int j  = (tile % Tiles::T) * 16 + (l & 15);  // its trial node, there and in the results
+  const int ic = i < NQ ? i : 0, jc = j < NQ ? j : 0;  // rows and columns past the nodes are computed and dropped
+
+  // values and gradient of node n's function at point q from the tables b, g
+  auto basis = [&](const double* b, const double* g, int n, int q, double* out) {
+    const int    x = n % N, y = (n / N) % N, z = n / (N * N), qx = q % N, qy = (q / N) % N, qz = q / (N * N);
+    const double bx = b[qx * N + x], by = b[qy * N + y], bz = b[qz * N + z];
+    if constexpr (VAL) out[0] = bx * by * bz;
+    out[NS - 3] = g[qx * N + x] * by * bz;
+    out[NS - 2] = bx * g[qy * N + y] * bz;
+    out[NS - 1] = bx * by * g[qz * N + z];
+  };
+  d4 acc[NC][NC];
+#pragma unroll
+  for (int c = 0; c < NC; c++)
+#pragma unroll
+    for (int c2 = 0; c2 < NC; c2++) acc[c][c2] = d4{0.0, 0.0, 0.0, 0.0};
+
+  for (int q0 = 0; q0 < NQ; q0 += 4) {
+    const int q  = q0 + (l >> 4);
+    const int qc = q < NQ ? q : 0;
+    double    tf[NS], uf[NS];
+    basis(stab + 2 * N * N, stab + 3 * N * N, ic, qc, tf);
+    basis(stab, stab + N * N, jc, qc, uf);
+    if (q >= NQ) {  // no such point: its products vanish whatever the tangent read in its place holds
+#pragma unroll
+      for (int a = 0; a < NS; a++) tf[a] = uf[a] = 0.0;
+    }
+    auto D = [&](int row, int col) -> double {
+      if constexpr (STAGE)
+        return sD[qc * DS + Shape::idx(row, col)];
+      else
+        return Dat(Shape::idx(row, col), qc);
+    };
+    // input / output number of slot a of component c
+    auto slot_of = [](int c, int a) { return VAL ? (a == 0 ? c : NC + c * 3 + a - 1) : c * 3 + a; };
 #pragma unroll
     for (int c = 0; c < NC; c++)
 #pragma unroll
-      for (int c2 = 0; c2 < NC; c2++) acc[c][c2] = 0.0;
-    for (int q = 0; q < NQ; q++) {
-      const int qx = q % N, qy = (q / N) % N, qz = q / (N * N);
-      // tangent entries of point q: staged in LDS, or read through the caches
-      auto Dq = [&](int k) -> double {
-        if constexpr (STAGE)
-          return sD[q * DS + k];
-        else
-          return Dat(k, q);
-      };
-      const double  ug[3] = {tG[qx * N + jx] * tB[qy * N + jy] * tB[qz * N + jz],
-                             tB[qx * N + jx] * tG[qy * N + jy] * tB[qz * N + jz],
-                             tB[qx * N + jx] * tB[qy * N + jy] * tG[qz * N + jz]};
-      const double  tg[3] = {tGw[qx * N + ix] * tBw[qy * N + iy] * tBw[qz * N + iz],
-                             tBw[qx * N + ix] * tGw[qy * N + iy] * tBw[qz * N + iz],
-                             tBw[qx * N + ix] * tBw[qy * N + iy] * tGw[qz * N + iz]};
-      const double  uv = tB[qx * N + jx] * tB[qy * N + jy] * tB[qz * N + jz];
-      const double  tv = tBw[qx * N + ix] * tBw[qy * N + iy] * tBw[qz * N + iz];
+      for (int a = 0; a < NS; a++)
+#pragma unroll
+        for (int c2 = 0; c2 < NC; c2++) {
+          double t = 0.0;
+#pragma unroll
+          for (int b = 0; b < NS; b++) t += D(slot_of(c, a), slot_of(c2, b)) * uf[b];
+          acc[c][c2] = __builtin_amdgcn_mfma_f64_16x16x4f64(tf[a], t, acc[c][c2], 0, 0, 0);
+        }
+  }
+
+  if (j >= NQ) return;
+  // the four node pairs' searches run side by side (rows past the nodes repeat the first), and without atomics all
+  // old values are read before the first is written: each is a chain of dependent loads otherwise
+  const int*    map  = P.map + size_t(slot) * NQ;
+  const int32_t colv = int32_t(lidx(map[j], 0, NC, P.nnodes, P.ordering));
+  const int     step = P.ordering ? NC : 1;
+  int64_t       row[4][NC];
+  int           nadj[4], lo[4], hi[4];
+  bool          valid[4];
+#pragma unroll
+  for (int r = 0; r < 4; r++) {
+    const int ir         = (tile / Tiles::T) * 16 + 4 * r + (l >> 4);
+    valid[r]             = ir < NQ;
+    const int64_t node_i = map[valid[r] ? ir : 0];
+#pragma unroll
+    for (int c = 0; c < NC; c++) row[r][c] = P.csr_row[lidx(node_i, c, NC, P.nnodes, P.ordering)];
+    nadj[r] = int(P.csr_row[lidx(node_i, 0, NC, P.nnodes, P.ordering) + 1] - row[r][0]) / NC;
+    lo[r]   = 0;
+    hi[r]   = nadj[r];  // the neighbour is in [lo, hi)
+  }
+  while (hi[0] - lo[0] > 1 || hi[1] - lo[1] > 1 || hi[2] - lo[2] > 1 || hi[3] - lo[3] > 1) {
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int  mid = (lo[r] + hi[r]) >> 1;
+      const bool up  = P.csr_col[row[r][0] + int64_t(mid) * step] <= colv;
+      if (hi[r] - lo[r] > 1) (up ? lo[r] : hi[r]) = mid;
+    }
+  }
+  auto at = [&](int r, int c, int c2) {
+    return P.csr_val + (row[r][c] + (P.ordering ? int64_t(lo[r]) * NC + c2 : int64_t(c2) * nadj[r] + lo[r]));
+  };
+  if (!P.scatter) {
+    double old[4][NC][NC];
+#pragma unroll
+    for (int r = 0; r < 4; r++)
 #pragma unroll
       for (int c = 0; c < NC; c++)
 #pragma unroll
-        for (int c2 = 0; c2 < NC; c2++) {
-          double a = 0.0;
+        for (int c2 = 0; c2 < NC; c2++) old[r][c][c2] = valid[r] ? *at(r, c, c2) : 0.0;
 #pragma unroll
-          for (int x = 0; x < 3; x++)
+    for (int r = 0; r < 4; r++)
 #pragma unroll
-            for (int y = 0; y < 3; y++) a += tg[x] * Dq(Shape::idx(VO + c * 3 + x, VO + c2 * 3 + y)) * ug[y];
-          if constexpr (VAL) {
-            a += tv * Dq(Shape::idx(c, c2)) * uv;
+      for (int c = 0; c < NC; c++)
 #pragma unroll
-            for (int y = 0; y < 3; y++)
-              a += tv * Dq(Shape::idx(c, VO + c2 * 3 + y)) * ug[y] + tg[y] * Dq(Shape::idx(VO + c * 3 + y, c2)) * uv;
-          }
-          acc[c][c2] += a;
-        }
-    }
-    const int64_t node_j = P.map[size_t(slot) * NQ + jn];
-#pragma unroll
-    for (int c = 0; c < NC; c++) {
-      const int64_t row = lidx(node_i, c, NC, P.nnodes, P.ordering);
-#pragma unroll
-      for (int c2 = 0; c2 < NC; c2++) {
-        const int32_t colv = int32_t(lidx(node_j, c2, NC, P.nnodes, P.ordering));
-        int64_t       lo = P.csr_row[row], hi = P.csr_row[row + 1];  // the column is in [lo, hi)
-        while (hi - lo > 1) {
-          const int64_t mid = (lo + hi) >> 1;
-          if (P.csr_col[mid] <= colv)
-            lo = mid;
-          else
-            hi = mid;
-        }
-        scatter_add(P.csr_val, lo, acc[c][c2], P.scatter);
-      }
-    }
+        for (int c2 = 0; c2 < NC; c2++)
+          if (valid[r]) *at(r, c, c2) = old[r][c][c2] + acc[c][c2][r];
+    return;
   }
+#pragma unroll
+  for (int r = 0; r < 4; r++)
+#pragma unroll
+    for (int c = 0; c < NC; c++)
+#pragma unroll
+      for (int c2 = 0; c2 < NC; c2++)
+        if (valid[r]) unsafeAtomicAdd(at(r, c, c2), acc[c][c2][r]);
 }
 
 // ---------------------------------------------------------------------------
@@ -1524,13 +1591,11 @@ inline int dispatch_gradient(const ElemLaunch& P, hipError_t* err)
   if (P.mode == MODE_ASSEMBLE) {
     const int64_t n = P.slot_end - P.slot_begin;
     if (n <= 0) return 1;
-    // the element's tangent is staged in LDS when it fits in 48 KB
-    constexpr int    NQ    = N * N * N;
-    constexpr size_t bytes = size_t(NQ) * TanShape<LAYOUT, NC>::DS * sizeof(double);
+    using Tiles            = AssembleTiles<N>;
+    constexpr size_t bytes = size_t(N * N * N) * TanShape<LAYOUT, NC>::DS * sizeof(double);
     constexpr bool   stage = bytes <= 48 * 1024;
-    const unsigned   threads = unsigned((NQ + 63) / 64 * 64);
-    hipLaunchKernelGGL((k_assemble<N, NC, LAYOUT, S, stage>), dim3(unsigned(n)), dim3(threads), stage ? bytes : 0,
-                       P.stream, P);
+    hipLaunchKernelGGL((k_assemble<N, NC, LAYOUT, S, stage>), dim3(unsigned(n * Tiles::GROUPS)),
+                       dim3(64 * Tiles::WAVES), stage ? bytes : 0, P.stream, P);
     *err = hipGetLastError();
     return 1;
   }
