@@ -238,11 +238,13 @@ int sx_form_update_qdata(sx_form* f, int flag);
 #define SX_WRT_SHAPE (-2)
 int sx_form_eval(sx_form* f, double t, const double* const* inputs, double* out, int wrt, sx_grad** grad_out);
 /* Form options (no reference counterpart: the reference runs serially).
- *   SX_OPT_SCATTER: SX_SCATTER_COLORED (default) launches one kernel per
- *     element colour and adds into the output with plain read-modify-writes:
- *     results are bitwise reproducible.  SX_SCATTER_ATOMIC launches all
- *     elements at once and adds with FP64 atomics: fewer L-vector passes,
- *     last-bit rounding depends on the order the hardware applies them.
+ *   SX_OPT_SCATTER: SX_SCATTER_COLORED (default) gives bitwise reproducible
+ *     results: the element kernel stores its values and a second kernel adds
+ *     them per node in element order (the form keeps up to 192 MB of element
+ *     values), or, on larger meshes, one kernel per element colour adds with
+ *     plain read-modify-writes.  SX_SCATTER_ATOMIC adds with FP64 atomics:
+ *     one pass, last-bit rounding depends on the order the hardware applies
+ *     them.
  *     Must be set before the first AddDomainIntegral.
  *   SX_OPT_XCD_REMAP: 1 gives each of the 8 XCDs a contiguous run of element
  *     blocks (L2 locality for shared nodes); 0 (default) keeps the hardware's

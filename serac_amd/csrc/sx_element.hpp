@@ -16,9 +16,10 @@
 // Q = p + 1 = nodes per direction (fn/functional.hpp:193).  LDS per element is
 // (6 + has_source) * nc * Q^3 values, reused across stages.
 //
-// The scatter-add is either a plain read-modify-write (one launch per element
-// colour: no two elements of a colour share a node) or an FP64/FP32 atomic add
-// (one launch for all elements).
+// The scatter-add is an FP64/FP32 atomic add, or a plain store of the element's
+// values for a node sum that follows (SCATTER_ELEMENT, reproducible), both in
+// one launch for all elements, or a plain read-modify-write (one launch per
+// element colour: no two elements of a colour share a node).
 //
 // Precision: residual and linearization compute in FP64.  The stored tangent
 // is kept in S = double, float or bf16; the J.v kernel computes in T = double
@@ -182,6 +183,25 @@ __device__ __forceinline__ void scatter_add(T* r, int64_t o, T v, int atomic)
 __device__ __forceinline__ int64_t lidx(int64_t node, int c, int nc, int64_t nnodes, int ordering)
 {
   return ordering ? node * nc + c : int64_t(c) * nnodes + node;
+}
+
+// SCATTER_ELEMENT: the element's values as one run of consecutive addresses,
+// through LDS (sv: NC * NQ values).  Every lane of the workgroup calls it (it
+// holds a barrier).
+template <int N, int NC, typename T>
+__device__ __forceinline__ void store_element(void* E, const T* acc, T* sv, int64_t slot, int li, bool active)
+{
+  constexpr int NQ = N * N * N;
+  if (active) {
+#pragma unroll
+    for (int c = 0; c < NC; c++) sv[li * NC + c] = acc[c];
+  }
+  lds_barrier();
+  if (active) {
+    T* Ee = static_cast<T*>(E) + size_t(slot) * (NC * NQ) + li;
+#pragma unroll
+    for (int t = 0; t < NC; t++) Ee[t * NQ] = sv[t * NQ + li];
+  }
 }
 
 // Scatter-add of one element's NC x NQ nodal values in address order.  Lane li
@@ -777,7 +797,9 @@ __global__ void __launch_bounds__(256, (element_waves<MODE, QF>())) k_element(co
       }
     }
   }
-  if (P.ordered) {
+  if (P.scatter == SCATTER_ELEMENT) {
+    store_element<N, NC>(P.E, acc, S_ + 2 * R, slot, li, active);
+  } else if (P.ordered) {
     scatter_element<N, NC, double, double>(r, acc, S_ + 2 * R, smem + (el > 0 && el < EB ? el - 1 : 0) * PER + 2 * R,
                                            snode, el, EB, node, li, active, P.nnodes, P.ordering, P.scatter,
                                            P.ordered == 2);
@@ -996,7 +1018,9 @@ __global__ void __launch_bounds__((jvp_group_lanes<N, T>())) k_jvp(const ElemLau
       }
     }
   }
-  if (P.ordered) {
+  if (P.scatter == SCATTER_ELEMENT) {
+    store_element<N, NC>(P.E, acc, S_ + 2 * R, slot, li, active);
+  } else if (P.ordered) {
     scatter_element<N, NC, T, V>(r, acc, S_ + 2 * R, smem + (el > 0 && el < EB ? el - 1 : 0) * PER + 2 * R, snode,
                                  el, EB, node, li, active, P.nnodes, P.ordering, P.scatter, P.ordered == 2);
   } else if (active) {
@@ -1204,6 +1228,10 @@ __global__ void __launch_bounds__(64 * EB) k_jvp_xy(const ElemLaunch P)
     }
   }
   // slot 2 is free here: the z integration reads slots 0 and 1 only
+  if (P.scatter == SCATTER_ELEMENT) {
+    store_element<N, NC>(P.E, acc, S_ + 2 * R, slot, li, active);
+    return;
+  }
   const int64_t node = active ? int64_t(sn_el[li]) : 0;
   if (P.ordered) {
     scatter_element<N, NC, T, V>(r, acc, S_ + 2 * R, smem + (el > 0 && el < EB ? el - 1 : 0) * PER + 2 * R, snode,
@@ -1357,7 +1385,9 @@ __global__ void __launch_bounds__(256) k_diagonal(const ElemLaunch P)
   const int64_t node = active ? int64_t(P.map[size_t(slot) * NQ + li]) : 0;
   double*       out  = static_cast<double*>(P.r);
   __syncthreads();  // the last z stage has read the slots
-  if (P.ordered) {
+  if (P.scatter == SCATTER_ELEMENT) {
+    store_element<N, NC>(P.E, acc, sv, slot, li, active);
+  } else if (P.ordered) {
     scatter_element<N, NC, double, double>(out, acc, sv, sf + (el > 0 && el < EB ? el - 1 : 0) * NF * NQ, snode, el,
                                            EB, node, li, active, P.nnodes, P.ordering, P.scatter, P.ordered == 2);
   } else if (active) {
@@ -1407,7 +1437,8 @@ __global__ void __launch_bounds__(64 * AssembleTiles<N>::WAVES, 2) k_assemble(co
   constexpr int  DS  = Shape::DS;
   __shared__ double        stab[TAB];
   extern __shared__ double sD[];  // [q][DS]
-  const int64_t slot = P.slot_begin + blockIdx.x / Tiles::GROUPS;
+  const int64_t pos  = P.slot_begin + blockIdx.x / Tiles::GROUPS;
+  const int64_t slot = P.slot_list ? P.slot_list[pos] : pos;
 
   using raw       = typename StoreTraits<S>::raw;
   const raw* Dsrc = reinterpret_cast<const raw*>(static_cast<const char*>(P.D) + size_t(slot) * Lay::stride * sizeof(S));

@@ -23,6 +23,12 @@ enum Layout { LAYOUT_GRAD_SYM = 0, LAYOUT_FULL_SYM = 1, LAYOUT_GRAD_FULL = 2 };
 // PREC_MIXED (J.v only): FP64 vectors, FP32 element arithmetic
 enum Precision { PREC_F64 = 0, PREC_F32 = 1, PREC_BF16 = 2, PREC_MIXED = 3 };
 
+// How the element kernels add their nodal values into the output:
+//   PLAIN:   read-modify-write (no two elements of the launch share a node)
+//   ATOMIC:  atomics
+//   ELEMENT: stored in `E`, [slot][node][component], for a node sum that follows
+enum Scatter { SCATTER_PLAIN = 0, SCATTER_ATOMIC = 1, SCATTER_ELEMENT = 2 };
+
 enum QFId {
   QF_ID_HEAT           = 1,
   QF_ID_MASS_DIFFUSION = 2,
@@ -36,7 +42,7 @@ struct ElemLaunch {
   int           order, nc, qf, mode, layout, ordering;
   int           tprec;      // Precision of the stored tangent
   int           vprec;      // Precision of the J.v vectors (residual/linearize: FP64)
-  int           scatter;    // 0: plain read-modify-write (colour launches), 1: atomics
+  int           scatter;    // Scatter
   int           xcd_remap;  // 1: give each XCD a contiguous range of element blocks
   int           ordered;    // 1: scatter each element's values in address order (through LDS)
   const int*    map;        // [slot][npe] global node ids
@@ -45,6 +51,7 @@ struct ElemLaunch {
   int64_t       nnodes;
   const void*   u;       // input L-vector (trial), FP64 or (J.v) vprec
   void*         r;       // output L-vector (test), accumulated into
+  void*         E;       // SCATTER_ELEMENT: the element values, in the kernel's arithmetic type
   void*         D;       // stored tangent, per-slot layout of sx_element.hpp TangentLayout
   const double* tables;  // B, G, Bw, Gw [Q][N] and GL points [Q]
   double*       qdata;         // quadrature-point state [row][k][q] (residual/linearize)
@@ -56,6 +63,7 @@ struct ElemLaunch {
   const double*  shape;        // residual/linearize: shape displacement p (3-component L-vector of the
                                // test space) or null; the geometry becomes X + p
   const double*  dshape;       // MODE_SHAPE_JVP: the direction of the shape displacement
+  const int*     slot_list;    // assembly: launch position -> slot, or null
   const double*  stop;         // J.v: when non-null and *stop != 0 the kernel returns at once
   double        params[16];
   double        t;
