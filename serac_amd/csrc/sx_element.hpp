@@ -497,9 +497,7 @@ __global__ void __launch_bounds__(256, (element_waves<MODE, QF>())) k_element(co
   constexpr int  NQ      = N * N * N;
   constexpr int  EB      = 256 / NQ;
   using Shape            = TanShape<LAYOUT, NC>;
-  constexpr bool FULL    = Shape::VAL;
   constexpr bool HAS_SRC = QF::HAS_SOURCE;
-  constexpr int  M       = Shape::M;
   constexpr int  DS      = Shape::DS;
   constexpr int  NST     = QF::STATE;
   constexpr int  R       = NC * NQ;  // one LDS region

@@ -102,6 +102,9 @@ struct sx_unet {
   Buf xin;       // BF16 input [n0][3]
   Buf yout;      // FP32 output [n0][3]
   Buf wflip, tmp, sums;
+  // backward pass on the matrix cores: BF16 planes of a layer's gradient
+  // (channel-last and channel-major), its input channel-major, its weights
+  Buf gcl, gcm, xcm, wpl;
 
   int64_t cin(int k) const { return kLayers[k].cin_a + kLayers[k].cin_b; }
 };
@@ -216,26 +219,60 @@ void weight_grad(sx_unet* N, int k, const void* xa, const void* xb, const float*
   UN_HIP(sxu::conv_wgrad(A, L.cout, false, N->stream));
 }
 
+// The gradients of layer k from g = dL/d(its output) on the matrix cores: weights and bias into G, the data gradient
+// of the parts of a stride-1 layer's input into da (channels cin_a) and db (channels cin_b) where not null
+void backward_layer_mfma(sx_unet* N, int k, const void* xa, const void* xb, const float* g, float* da, float* db)
+{
+  const LayerDef&    L  = kLayers[k];
+  hipStream_t        s  = N->stream;
+  const int          up = L.mode == 1 ? 2 : 1;
+  const sxu::PadGrid P  = sxu::pad_grid(N->dims[L.lin]);
+  const uint16_t*    y  = L.relu && !N->identity ? N->act[k].as<uint16_t>() : nullptr;
+  const uint16_t*    w  = N->Wbf.as<uint16_t>() + N->woff[k];
+  float*             dw = N->G.as<float>() + N->woff[k];
+  UN_HIP(sxu::bias_grad(g, y, N->nvox[L.lout], L.cout, N->G.as<float>() + N->boff[k], s));
+  UN_HIP(sxu::planes_cm(g, y, L.cout, up, N->dims[L.lout], P, N->gcm.as<uint16_t>(), s));
+  const void* xs[2] = {xa, xb};
+  const int   cs[2] = {L.cin_a, L.cin_b};
+  for (int i = 0, first = 0; i < 2 && cs[i] > 0; first += cs[i], i++) {
+    UN_HIP(sxu::input_cm(static_cast<const uint16_t*>(xs[i]), cs[i], N->dims[L.lin], P, N->xcm.as<uint16_t>(), s));
+    UN_HIP(sxu::wgrad_mfma(N->xcm.as<uint16_t>(), cs[i], int(N->cin(k)), first, N->gcm.as<uint16_t>(), L.cout, P, dw, s));
+  }
+  if (!da && !db) return;
+  UN_HIP(sxu::planes_cl(g, y, L.cout, P, N->gcl.as<uint16_t>(), s));
+  if (da)
+    UN_HIP(sxu::dgrad_mfma(N->gcl.as<uint16_t>(), w, int(N->cin(k)), L.cout, 0, L.cin_a, P, N->wpl.as<uint16_t>(), da, s));
+  if (db)
+    UN_HIP(sxu::dgrad_mfma(N->gcl.as<uint16_t>(), w, int(N->cin(k)), L.cout, L.cin_a, L.cin_b, P, N->wpl.as<uint16_t>(),
+                           db, s));
+}
+
 // backward from dL/dy (in gact[11]); gradients accumulate into G
 void backward(sx_unet* N)
 {
   hipStream_t s   = N->stream;
   auto        nel = [&](int k) { return N->nvox[kLayers[k].lout] * kLayers[k].cout; };
-  float*      g;
+  // layer k: weight gradients, and the data gradients of its input parts into
+  // da and db (null: none)
+  auto layer = [&](int k, const void* xa, const void* xb, float* da, float* db) {
+    const LayerDef& L = kLayers[k];
+    float*          g = N->gact[k].as<float>();
+    const bool      strided = L.mode == 1;
+    if (N->use_mfma) backward_layer_mfma(N, k, xa, xb, g, strided ? nullptr : da, strided ? nullptr : db);
+    if (N->use_mfma && !strided) return;
+    if (L.relu && !N->identity) UN_HIP(sxu::relu_bwd(g, N->act[k].as<uint16_t>(), nel(k), s));
+    if (!N->use_mfma) weight_grad(N, k, xa, xb, g);
+    if (da) data_grad(N, k, g, 0, L.cin_a, da);
+    if (db) data_grad(N, k, g, L.cin_a, L.cin_b, db);
+  };
   // head (no activation)
-  g = N->gact[11].as<float>();
-  weight_grad(N, 11, N->act[10].p, nullptr, g);
-  data_grad(N, 11, g, 0, 16, N->gact[10].as<float>());
+  layer(11, N->act[10].p, nullptr, N->gact[10].as<float>(), nullptr);
   // decoder 10, 9, 8: input parts [P c, skip]
   const int src[3] = {7, 8, 9}, skip[3] = {5, 3, 1};
   for (int j = 2; j >= 0; j--) {
     const int k = 8 + j;
-    g           = N->gact[k].as<float>();
-    if (!N->identity) UN_HIP(sxu::relu_bwd(g, N->act[k].as<uint16_t>(), nel(k), s));
-    weight_grad(N, k, N->up[j].p, N->act[skip[j]].p, g);
-    data_grad(N, k, g, 0, kLayers[k].cin_a, N->gup[j].as<float>());
     // the skip's gradient from the decoder starts the skip's accumulation
-    data_grad(N, k, g, kLayers[k].cin_a, kLayers[k].cin_b, N->gact[skip[j]].as<float>());
+    layer(k, N->up[j].p, N->act[skip[j]].p, N->gup[j].as<float>(), N->gact[skip[j]].as<float>());
     // the prolonged source's gradient is the restriction of gup
     const int lc = kLayers[src[j]].lout, lf = kLayers[k].lout;
     UN_HIP(sxu::restrict_f32(N->gup[j].as<float>(), N->dims[lf], N->gact[src[j]].as<float>(), N->dims[lc],
@@ -243,22 +280,17 @@ void backward(sx_unet* N)
   }
   // encoder 7 .. 0
   for (int k = 7; k >= 0; k--) {
-    g = N->gact[k].as<float>();
-    if (!N->identity) UN_HIP(sxu::relu_bwd(g, N->act[k].as<uint16_t>(), nel(k), s));
-    const void* xin = k == 0 ? N->xin.p : N->act[k - 1].p;
-    weight_grad(N, k, xin, nullptr, g);
-    if (k == 0) break;
+    if (k == 0) {
+      layer(0, N->xin.p, nullptr, nullptr, nullptr);
+      break;
+    }
     // layer k's input is act[k-1]; odd encoder layers (b) feed the decoder
     // too, so their gradient already holds the skip term and gets this added
     float*        gin = N->gact[k - 1].as<float>();
     const int64_t nin = N->nvox[kLayers[k].lin] * kLayers[k].cin_a;
     const bool    has_skip = (k - 1 == 1 || k - 1 == 3 || k - 1 == 5);
-    if (has_skip) {
-      data_grad(N, k, g, 0, kLayers[k].cin_a, N->tmp.as<float>());
-      UN_HIP(sxu::add_f32(gin, N->tmp.as<float>(), nin, s));
-    } else {
-      data_grad(N, k, g, 0, kLayers[k].cin_a, gin);
-    }
+    layer(k, N->act[k - 1].p, nullptr, has_skip ? N->tmp.as<float>() : gin, nullptr);
+    if (has_skip) UN_HIP(sxu::add_f32(gin, N->tmp.as<float>(), nin, s));
   }
 }
 
@@ -343,6 +375,19 @@ void init(sx_unet* N, int nx, int ny, int nz, uint64_t seed)
   N->wflip.alloc(size_t(wmax) * 2);
   N->tmp.alloc(size_t(tmax) * 4);
   N->sums.alloc(2 * sizeof(double));
+  size_t gcl = 0, gcm = 0, xcm = 0, wpl = 0;
+  for (int k = 0; k < 12; k++) {
+    const LayerDef&    L = kLayers[k];
+    const sxu::PadGrid P = sxu::pad_grid(N->dims[L.lin]);
+    if (L.mode == 0) gcl = std::max(gcl, sxu::planes_cl_elems(P, L.cout));
+    gcm = std::max(gcm, size_t(P.row) * size_t(3 * L.cout));
+    xcm = std::max(xcm, size_t(P.row) * size_t(std::max(L.cin_a, L.cin_b)));
+    wpl = std::max(wpl, size_t(std::max(L.cin_a, L.cin_b)) * size_t(sxu::plane_kpad(L.cout)));
+  }
+  N->gcl.alloc(gcl * 2);
+  N->gcm.alloc(gcm * 2);
+  N->xcm.alloc(xcm * 2);
+  N->wpl.alloc(wpl * 2);
   UN_HIP(hipStreamCreateWithFlags(&N->stream, hipStreamNonBlocking));
 }
 

@@ -387,6 +387,267 @@ __global__ void __launch_bounds__(kThreads) k_conv_wgrad(WGradArgs A, int chunks
   if (tap == 0 && A.db && int(threadIdx.x) < COUT) atomicAdd(&A.db[threadIdx.x], bpart);
 }
 
+// ---------------------------------------------------------------------------
+// backward convolutions on the matrix cores
+// ---------------------------------------------------------------------------
+// The gradient g that arrives at a layer is FP32 and stays so: it is split into
+// three BF16 planes, g = hi + mid + lo (each the rounding of what the previous
+// ones leave, 8 significant bits a plane, so the sum is exact), and every
+// product of an activation or weight (BF16) with g becomes three BF16 products
+// accumulated in FP32.
+//
+// Both convolutions of the backward pass then run over a zero-padded grid,
+// flattened: with px = nx + 2 nodes in a padded row, the neighbour at tap
+// (dx, dy, dz) of node o is o + dx + px dy + px py dz, whatever o, so there are
+// no bounds to test and one constant per tap.
+//   planes_cl: [padded node][plane][channel], for the data gradient
+//   planes_cm: [plane][channel][padded node], for the weight gradient
+//   input_cm:  [channel][padded node], the layer's input
+// The channel-major arrays have kPadGuard(px, py) zeros before and after each
+// row, since o of a padding node reaches past the grid (its g is zero).
+
+__device__ __forceinline__ void split3(float g, uint16_t* out)
+{
+  out[0]         = f2bf(g);
+  const float r1 = g - bf2f(out[0]);
+  out[1]         = f2bf(r1);
+  out[2]         = f2bf(r1 - bf2f(out[1]));
+}
+
+// padded coordinates of padded node v; false on the padding
+__device__ __forceinline__ bool pad_interior(int v, const PadGrid& P, int& x, int& y, int& z)
+{
+  x = v % P.px - 1;
+  y = (v / P.px) % P.py - 1;
+  z = v / (P.px * P.py) - 1;
+  return v >= 0 && x >= 0 && x < P.px - 2 && y >= 0 && y < P.py - 2 && z >= 0 && z < P.pz - 2;
+}
+
+// channel-last planes of g (masked by the activation's output y where given);
+// CP channels per plane set: 3 C, or 16 for C = 3
+__global__ void __launch_bounds__(kThreads) k_planes_cl(const float* g, const uint16_t* y, int C, int CP, PadGrid P,
+                                                        uint16_t* out)
+{
+  const int64_t n = int64_t(P.nodes) * C;
+  for (int64_t t = int64_t(blockIdx.x) * kThreads + threadIdx.x; t < n; t += int64_t(gridDim.x) * kThreads) {
+    const int v = int(t / C), c = int(t - int64_t(v) * C);
+    int       ix, iy, iz;
+    float     gv = 0.0f;
+    if (pad_interior(v, P, ix, iy, iz)) {
+      const int64_t s = ((int64_t(iz) * (P.py - 2) + iy) * (P.px - 2) + ix) * C + c;
+      gv              = g[s];
+      if (y && !(bf2f(y[s]) > 0.0f)) gv = 0.0f;
+    }
+    uint16_t h[3];
+    split3(gv, h);
+    uint16_t* o = out + (int64_t(P.guard) + v) * CP + c;
+    o[0]        = h[0];
+    o[C]        = h[1];
+    o[2 * C]    = h[2];
+    if (c == 0)
+      for (int k = 3 * C; k < CP; k++) o[k] = 0;
+  }
+}
+
+// channel-major planes of g on the padded grid P: a tile of 64 nodes goes
+// through LDS.  up = 2: g lives on the grid of every other node of P
+// (a stride-2 layer: the weight gradient sums over the fine nodes, where g is
+// zero in between).
+template <int NPL>
+__global__ void __launch_bounds__(kThreads) k_to_cm(const void* src, const uint16_t* y, int C, int up, Dims3 d,
+                                                    PadGrid P, uint16_t* out)
+{
+  constexpr int       VT = 64;
+  __shared__ uint16_t tile[NPL][64][VT + 2];
+  const int           base = int(blockIdx.x) * VT - P.guard;  // padded node of the tile's first column
+  const int           c0   = int(blockIdx.y) * 64, nc = min(64, C - c0);
+  for (int t = threadIdx.x; t < VT * nc; t += kThreads) {
+    const int j = t / nc, c = t - j * nc, v = base + j;
+    int       ix, iy, iz;
+    bool      in = v >= 0 && v < P.nodes && pad_interior(v, P, ix, iy, iz);
+    if (in && up == 2) {
+      in = !((ix | iy | iz) & 1);
+      ix >>= 1;
+      iy >>= 1;
+      iz >>= 1;
+    }
+    uint16_t h[3] = {0, 0, 0};
+    if (in) {
+      const int64_t s = ((int64_t(iz) * d.n[1] + iy) * d.n[0] + ix) * C + c0 + c;
+      if constexpr (NPL == 3) {
+        float gv = static_cast<const float*>(src)[s];
+        if (y && !(bf2f(y[s]) > 0.0f)) gv = 0.0f;
+        split3(gv, h);
+      } else {
+        h[0] = static_cast<const uint16_t*>(src)[s];
+      }
+    }
+#pragma unroll
+    for (int p = 0; p < NPL; p++) tile[p][c][j] = h[p];
+  }
+  __syncthreads();
+  for (int t = threadIdx.x; t < VT * nc * NPL; t += kThreads) {
+    const int     j = t % VT, c = (t / VT) % nc, p = t / (VT * nc);
+    const int64_t col = int64_t(blockIdx.x) * VT + j;
+    if (col < P.row) out[(int64_t(p) * C + c0 + c) * P.row + col] = tile[p][c][j];
+  }
+}
+
+// wt[ci][tap'][plane][co] = w[26 - tap'][c0 + ci][co], three times over, for
+// ci < cpart: the data gradient's weights along its K, padded with zeros
+__global__ void k_weights_planes(const uint16_t* w, int cin, int cout, int c0, int cpart, int CP, int kpad, uint16_t* wt)
+{
+  const int64_t n = int64_t(cpart) * kpad;
+  for (int64_t t = int64_t(blockIdx.x) * kThreads + threadIdx.x; t < n; t += int64_t(gridDim.x) * kThreads) {
+    const int ci = int(t / kpad), k = int(t % kpad), tap = k / CP, pc = k % CP;
+    wt[t] = tap < 27 && pc < 3 * cout ? w[(int64_t(26 - tap) * cin + c0 + ci) * cout + pc % cout] : uint16_t(0);
+  }
+}
+
+// Data gradient: out[node][co] (FP32, unpadded) = sum_k planes[node + tap][plane, channel] wt[co][k], an implicit
+// GEMM of 16-node row tiles by 16-channel column tiles on mfma_f32_16x16x32_bf16.  KS = 1: a wave owns RT row tiles
+// and NT column tiles, all of K.  KS = 4 (coarse levels, where that leaves most of the GPU idle): the workgroup's
+// four waves share one row tile's K and add their parts in LDS.
+// 65^3 grid, 16 <- 32 channels: 105 us where the vector units took 304; 17^3, 64 <- 64: 66 us (107).
+template <int NT, int RT, int KS>
+__global__ void __launch_bounds__(kThreads) k_dgrad(const uint16_t* planes, int CP, const uint16_t* wt, int kpad, int K,
+                                                    PadGrid P, float* out, int cout)
+{
+  extern __shared__ int soff[];  // element offset of every 8-channel group of K
+  for (int t = threadIdx.x; t < kpad / 8; t += kThreads) {
+    const int k = 8 * t, tap = k / CP;
+    const int d = (tap % 3 - 1) + P.px * ((tap / 3) % 3 - 1) + P.px * P.py * (tap / 9 - 1);
+    soff[t]     = k < K ? d * CP + (k - tap * CP) : 0;  // past K the weights are zero
+  }
+  __syncthreads();
+  const int lane = int(threadIdx.x) & 63, wave = int(threadIdx.x) >> 6;
+  const int m = lane & 15, kg = lane >> 4;
+  const int base = (KS == 1 ? int(blockIdx.x) * 4 + wave : int(blockIdx.x)) * (RT * 16);
+  const int ct0  = int(blockIdx.y) * NT;
+  f32x4_t   acc[RT][NT];
+#pragma unroll
+  for (int rt = 0; rt < RT; rt++)
+#pragma unroll
+    for (int ct = 0; ct < NT; ct++) acc[rt][ct] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  const uint16_t* pa[RT];
+#pragma unroll
+  for (int rt = 0; rt < RT; rt++) pa[rt] = planes + (int64_t(P.guard) + min(base + rt * 16 + m, P.nodes - 1)) * CP;
+  const uint16_t* pb = wt + int64_t(ct0 * 16 + m) * kpad;
+  const int       steps = kpad / 32;
+  const int       s0 = KS == 1 ? 0 : steps * wave / KS, s1 = KS == 1 ? steps : steps * (wave + 1) / KS;
+#pragma unroll 4
+  for (int s = s0; s < s1; s++) {
+    const int off = soff[s * 4 + kg];
+    bf16x8_t  av[RT];
+#pragma unroll
+    for (int rt = 0; rt < RT; rt++) av[rt] = *reinterpret_cast<const bf16x8_t*>(pa[rt] + off);
+#pragma unroll
+    for (int ct = 0; ct < NT; ct++) {
+      const bf16x8_t bv = *reinterpret_cast<const bf16x8_t*>(pb + int64_t(ct * 16) * kpad + s * 32 + 8 * kg);
+#pragma unroll
+      for (int rt = 0; rt < RT; rt++)
+        acc[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[rt], bv, acc[rt][ct], 0, 0, 0);
+    }
+  }
+  if constexpr (KS > 1) {
+    __shared__ f32x4_t part[3][RT * NT][64];
+    if (wave > 0) {
+#pragma unroll
+      for (int t = 0; t < RT * NT; t++) part[wave - 1][t][lane] = acc[t / NT][t % NT];
+    }
+    __syncthreads();
+    if (wave > 0) return;
+#pragma unroll
+    for (int t = 0; t < RT * NT; t++)
+      acc[t / NT][t % NT] += (part[0][t][lane] + part[1][t][lane]) + part[2][t][lane];
+  }
+#pragma unroll
+  for (int rt = 0; rt < RT; rt++)
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int v = base + rt * 16 + 4 * kg + r;
+      int       ix, iy, iz;
+      if (v >= P.nodes || !pad_interior(v, P, ix, iy, iz)) continue;
+      float* o = out + ((int64_t(iz) * (P.py - 2) + iy) * (P.px - 2) + ix) * cout + ct0 * 16 + m;
+#pragma unroll
+      for (int ct = 0; ct < NT; ct++) o[ct * 16] = acc[rt][ct][r];
+    }
+}
+
+// Weight gradient: dw[tap][ci][co] += sum over the padded nodes o of
+// x[ci][o + tap] g[co][o], 16 x 16 tiles of (ci, co) with K = 32 nodes per mfma
+// and one mfma per plane of g.  A workgroup takes one tile and a run of nodes,
+// each wave every fourth tap; the parts are added with FP32 atomics.  x at
+// o + tap is 16 bytes at any 2-byte address, read straight from memory (the
+// rows of a tile stay in the caches across taps).
+// 65^3 grid, 32 x 16 channels: 192 us where the vector units took 880.  Bound by the latency of the loads.
+__global__ void __launch_bounds__(kThreads) k_wgrad(const uint16_t* x, int cin, const uint16_t* g, int cout, PadGrid P,
+                                                    int steps_per_run, float* dw, int cin_all, int ci_first)
+{
+  constexpr int TW   = 7;  // taps per wave
+  const int     lane = int(threadIdx.x) & 63, wave = int(threadIdx.x) >> 6;
+  const int     m = lane & 15, kg = lane >> 4;
+  const int     cot = (cout + 15) / 16;
+  const int     ci0 = (int(blockIdx.y) / cot) * 16, co0 = (int(blockIdx.y) % cot) * 16;
+  const int     ci = min(ci0 + m, cin - 1), co = min(co0 + m, cout - 1);  // rows past the channels are dropped
+  const int     steps = (P.nodes + 31) / 32;
+  const int     s0 = int(blockIdx.x) * steps_per_run, s1 = min(steps, s0 + steps_per_run);
+  const uint16_t* px = x + int64_t(ci) * P.row + P.guard + 8 * kg;
+  const uint16_t* pg = g + int64_t(co) * P.row + P.guard + 8 * kg;
+  const int64_t   plane = int64_t(cout) * P.row;
+  int             off[TW];
+  f32x4_t         acc[TW];
+#pragma unroll
+  for (int t = 0; t < TW; t++) {
+    const int tap = min(wave + 4 * t, 26);
+    off[t]        = (tap % 3 - 1) + P.px * ((tap / 3) % 3 - 1) + P.px * P.py * (tap / 9 - 1);
+    acc[t]        = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  }
+#pragma unroll 2
+  for (int s = s0; s < s1; s++) {
+    bf16x8_t bv[3], av[TW];
+#pragma unroll
+    for (int p = 0; p < 3; p++) bv[p] = *reinterpret_cast<const bf16x8_t*>(pg + p * plane + int64_t(s) * 32);
+#pragma unroll
+    for (int t = 0; t < TW; t++) __builtin_memcpy(&av[t], px + int64_t(s) * 32 + off[t], 16);
+#pragma unroll
+    for (int t = 0; t < TW; t++)
+#pragma unroll
+      for (int p = 0; p < 3; p++) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[t], bv[p], acc[t], 0, 0, 0);
+  }
+  if (co0 + m >= cout) return;
+#pragma unroll
+  for (int t = 0; t < TW; t++) {
+    const int tap = wave + 4 * t;
+    if (tap > 26) continue;
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int i = ci0 + 4 * kg + r;
+      if (i < cin) atomicAdd(&dw[(int64_t(tap) * cin_all + ci_first + i) * cout + co0 + m], acc[t][r]);
+    }
+  }
+}
+
+// db[co] += sum_o g[o][co], g masked by the activation's output y where given
+__global__ void __launch_bounds__(kThreads) k_bias_grad(const float* g, const uint16_t* y, int64_t n, int C, float* db)
+{
+  __shared__ float sh[kThreads];
+  const int        per = kThreads / C * C;  // threads in use: a multiple of the channels
+  float            s   = 0.0f;
+  if (int(threadIdx.x) < per)
+    for (int64_t i = int64_t(blockIdx.x) * per + threadIdx.x; i < n * C; i += int64_t(gridDim.x) * per) {
+      const float v = g[i];
+      if (!y || bf2f(y[i]) > 0.0f) s += v;
+    }
+  sh[threadIdx.x] = s;
+  __syncthreads();
+  if (int(threadIdx.x) < C) {
+    float a = 0.0f;
+    for (int k = int(threadIdx.x); k < per; k += C) a += sh[k];
+    atomicAdd(&db[threadIdx.x], a);
+  }
+}
+
 // wt[tap'][co][ci] = w[26 - tap'][c0 + ci][co] for ci < cpart: the weights of
 // the data-gradient convolution of input part [c0, c0 + cpart)
 __global__ void k_flip_weights(const uint16_t* w, int cin, int cout, int c0, int cpart, uint16_t* wt)
@@ -741,6 +1002,91 @@ hipError_t conv_mfma(const ConvArgs& A, int cout, const uint16_t* wt, hipStream_
     case 32: hipLaunchKernelGGL((k_conv_mfma<32, MFMA_RT32>), grid(MFMA_RT32), block, 0, s, A, wt, kpad); break;
     default: hipLaunchKernelGGL((k_conv_mfma<64, MFMA_RT64>), grid(MFMA_RT64), block, 0, s, A, wt, kpad); break;
   }
+  return hipGetLastError();
+}
+
+PadGrid pad_grid(Dims3 d)
+{
+  PadGrid P;
+  P.px    = d.n[0] + 2;
+  P.py    = d.n[1] + 2;
+  P.pz    = d.n[2] + 2;
+  P.nodes = P.px * P.py * P.pz;
+  // the farthest neighbour and a K step of 32 nodes past the end; rows start and stay 16-byte aligned
+  P.guard = (P.px * P.py + P.px + 1 + 32 + 63) / 64 * 64;
+  P.row   = int64_t(P.guard) * 2 + (P.nodes + 63) / 64 * 64;
+  return P;
+}
+int    plane_channels(int cout) { return cout % 16 == 0 ? 3 * cout : (3 * cout + 15) / 16 * 16; }
+int    plane_kpad(int cout) { return (27 * plane_channels(cout) + 31) / 32 * 32; }
+size_t planes_cl_elems(const PadGrid& P, int cout) { return size_t(P.row) * size_t(plane_channels(cout)); }
+
+hipError_t planes_cl(const float* g, const uint16_t* y, int cout, const PadGrid& P, uint16_t* out, hipStream_t s)
+{
+  hipLaunchKernelGGL(k_planes_cl, dim3(std::min<unsigned>(blocks_for(int64_t(P.nodes) * cout), 8192)), dim3(kThreads), 0,
+                     s, g, y, cout, plane_channels(cout), P, out);
+  return hipGetLastError();
+}
+
+hipError_t planes_cm(const float* g, const uint16_t* y, int cout, int up, Dims3 d, const PadGrid& P, uint16_t* out,
+                     hipStream_t s)
+{
+  const dim3 grid{unsigned((P.row + 63) / 64), unsigned((cout + 63) / 64)};
+  hipLaunchKernelGGL(k_to_cm<3>, grid, dim3(kThreads), 0, s, g, y, cout, up, d, P, out);
+  return hipGetLastError();
+}
+
+hipError_t input_cm(const uint16_t* x, int cin, Dims3 d, const PadGrid& P, uint16_t* out, hipStream_t s)
+{
+  const dim3 grid{unsigned((P.row + 63) / 64), unsigned((cin + 63) / 64)};
+  hipLaunchKernelGGL(k_to_cm<1>, grid, dim3(kThreads), 0, s, x, static_cast<const uint16_t*>(nullptr), cin, 1, d, P,
+                     out);
+  return hipGetLastError();
+}
+
+hipError_t dgrad_mfma(const uint16_t* planes, const uint16_t* w, int cin, int cout, int c0, int cpart, const PadGrid& P,
+                      uint16_t* wt, float* out, hipStream_t s)
+{
+  if (cpart % 16) return hipErrorInvalidValue;
+  const int CP = plane_channels(cout), kpad = plane_kpad(cout), K = 27 * CP;
+  hipLaunchKernelGGL(k_weights_planes, dim3(std::min<unsigned>(blocks_for(int64_t(cpart) * kpad), 2048)), dim3(kThreads),
+                     0, s, w, cin, cout, c0, cpart, CP, kpad, wt);
+  const size_t shmem = size_t(kpad / 8) * sizeof(int);
+  const dim3   block{unsigned(kThreads)};
+  if (P.nodes < kChannelParallelBelow) {
+    const dim3 g{unsigned((P.nodes + 15) / 16), unsigned(cpart / 16)};
+    hipLaunchKernelGGL((k_dgrad<1, 1, 4>), g, block, shmem, s, planes, CP, wt, kpad, K, P, out, cpart);
+  } else {
+    const unsigned tiles = unsigned((P.nodes + 15) / 16);
+    if (cpart % 64 == 0)
+      hipLaunchKernelGGL((k_dgrad<4, 1, 1>), dim3((tiles + 3) / 4, unsigned(cpart / 64)), block, shmem, s, planes, CP, wt,
+                         kpad, K, P, out, cpart);
+    else if (cpart % 32 == 0)
+      hipLaunchKernelGGL((k_dgrad<2, 2, 1>), dim3((tiles + 7) / 8, unsigned(cpart / 32)), block, shmem, s, planes, CP, wt,
+                         kpad, K, P, out, cpart);
+    else
+      hipLaunchKernelGGL((k_dgrad<1, 2, 1>), dim3((tiles + 7) / 8, unsigned(cpart / 16)), block, shmem, s, planes, CP, wt,
+                         kpad, K, P, out, cpart);
+  }
+  return hipGetLastError();
+}
+
+hipError_t wgrad_mfma(const uint16_t* x_cm, int cin, int cin_all, int ci_first, const uint16_t* g_cm, int cout,
+                      const PadGrid& P, float* dw, hipStream_t s)
+{
+  const int tiles = (cin + 15) / 16 * ((cout + 15) / 16), steps = (P.nodes + 31) / 32;
+  // about 768 workgroups, at least 8 steps each
+  const int runs = std::max(1, std::min(steps / 8, (768 + tiles - 1) / tiles));
+  const int per  = (steps + runs - 1) / runs;
+  hipLaunchKernelGGL(k_wgrad, dim3(unsigned((steps + per - 1) / per), unsigned(tiles)), dim3(kThreads), 0, s, x_cm, cin,
+                     g_cm, cout, P, per, dw, cin_all, ci_first);
+  return hipGetLastError();
+}
+
+hipError_t bias_grad(const float* g, const uint16_t* y, int64_t n, int cout, float* db, hipStream_t s)
+{
+  hipLaunchKernelGGL(k_bias_grad, dim3(std::min<unsigned>(blocks_for(n * cout), 256)), dim3(kThreads), 0, s, g, y, n,
+                     cout, db);
   return hipGetLastError();
 }
 
