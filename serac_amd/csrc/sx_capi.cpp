@@ -2358,15 +2358,6 @@ void mg_level_apply(sx_multigrid* M, sx_grad* g, const int32_t* ess, int64_t nes
   }
 }
 
-double mg_read_dot(sx_multigrid* M, const double* a, const double* b, int64_t n, hipStream_t s)
-{
-  SX_HIP(sxk::vec_dot_dev(a, b, n, M->part.as<double>(), M->scal.as<double>(), 0, 0, s));
-  double v = 0.0;
-  SX_HIP(hipMemcpyAsync(&v, M->scal.as<double>(), sizeof(double), hipMemcpyDeviceToHost, s));
-  SX_HIP(hipStreamSynchronize(s));
-  return v;
-}
-
 // dense inverse of the coarsest operator: symmetrised, constrained rows set to
 // identity, inverted by Gauss-Jordan elimination with partial pivoting
 void mg_coarse_inverse(sx_multigrid* M, hipStream_t s)
@@ -2546,9 +2537,9 @@ void mg_setup(sx_multigrid* M, sx_grad* g, const int32_t* ess, int64_t ness)
             mg_level_apply(M, g, ess, ness, l, F.d.as<double>(), F.t.as<double>());
             if (l == 0)
               SX_HIP(sxm::fe_restrict(M->G, F.t.as<double>(), C.r.as<double>(), C.mask.as<uint8_t>(), M->rt1.as<double>(),
-                                     M->rt2.as<double>(), s));
+                                     M->rt2.as<double>(), sxm::ChebStart{}, s));
             else
-              SX_HIP(sxm::grid_restrict(F.t.as<double>(), F.g, C.r.as<double>(), C.g, C.mask.as<uint8_t>(), s));
+              SX_HIP(sxm::grid_restrict(F.t.as<double>(), F.g, C.r.as<double>(), C.g, C.mask.as<uint8_t>(), sxm::ChebStart{}, s));
             SX_HIP(sxm::probe_extract(C.r.as<double>(), C.g, cx, cy, cz, ci, C.mask.as<uint8_t>(), C.S.as<double>(),
                                       s));
           }
@@ -2560,17 +2551,22 @@ void mg_setup(sx_multigrid* M, sx_grad* g, const int32_t* ess, int64_t ness)
     MgLevel& V = M->lv[size_t(l)];
     double*  v = V.d.as<double>();
     SX_HIP(sxm::seed_field(v, V.n, uint64_t(l + 1), V.mask.as<uint8_t>(), s));
-    double nrm = std::sqrt(mg_read_dot(M, v, v, V.n, s));
-    SX_REQUIRE(nrm > 0.0, SX_ERR_STATE, "multigrid: every DOF of a level is constrained");
-    SX_HIP(sxm::scale(v, 1.0 / nrm, V.n, s));
-    double lam = 0.0;
+    // the norms stay on the device, read once: scal[1] the start's, scal[0] the last step's
+    double *part = M->part.as<double>(), *scal = M->scal.as<double>();
+    SX_HIP(sxk::vec_dot_dev(v, v, V.n, part, scal, 1, 0, s));
+    SX_HIP(sxm::normalize(v, scal + 1, V.n, s));
     for (int it = 0; it < M->power_iters; it++) {
+      if (it > 0) SX_HIP(sxm::normalize(v, scal, V.n, s));
       mg_level_apply(M, g, ess, ness, l, v, V.t.as<double>());
       SX_HIP(sxm::mul_dinv(V.dinv.as<double>(), V.t.as<double>(), v, V.n, s));
-      lam = std::sqrt(mg_read_dot(M, v, v, V.n, s));
-      SX_REQUIRE(lam > 0.0 && std::isfinite(lam), SX_ERR_NOCONV, "multigrid: power iteration broke down");
-      SX_HIP(sxm::scale(v, 1.0 / lam, V.n, s));
+      SX_HIP(sxk::vec_dot_dev(v, v, V.n, part, scal, 0, 0, s));
     }
+    double h[2];
+    SX_HIP(hipMemcpyAsync(h, scal, sizeof(h), hipMemcpyDeviceToHost, s));
+    SX_HIP(hipStreamSynchronize(s));
+    SX_REQUIRE(h[1] > 0.0, SX_ERR_STATE, "multigrid: every DOF of a level is constrained");
+    const double lam = std::sqrt(h[0]);
+    SX_REQUIRE(lam > 0.0 && std::isfinite(lam), SX_ERR_NOCONV, "multigrid: power iteration broke down");
     V.lmax            = lam;
     const double up   = M->safety * lam, lo = up / M->range;
     const double th   = 0.5 * (up + lo), de = 0.5 * (up - lo), sigma = th / de;
@@ -2590,39 +2586,66 @@ void mg_setup(sx_multigrid* M, sx_grad* g, const int32_t* ess, int64_t ness)
   M->setups++;
 }
 
-// Chebyshev smoothing of A_l x = b: from x = 0 (pre; leaves r = b - A x) or
-// from the current x (post)
-void mg_smooth(sx_multigrid* M, sx_grad* g, const int32_t* ess, int64_t ness, int l, const double* b, double* x,
-               bool pre)
+// The start of level l's smoothing, for the restriction that makes its right
+// side (none on the coarsest level, which is solved).
+sxm::ChebStart mg_start(sx_multigrid* M, size_t l)
 {
-  MgLevel&    V = M->lv[size_t(l)];
+  sxm::ChebStart st;
+  if (l + 1 == M->lv.size()) return st;
+  MgLevel& V = M->lv[l];
+  st.dinv    = V.dinv.as<const double>();
+  st.inv_theta = 1.0 / V.theta;
+  st.x       = V.x.as<double>();
+  st.d       = V.d.as<double>();
+  st.r       = V.r.as<double>();
+  return st;
+}
+
+// Chebyshev smoothing of a vertex level's A x = b: from x = 0, started by the
+// restriction (pre; leaves r = b - A x), or from the current x (post).  Every
+// product with the stencil carries the vector updates around it: two passes
+// each way at degree 2 where products and updates apart took five.
+void mg_smooth_vertex(sx_multigrid* M, hipStream_t s, int l, bool pre)
+{
+  MgLevel&      V = M->lv[size_t(l)];
+  const double *S = V.S.as<const double>(), *dinv = V.dinv.as<const double>();
+  double *      x = V.x.as<double>(), *r = V.r.as<double>(), *d = V.d.as<double>(), *d_new = V.t.as<double>();
+  if (!pre) SX_HIP(sxm::stencil_cheb_restart(S, V.g, x, V.b.as<const double>(), r, d, dinv, V.theta, s));
+  for (size_t k = 0; k < V.c1.size(); k++) {
+    SX_HIP(sxm::stencil_cheb_step(S, V.g, d, d_new, r, dinv, V.c1[k], V.c2[k], x, !pre && k == 0, s));
+    std::swap(d, d_new);
+  }
+  if (!pre && V.c1.empty()) SX_HIP(sxk::vec_axpy(1.0, d, x, V.n, s));
+  if (pre) SX_HIP(sxm::stencil_residual(S, V.g, d, r, s));
+}
+
+// The same on level 0 (FP64 vectors).  t = J d is taken as it comes: the steps
+// keep the essential rows, where dinv is zero.
+void mg_smooth0(sx_multigrid* M, sx_grad* g, const double* b, double* x, bool pre)
+{
+  MgLevel&    V = M->lv[0];
   hipStream_t s = g->form->stream;
-  double *    r = V.r.as<double>(), *d = V.d.as<double>(), *t = V.t.as<double>();
+  double *    r = V.r.as<double>(), *d = V.d.as<double>(), *t = V.t.as<double>(), *dinv = V.dinv.as<double>();
+  auto        apply = [&](const double* in) {
+    apply_gradient(g, in, t, nullptr, nullptr, sxk::PREC_F64, false, M->lo_active);
+  };
   if (pre) {
-    SX_HIP(sxm::cheb_init(b, V.dinv.as<double>(), V.theta, x, d, r, 0, 1, V.n, s));
+    SX_HIP(sxm::cheb_init(b, dinv, V.theta, x, d, r, V.n, s));
   } else {
-    mg_level_apply(M, g, ess, ness, l, x, t);
-    SX_HIP(sxm::residual(b, t, r, V.n, s));
-    SX_HIP(sxm::cheb_init(r, V.dinv.as<double>(), V.theta, x, d, r, 1, 0, V.n, s));
+    apply(x);
+    SX_HIP(sxm::cheb_restart(b, t, dinv, V.theta, x, d, r, V.n, s));
   }
   for (size_t k = 0; k < V.c1.size(); k++) {
-    mg_level_apply(M, g, ess, ness, l, d, t);
-    SX_HIP(sxm::cheb_step(r, t, d, V.dinv.as<double>(), V.c1[k], V.c2[k], x, V.n, s));
+    apply(d);
+    SX_HIP(sxm::cheb_step(r, t, d, dinv, V.c1[k], V.c2[k], x, V.n, s));
   }
   if (pre) {
-    mg_level_apply(M, g, ess, ness, l, d, t);
-    SX_HIP(sxm::sub_inplace(r, t, V.n, s));
+    apply(d);
+    SX_HIP(sxm::cheb_residual(r, t, dinv, V.n, s));
   }
 }
 
-// y = A_0 x on FP32 vectors (x is zero on the essential rows)
-void mg_level0_apply_f32(sx_multigrid* M, sx_grad* g, const float* x, float* y)
-{
-  apply_gradient(g, x, y, nullptr, nullptr, sxk::PREC_F32, false, M->lo_active);
-  SX_HIP(sxm::apply_mask(y, M->lv[0].mask.as<uint8_t>(), M->lv[0].n, g->form->stream));
-}
-
-// mg_smooth on level 0 with FP32 vectors (b = fb, x = fx)
+// mg_smooth0 with FP32 vectors (b = fb, x = fx)
 void mg_smooth0_f32(sx_multigrid* M, sx_grad* g, bool pre)
 {
   MgLevel&      V = M->lv[0];
@@ -2630,64 +2653,68 @@ void mg_smooth0_f32(sx_multigrid* M, sx_grad* g, bool pre)
   const int64_t n = V.n;
   float *b = M->fb.as<float>(), *x = M->fx.as<float>(), *r = M->fr.as<float>(), *d = M->fd.as<float>(),
         *t = M->ft.as<float>(), *dinv = M->fdinv.as<float>();
+  auto apply = [&](const float* in) {
+    apply_gradient(g, in, t, nullptr, nullptr, sxk::PREC_F32, false, M->lo_active);
+  };
   if (pre) {
-    SX_HIP(sxm::cheb_init(b, dinv, V.theta, x, d, r, 0, 1, n, s));
+    SX_HIP(sxm::cheb_init(b, dinv, V.theta, x, d, r, n, s));
   } else {
-    mg_level0_apply_f32(M, g, x, t);
-    SX_HIP(sxm::residual(b, t, r, n, s));
-    SX_HIP(sxm::cheb_init(r, dinv, V.theta, x, d, r, 1, 0, n, s));
+    apply(x);
+    SX_HIP(sxm::cheb_restart(b, t, dinv, V.theta, x, d, r, n, s));
   }
   for (size_t k = 0; k < V.c1.size(); k++) {
-    mg_level0_apply_f32(M, g, d, t);
+    apply(d);
     SX_HIP(sxm::cheb_step(r, t, d, dinv, V.c1[k], V.c2[k], x, n, s));
   }
   if (pre) {
-    mg_level0_apply_f32(M, g, d, t);
-    SX_HIP(sxm::sub_inplace(r, t, n, s));
+    apply(d);
+    SX_HIP(sxm::cheb_residual(r, t, dinv, n, s));
   }
 }
 
-void mg_vcycle(sx_multigrid* M, sx_grad* g, const int32_t* ess, int64_t ness, int l, const double* b, double* x);
+// x_l = V-cycle(b_l) on vertex level l, its right side and the start of its
+// smoothing left by the restriction
+void mg_vcycle_vertex(sx_multigrid* M, hipStream_t s, size_t l)
+{
+  MgLevel& V = M->lv[l];
+  if (l + 1 == M->lv.size()) {
+    SX_HIP(sxm::dense_mv(M->coarse_inv.as<double>(), M->ncoarse, V.b.as<double>(), V.x.as<double>(), s));
+    return;
+  }
+  MgLevel& C = M->lv[l + 1];
+  mg_smooth_vertex(M, s, int(l), true);
+  SX_HIP(sxm::grid_restrict(V.r.as<double>(), V.g, C.b.as<double>(), C.g, C.mask.as<uint8_t>(), mg_start(M, l + 1), s));
+  mg_vcycle_vertex(M, s, l + 1);
+  SX_HIP(sxm::grid_prolong_add(C.x.as<double>(), C.g, V.x.as<double>(), V.g, V.mask.as<uint8_t>(), s));
+  mg_smooth_vertex(M, s, int(l), false);
+}
 
 // level 0 of the V-cycle on FP32 vectors: fx = V(fb)
-void mg_vcycle0_f32(sx_multigrid* M, sx_grad* g, const int32_t* ess, int64_t ness)
+void mg_vcycle0_f32(sx_multigrid* M, sx_grad* g)
 {
   hipStream_t s = g->form->stream;
   MgLevel&    C = M->lv[1];
   mg_smooth0_f32(M, g, true);
   SX_HIP(sxm::fe_restrict(M->G, M->fr.as<float>(), C.b.as<double>(), C.mask.as<uint8_t>(), M->rt1.as<double>(),
-                          M->rt2.as<double>(), s));
-  mg_vcycle(M, g, ess, ness, 1, C.b.as<double>(), C.x.as<double>());
+                          M->rt2.as<double>(), mg_start(M, 1), s));
+  mg_vcycle_vertex(M, s, 1);
   SX_HIP(sxm::fe_prolong_add(M->G, C.x.as<double>(), M->fx.as<float>(), s));
   SX_HIP(sxm::apply_mask(M->fx.as<float>(), M->lv[0].mask.as<uint8_t>(), M->lv[0].n, s));
   mg_smooth0_f32(M, g, false);
 }
 
-// x = V-cycle(b) on level l (x is overwritten)
-void mg_vcycle(sx_multigrid* M, sx_grad* g, const int32_t* ess, int64_t ness, int l, const double* b, double* x)
+// x = V-cycle(b) from level 0 (x is overwritten)
+void mg_vcycle(sx_multigrid* M, sx_grad* g, const int32_t* ess, int64_t ness, const double* b, double* x)
 {
   hipStream_t s = g->form->stream;
-  const int   L = int(M->lv.size());
-  MgLevel&    V = M->lv[size_t(l)];
-  if (l == L - 1) {
-    SX_HIP(sxm::dense_mv(M->coarse_inv.as<double>(), M->ncoarse, b, x, s));
-    return;
-  }
-  MgLevel& C = M->lv[size_t(l + 1)];
-  mg_smooth(M, g, ess, ness, l, b, x, true);
-  if (l == 0)
-    SX_HIP(sxm::fe_restrict(M->G, V.r.as<double>(), C.b.as<double>(), C.mask.as<uint8_t>(), M->rt1.as<double>(),
-                             M->rt2.as<double>(), s));
-  else
-    SX_HIP(sxm::grid_restrict(V.r.as<double>(), V.g, C.b.as<double>(), C.g, C.mask.as<uint8_t>(), s));
-  mg_vcycle(M, g, ess, ness, l + 1, C.b.as<double>(), C.x.as<double>());
-  if (l == 0) {
-    SX_HIP(sxm::fe_prolong_add(M->G, C.x.as<double>(), x, s));
-    SX_HIP(sxk::set_rows(x, ess, ness, 0.0, s));
-  } else {
-    SX_HIP(sxm::grid_prolong_add(C.x.as<double>(), C.g, x, V.g, V.mask.as<uint8_t>(), s));
-  }
-  mg_smooth(M, g, ess, ness, l, b, x, false);
+  MgLevel &   V = M->lv[0], &C = M->lv[1];
+  mg_smooth0(M, g, b, x, true);
+  SX_HIP(sxm::fe_restrict(M->G, V.r.as<double>(), C.b.as<double>(), C.mask.as<uint8_t>(), M->rt1.as<double>(),
+                          M->rt2.as<double>(), mg_start(M, 1), s));
+  mg_vcycle_vertex(M, s, 1);
+  SX_HIP(sxm::fe_prolong_add(M->G, C.x.as<double>(), x, s));
+  SX_HIP(sxk::set_rows(x, ess, ness, 0.0, s));
+  mg_smooth0(M, g, b, x, false);
 }
 
 // z = M r: the V-cycle on the free DOFs, the identity on the essential ones
@@ -2697,14 +2724,14 @@ void mg_apply(sx_multigrid* M, sx_grad* g, const int32_t* ess, int64_t ness, con
   MgLevel&    l0 = M->lv[0];
   if (M->smoother_f32 && M->fb.ptr) {
     SX_HIP(sxm::to_f32(r, M->fb.as<float>(), l0.mask.as<uint8_t>(), l0.n, s));
-    mg_vcycle0_f32(M, g, ess, ness);
+    mg_vcycle0_f32(M, g);
     SX_HIP(sxm::to_f64(M->fx.as<float>(), z, l0.n, s));
     SX_HIP(sxk::copy_rows(z, r, ess, ness, s));
     return;
   }
   SX_HIP(hipMemcpyAsync(l0.b.ptr, r, size_t(l0.n) * 8, hipMemcpyDeviceToDevice, s));
   SX_HIP(sxk::set_rows(l0.b.as<double>(), ess, ness, 0.0, s));
-  mg_vcycle(M, g, ess, ness, 0, l0.b.as<double>(), z);
+  mg_vcycle(M, g, ess, ness, l0.b.as<double>(), z);
   SX_HIP(sxk::copy_rows(z, r, ess, ness, s));
 }
 

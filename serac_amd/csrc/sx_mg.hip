@@ -33,18 +33,31 @@ __device__ __forceinline__ double fe_weight(const sxu::FEGrid& G, int d)
   return d >= 0 ? 1.0 - G.xi[d] : G.xi[G.p + d];
 }
 
+// b's entry t of a level whose smoothing from zero starts here (start.x set):
+// d = dinv b / theta, x = d, r = b
+__device__ __forceinline__ void start_smoothing(const ChebStart& st, int64_t t, double b)
+{
+  if (st.x == nullptr) return;
+  const double d = st.dinv[t] * b * st.inv_theta;
+  st.x[t]        = d;
+  st.d[t]        = d;
+  st.r[t]        = b;
+}
+
 // One direction of the separable restriction P^T = Rz Ry Rx: out has the
 // dims of in except nv[dir] along dir, out(i) = sum_d w(d) in(p i + d).  The
 // last pass (dir 2) applies the vertex mask.
 template <typename TI>
 __global__ void __launch_bounds__(kThreads) k_fe_restrict_dir(sxu::FEGrid G, const TI* in, Grid3 din, double* out,
-                                                              Grid3 dout, int dir, const uint8_t* mask)
+                                                              Grid3 dout, int dir, const uint8_t* mask,
+                                                              ChebStart start)
 {
   const int64_t n      = int64_t(dout.n[0]) * dout.n[1] * dout.n[2] * 3;
   const int64_t stride = dir == 0 ? 3 : (dir == 1 ? int64_t(din.n[0]) * 3 : int64_t(din.n[0]) * din.n[1] * 3);
   for (int64_t t = int64_t(blockIdx.x) * kThreads + threadIdx.x; t < n; t += int64_t(gridDim.x) * kThreads) {
     if (mask && mask[t]) {
       out[t] = 0.0;
+      start_smoothing(start, t, 0.0);
       continue;
     }
     const int c = int(t % 3);
@@ -61,6 +74,7 @@ __global__ void __launch_bounds__(kThreads) k_fe_restrict_dir(sxu::FEGrid G, con
       s += fe_weight(G, d) * double(base[int64_t(d) * stride]);
     }
     out[t] = s;
+    start_smoothing(start, t, s);
   }
 }
 
@@ -91,12 +105,13 @@ __global__ void __launch_bounds__(kThreads) k_fe_prolong_add(sxu::FEGrid G, cons
 }
 
 __global__ void __launch_bounds__(kThreads) k_grid_restrict(const double* rf, Grid3 f, double* rc, Grid3 c,
-                                                            const uint8_t* maskc)
+                                                            const uint8_t* maskc, ChebStart start)
 {
   const int64_t nc = nverts(c);
   for (int64_t t = int64_t(blockIdx.x) * kThreads + threadIdx.x; t < nc * 3; t += int64_t(gridDim.x) * kThreads) {
     if (maskc[t]) {
       rc[t] = 0.0;
+      start_smoothing(start, t, 0.0);
       continue;
     }
     const int comp = int(t % 3);
@@ -119,6 +134,7 @@ __global__ void __launch_bounds__(kThreads) k_grid_restrict(const double* rf, Gr
       }
     }
     rc[t] = s;
+    start_smoothing(start, t, s);
   }
 }
 
@@ -150,34 +166,72 @@ __global__ void __launch_bounds__(kThreads) k_grid_prolong_add(const double* ec,
   }
 }
 
-__global__ void __launch_bounds__(kThreads) k_stencil_apply(const double* S, Grid3 g, const double* x, double* y)
+// t = S x at every vertex, and what the smoother does with t there:
+//   APPLY: y = t
+//   STEP:  r -= t; d = c1 x + c2 dinv r into y; sol += d (and += x with `both`)
+//   SUB:   r -= t
+//   START: r = b - t; d = dinv r c1 into y
+// (x is d in STEP and SUB; neighbours read it, so the new d goes to another
+// array, and START leaves the sum sol + d to the next step for the same
+// reason.)  A workgroup takes 64 vertices; each of its nine waves takes the
+// three neighbours of one (y, z) offset, so a vertex's 27 x 9 coefficients are
+// in flight at once instead of one after another, and the parts meet in LDS
+// in a fixed order.  What bounds it: latency up to 33^3 vertices (25^3, 13^3 and 7^3
+// together: 14.5 us a product with a thread per vertex, and 4 us for each
+// vector update around it; 5.3 to 6.1 us now with the updates inside), the
+// coefficients' bytes above (65^3: 534 MB).
+enum StencilMode { ST_APPLY, ST_STEP, ST_SUB, ST_START };
+constexpr int kStencilWaves = 9;
+
+template <int MODE>
+__global__ void __launch_bounds__(64 * kStencilWaves) k_stencil(const double* S, Grid3 g, const double* x, double* y,
+                                                                double* r, const double* b, const double* dinv,
+                                                                double* sol, double c1, double c2, int both)
 {
-  const int64_t nv = nverts(g);
-  for (int64_t v = int64_t(blockIdx.x) * kThreads + threadIdx.x; v < nv; v += int64_t(gridDim.x) * kThreads) {
+  __shared__ double part[kStencilWaves][64 * 3];
+  const int64_t     nv = nverts(g);
+  const int         lane = int(threadIdx.x) & 63, wave = int(threadIdx.x) >> 6;
+  const int64_t     v = int64_t(blockIdx.x) * 64 + lane;
+  double            a0 = 0.0, a1 = 0.0, a2 = 0.0;
+  if (v < nv) {
     int ix, iy, iz;
     coords(g, v, ix, iy, iz);
-    double a0 = 0.0, a1 = 0.0, a2 = 0.0;
-    for (int oz = -1; oz <= 1; oz++) {
-      const int jz = iz + oz;
-      if (jz < 0 || jz >= g.n[2]) continue;
-      for (int oy = -1; oy <= 1; oy++) {
-        const int jy = iy + oy;
-        if (jy < 0 || jy >= g.n[1]) continue;
-        for (int ox = -1; ox <= 1; ox++) {
-          const int jx = ix + ox;
-          if (jx < 0 || jx >= g.n[0]) continue;
-          const int64_t j  = (int64_t(jz) * g.n[1] + jy) * g.n[0] + jx;
-          const double  x0 = x[j * 3], x1 = x[j * 3 + 1], x2 = x[j * 3 + 2];
-          const double* s  = S + int64_t((oz + 1) * 9 + (oy + 1) * 3 + (ox + 1)) * 9 * nv + v;
-          a0 += s[0] * x0 + s[nv] * x1 + s[2 * nv] * x2;
-          a1 += s[3 * nv] * x0 + s[4 * nv] * x1 + s[5 * nv] * x2;
-          a2 += s[6 * nv] * x0 + s[7 * nv] * x1 + s[8 * nv] * x2;
-        }
+    const int jy = iy + wave % 3 - 1, jz = iz + wave / 3 - 1;
+    if (jy >= 0 && jy < g.n[1] && jz >= 0 && jz < g.n[2]) {
+#pragma unroll
+      for (int ox = -1; ox <= 1; ox++) {
+        const int jx = ix + ox;
+        if (jx < 0 || jx >= g.n[0]) continue;
+        const int64_t j  = (int64_t(jz) * g.n[1] + jy) * g.n[0] + jx;
+        const double  x0 = x[j * 3], x1 = x[j * 3 + 1], x2 = x[j * 3 + 2];
+        const double* s  = S + int64_t(wave * 3 + ox + 1) * 9 * nv + v;
+        a0 += s[0] * x0 + s[nv] * x1 + s[2 * nv] * x2;
+        a1 += s[3 * nv] * x0 + s[4 * nv] * x1 + s[5 * nv] * x2;
+        a2 += s[6 * nv] * x0 + s[7 * nv] * x1 + s[8 * nv] * x2;
       }
     }
-    y[v * 3]     = a0;
-    y[v * 3 + 1] = a1;
-    y[v * 3 + 2] = a2;
+  }
+  part[wave][lane * 3]     = a0;
+  part[wave][lane * 3 + 1] = a1;
+  part[wave][lane * 3 + 2] = a2;
+  __syncthreads();
+  const int64_t i = int64_t(blockIdx.x) * 192 + threadIdx.x;
+  if (threadIdx.x >= 192 || i >= nv * 3) return;
+  double t = 0.0;
+#pragma unroll
+  for (int w = 0; w < kStencilWaves; w++) t += part[w][threadIdx.x];
+  if constexpr (MODE == ST_APPLY) y[i] = t;
+  if constexpr (MODE == ST_SUB) r[i] -= t;
+  if constexpr (MODE == ST_STEP) {
+    const double ri = r[i] - t, di = x[i], dn = c1 * di + c2 * dinv[i] * ri;
+    r[i]            = ri;
+    y[i]            = dn;
+    sol[i] += both ? di + dn : dn;
+  }
+  if constexpr (MODE == ST_START) {
+    const double ri = b[i] - t;
+    r[i]            = ri;
+    y[i]            = dinv[i] * ri * c1;
   }
 }
 
@@ -269,17 +323,34 @@ __global__ void __launch_bounds__(kThreads) k_coarsen_mask(const uint8_t* mf, Gr
   }
 }
 
+// Level-0 smoothing steps.  t = J d has values on the essential rows, where
+// dinv is zero: r stays zero there.
 template <typename T>
-__global__ void __launch_bounds__(kThreads) k_cheb_init(const T* b, const T* dinv, double inv_theta, T* x, T* d,
-                                                        T* r, int x_add, int copy_r, int64_t n)
+__global__ void __launch_bounds__(kThreads) k_cheb_init(const T* b, const T* dinv, double inv_theta, T* x, T* d, T* r,
+                                                        int64_t n)
 {
   const T it = T(inv_theta);
   for (int64_t i = int64_t(blockIdx.x) * kThreads + threadIdx.x; i < n; i += int64_t(gridDim.x) * kThreads) {
     const T bi = b[i];
     const T di = dinv[i] * bi * it;
     d[i]       = di;
-    x[i]       = x_add ? x[i] + di : di;
-    if (copy_r) r[i] = bi;
+    x[i]       = di;
+    r[i]       = bi;
+  }
+}
+
+template <typename T>
+__global__ void __launch_bounds__(kThreads) k_cheb_restart(const T* b, const T* t, const T* dinv, double inv_theta,
+                                                           T* x, T* d, T* r, int64_t n)
+{
+  const T it = T(inv_theta);
+  for (int64_t i = int64_t(blockIdx.x) * kThreads + threadIdx.x; i < n; i += int64_t(gridDim.x) * kThreads) {
+    const T inv = dinv[i];
+    const T ri  = inv == T(0) ? T(0) : b[i] - t[i];
+    const T di  = inv * ri * it;
+    r[i]        = ri;
+    d[i]        = di;
+    x[i] += di;
   }
 }
 
@@ -289,26 +360,20 @@ __global__ void __launch_bounds__(kThreads) k_cheb_step(T* r, const T* t, T* d, 
 {
   const T a = T(c1), b = T(c2);
   for (int64_t i = int64_t(blockIdx.x) * kThreads + threadIdx.x; i < n; i += int64_t(gridDim.x) * kThreads) {
-    const T ri = r[i] - t[i];
-    r[i]       = ri;
-    const T di = a * d[i] + b * dinv[i] * ri;
-    d[i]       = di;
+    const T inv = dinv[i];
+    const T ri  = inv == T(0) ? T(0) : r[i] - t[i];
+    r[i]        = ri;
+    const T di  = a * d[i] + b * inv * ri;
+    d[i]        = di;
     x[i] += di;
   }
 }
 
 template <typename T>
-__global__ void __launch_bounds__(kThreads) k_residual(const T* b, const T* t, T* r, int64_t n)
+__global__ void __launch_bounds__(kThreads) k_cheb_residual(T* r, const T* t, const T* dinv, int64_t n)
 {
   for (int64_t i = int64_t(blockIdx.x) * kThreads + threadIdx.x; i < n; i += int64_t(gridDim.x) * kThreads)
-    r[i] = b[i] - t[i];
-}
-
-template <typename T>
-__global__ void __launch_bounds__(kThreads) k_sub_inplace(T* r, const T* t, int64_t n)
-{
-  for (int64_t i = int64_t(blockIdx.x) * kThreads + threadIdx.x; i < n; i += int64_t(gridDim.x) * kThreads)
-    r[i] -= t[i];
+    r[i] = dinv[i] == T(0) ? T(0) : r[i] - t[i];
 }
 
 template <typename T>
@@ -380,8 +445,10 @@ __global__ void __launch_bounds__(kThreads) k_mul_dinv(const double* dinv, const
     v[i] = dinv[i] * t[i];
 }
 
-__global__ void __launch_bounds__(kThreads) k_scale(double* v, double a, int64_t n)
+// v /= sqrt(*norm2)
+__global__ void __launch_bounds__(kThreads) k_normalize(double* v, const double* norm2, int64_t n)
 {
+  const double a = 1.0 / sqrt(*norm2);
   for (int64_t i = int64_t(blockIdx.x) * kThreads + threadIdx.x; i < n; i += int64_t(gridDim.x) * kThreads)
     v[i] *= a;
 }
@@ -620,19 +687,27 @@ int64_t fe_restrict_scratch(const sxu::FEGrid& G, int pass)
   return pass == 0 ? int64_t(G.nn[2]) * G.nn[1] * G.nv[0] * 3 : int64_t(G.nn[2]) * G.nv[1] * G.nv[0] * 3;
 }
 
-hipError_t fe_restrict(const sxu::FEGrid& G, const double* r, double* rc, const uint8_t* mask, double* t1, double* t2,
-                       hipStream_t s)
+template <typename T>
+static hipError_t launch_fe_restrict(const sxu::FEGrid& G, const T* r, double* rc, const uint8_t* mask, double* t1,
+                                     double* t2, const ChebStart& start, hipStream_t s)
 {
   const Grid3 d0{{G.nn[0], G.nn[1], G.nn[2]}}, d1{{G.nv[0], G.nn[1], G.nn[2]}}, d2{{G.nv[0], G.nv[1], G.nn[2]}},
       d3{{G.nv[0], G.nv[1], G.nv[2]}};
-  const uint8_t* none = nullptr;
-  hipLaunchKernelGGL(k_fe_restrict_dir<double>, dim3(blocks_for(fe_restrict_scratch(G, 0))), dim3(kThreads), 0, s, G, r, d0,
-                     t1, d1, 0, none);
-  hipLaunchKernelGGL(k_fe_restrict_dir<double>, dim3(blocks_for(fe_restrict_scratch(G, 1))), dim3(kThreads), 0, s, G, t1, d1,
-                     t2, d2, 1, none);
-  hipLaunchKernelGGL(k_fe_restrict_dir<double>, dim3(blocks_for(int64_t(G.nv[0]) * G.nv[1] * G.nv[2] * 3)), dim3(kThreads), 0,
-                     s, G, t2, d2, rc, d3, 2, mask);
+  const uint8_t*  none = nullptr;
+  const ChebStart no_start{};
+  hipLaunchKernelGGL(k_fe_restrict_dir<T>, dim3(blocks_for(fe_restrict_scratch(G, 0))), dim3(kThreads), 0, s, G, r, d0,
+                     t1, d1, 0, none, no_start);
+  hipLaunchKernelGGL(k_fe_restrict_dir<double>, dim3(blocks_for(fe_restrict_scratch(G, 1))), dim3(kThreads), 0, s, G,
+                     static_cast<const double*>(t1), d1, t2, d2, 1, none, no_start);
+  hipLaunchKernelGGL(k_fe_restrict_dir<double>, dim3(blocks_for(int64_t(G.nv[0]) * G.nv[1] * G.nv[2] * 3)),
+                     dim3(kThreads), 0, s, G, static_cast<const double*>(t2), d2, rc, d3, 2, mask, start);
   return hipGetLastError();
+}
+
+hipError_t fe_restrict(const sxu::FEGrid& G, const double* r, double* rc, const uint8_t* mask, double* t1, double* t2,
+                       const ChebStart& start, hipStream_t s)
+{
+  return launch_fe_restrict(G, r, rc, mask, t1, t2, start, s);
 }
 
 hipError_t fe_prolong_add(const sxu::FEGrid& G, const double* ec, double* z, hipStream_t s)
@@ -642,10 +717,11 @@ hipError_t fe_prolong_add(const sxu::FEGrid& G, const double* ec, double* z, hip
   return hipGetLastError();
 }
 
-hipError_t grid_restrict(const double* rf, Grid3 f, double* rc, Grid3 c, const uint8_t* maskc, hipStream_t s)
+hipError_t grid_restrict(const double* rf, Grid3 f, double* rc, Grid3 c, const uint8_t* maskc, const ChebStart& start,
+                         hipStream_t s)
 {
   const int64_t n = int64_t(c.n[0]) * c.n[1] * c.n[2] * 3;
-  hipLaunchKernelGGL(k_grid_restrict, dim3(blocks_for(n)), dim3(kThreads), 0, s, rf, f, rc, c, maskc);
+  hipLaunchKernelGGL(k_grid_restrict, dim3(blocks_for(n)), dim3(kThreads), 0, s, rf, f, rc, c, maskc, start);
   return hipGetLastError();
 }
 
@@ -656,10 +732,41 @@ hipError_t grid_prolong_add(const double* ec, Grid3 c, double* zf, Grid3 f, cons
   return hipGetLastError();
 }
 
+static unsigned stencil_blocks(const Grid3& g) { return unsigned((int64_t(g.n[0]) * g.n[1] * g.n[2] + 63) / 64); }
+
 hipError_t stencil_apply(const double* S, Grid3 g, const double* x, double* y, hipStream_t s)
 {
-  const int64_t n = int64_t(g.n[0]) * g.n[1] * g.n[2];
-  hipLaunchKernelGGL(k_stencil_apply, dim3(blocks_for(n)), dim3(kThreads), 0, s, S, g, x, y);
+  const double* none = nullptr;
+  double*       no   = nullptr;
+  hipLaunchKernelGGL(k_stencil<ST_APPLY>, dim3(stencil_blocks(g)), dim3(64 * kStencilWaves), 0, s, S, g, x, y, no, none,
+                     none, no, 0.0, 0.0, 0);
+  return hipGetLastError();
+}
+
+hipError_t stencil_cheb_step(const double* S, Grid3 g, const double* d, double* d_new, double* r, const double* dinv,
+                             double c1, double c2, double* x, bool both, hipStream_t s)
+{
+  const double* none = nullptr;
+  hipLaunchKernelGGL(k_stencil<ST_STEP>, dim3(stencil_blocks(g)), dim3(64 * kStencilWaves), 0, s, S, g, d, d_new, r,
+                     none, dinv, x, c1, c2, int(both));
+  return hipGetLastError();
+}
+
+hipError_t stencil_residual(const double* S, Grid3 g, const double* d, double* r, hipStream_t s)
+{
+  const double* none = nullptr;
+  double*       no   = nullptr;
+  hipLaunchKernelGGL(k_stencil<ST_SUB>, dim3(stencil_blocks(g)), dim3(64 * kStencilWaves), 0, s, S, g, d, no, r, none,
+                     none, no, 0.0, 0.0, 0);
+  return hipGetLastError();
+}
+
+hipError_t stencil_cheb_restart(const double* S, Grid3 g, const double* x, const double* b, double* r, double* d,
+                                const double* dinv, double theta, hipStream_t s)
+{
+  double* no = nullptr;
+  hipLaunchKernelGGL(k_stencil<ST_START>, dim3(stencil_blocks(g)), dim3(64 * kStencilWaves), 0, s, S, g, x, d, r, b,
+                     dinv, no, 1.0 / theta, 0.0, 0);
   return hipGetLastError();
 }
 
@@ -713,11 +820,9 @@ hipError_t coarsen_mask(const uint8_t* mf, Grid3 f, uint8_t* mc, Grid3 c, hipStr
   return hipGetLastError();
 }
 
-hipError_t cheb_init(const double* b, const double* dinv, double theta, double* x, double* d, double* r, int x_add,
-                     int copy_r, int64_t n, hipStream_t s)
+hipError_t cheb_init(const double* b, const double* dinv, double theta, double* x, double* d, double* r, int64_t n, hipStream_t s)
 {
-  hipLaunchKernelGGL(k_cheb_init<double>, dim3(blocks_for(n)), dim3(kThreads), 0, s, b, dinv, 1.0 / theta, x, d, r, x_add,
-                     copy_r, n);
+  hipLaunchKernelGGL(k_cheb_init<double>, dim3(blocks_for(n)), dim3(kThreads), 0, s, b, dinv, 1.0 / theta, x, d, r, n);
   return hipGetLastError();
 }
 
@@ -728,15 +833,15 @@ hipError_t cheb_step(double* r, const double* t, double* d, const double* dinv, 
   return hipGetLastError();
 }
 
-hipError_t residual(const double* b, const double* t, double* r, int64_t n, hipStream_t s)
+hipError_t cheb_restart(const double* b, const double* t, const double* dinv, double theta, double* x, double* d, double* r, int64_t n, hipStream_t s)
 {
-  hipLaunchKernelGGL(k_residual<double>, dim3(blocks_for(n)), dim3(kThreads), 0, s, b, t, r, n);
+  hipLaunchKernelGGL(k_cheb_restart<double>, dim3(blocks_for(n)), dim3(kThreads), 0, s, b, t, dinv, 1.0 / theta, x, d, r, n);
   return hipGetLastError();
 }
 
-hipError_t sub_inplace(double* r, const double* t, int64_t n, hipStream_t s)
+hipError_t cheb_residual(double* r, const double* t, const double* dinv, int64_t n, hipStream_t s)
 {
-  hipLaunchKernelGGL(k_sub_inplace<double>, dim3(blocks_for(n)), dim3(kThreads), 0, s, r, t, n);
+  hipLaunchKernelGGL(k_cheb_residual<double>, dim3(blocks_for(n)), dim3(kThreads), 0, s, r, t, dinv, n);
   return hipGetLastError();
 }
 
@@ -768,9 +873,9 @@ hipError_t mul_dinv(const double* dinv, const double* t, double* v, int64_t n, h
   return hipGetLastError();
 }
 
-hipError_t scale(double* v, double a, int64_t n, hipStream_t s)
+hipError_t normalize(double* v, const double* norm2, int64_t n, hipStream_t s)
 {
-  hipLaunchKernelGGL(k_scale, dim3(blocks_for(n)), dim3(kThreads), 0, s, v, a, n);
+  hipLaunchKernelGGL(k_normalize, dim3(blocks_for(n)), dim3(kThreads), 0, s, v, norm2, n);
   return hipGetLastError();
 }
 
@@ -859,18 +964,9 @@ hipError_t vertex_compatible(const sxu::FEGrid& G, const int32_t* rows, int64_t 
 
 // FP32 level-0 vectors
 hipError_t fe_restrict(const sxu::FEGrid& G, const float* r, double* rc, const uint8_t* mask, double* t1, double* t2,
-                       hipStream_t s)
+                       const ChebStart& start, hipStream_t s)
 {
-  const Grid3 d0{{G.nn[0], G.nn[1], G.nn[2]}}, d1{{G.nv[0], G.nn[1], G.nn[2]}}, d2{{G.nv[0], G.nv[1], G.nn[2]}},
-      d3{{G.nv[0], G.nv[1], G.nv[2]}};
-  const uint8_t* none = nullptr;
-  hipLaunchKernelGGL(k_fe_restrict_dir<float>, dim3(blocks_for(fe_restrict_scratch(G, 0))), dim3(kThreads), 0, s, G, r,
-                     d0, t1, d1, 0, none);
-  hipLaunchKernelGGL(k_fe_restrict_dir<double>, dim3(blocks_for(fe_restrict_scratch(G, 1))), dim3(kThreads), 0, s, G,
-                     static_cast<const double*>(t1), d1, t2, d2, 1, none);
-  hipLaunchKernelGGL(k_fe_restrict_dir<double>, dim3(blocks_for(int64_t(G.nv[0]) * G.nv[1] * G.nv[2] * 3)),
-                     dim3(kThreads), 0, s, G, static_cast<const double*>(t2), d2, rc, d3, 2, mask);
-  return hipGetLastError();
+  return launch_fe_restrict(G, r, rc, mask, t1, t2, start, s);
 }
 hipError_t fe_prolong_add(const sxu::FEGrid& G, const double* ec, float* z, hipStream_t s)
 {
@@ -878,11 +974,9 @@ hipError_t fe_prolong_add(const sxu::FEGrid& G, const double* ec, float* z, hipS
   hipLaunchKernelGGL(k_fe_prolong_add<float>, dim3(blocks_for(n)), dim3(kThreads), 0, s, G, ec, z);
   return hipGetLastError();
 }
-hipError_t cheb_init(const float* b, const float* dinv, double theta, float* x, float* d, float* r, int x_add,
-                     int copy_r, int64_t n, hipStream_t s)
+hipError_t cheb_init(const float* b, const float* dinv, double theta, float* x, float* d, float* r, int64_t n, hipStream_t s)
 {
-  hipLaunchKernelGGL(k_cheb_init<float>, dim3(blocks_for(n)), dim3(kThreads), 0, s, b, dinv, 1.0 / theta, x, d, r,
-                     x_add, copy_r, n);
+  hipLaunchKernelGGL(k_cheb_init<float>, dim3(blocks_for(n)), dim3(kThreads), 0, s, b, dinv, 1.0 / theta, x, d, r, n);
   return hipGetLastError();
 }
 hipError_t cheb_step(float* r, const float* t, float* d, const float* dinv, double c1, double c2, float* x, int64_t n,
@@ -891,14 +985,14 @@ hipError_t cheb_step(float* r, const float* t, float* d, const float* dinv, doub
   hipLaunchKernelGGL(k_cheb_step<float>, dim3(blocks_for(n)), dim3(kThreads), 0, s, r, t, d, dinv, c1, c2, x, n);
   return hipGetLastError();
 }
-hipError_t residual(const float* b, const float* t, float* r, int64_t n, hipStream_t s)
+hipError_t cheb_restart(const float* b, const float* t, const float* dinv, double theta, float* x, float* d, float* r, int64_t n, hipStream_t s)
 {
-  hipLaunchKernelGGL(k_residual<float>, dim3(blocks_for(n)), dim3(kThreads), 0, s, b, t, r, n);
+  hipLaunchKernelGGL(k_cheb_restart<float>, dim3(blocks_for(n)), dim3(kThreads), 0, s, b, t, dinv, 1.0 / theta, x, d, r, n);
   return hipGetLastError();
 }
-hipError_t sub_inplace(float* r, const float* t, int64_t n, hipStream_t s)
+hipError_t cheb_residual(float* r, const float* t, const float* dinv, int64_t n, hipStream_t s)
 {
-  hipLaunchKernelGGL(k_sub_inplace<float>, dim3(blocks_for(n)), dim3(kThreads), 0, s, r, t, n);
+  hipLaunchKernelGGL(k_cheb_residual<float>, dim3(blocks_for(n)), dim3(kThreads), 0, s, r, t, dinv, n);
   return hipGetLastError();
 }
 hipError_t apply_mask(float* x, const uint8_t* mask, int64_t n, hipStream_t s)

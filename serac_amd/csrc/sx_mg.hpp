@@ -23,20 +23,38 @@ struct Grid3 {
   int n[3];  // vertices per direction
 };
 
+// the start of a level's smoothing from zero, made where its right side b is
+// (x null: none): d = dinv b / theta, x = d, r = b
+struct ChebStart {
+  const double* dinv      = nullptr;
+  double        inv_theta = 0.0;
+  double *      x = nullptr, *d = nullptr, *r = nullptr;
+};
+
 // level 0 <-> 1: rc = P^T r on the vertex grid (zero where mask is set), in
 // three passes, one direction each, through scratch t1 and t2 of
 // fe_restrict_scratch(G, 0) and (G, 1) doubles; z += P ec on the nodal grid
 // (P: the order-p interpolation of the vertex field)
 int64_t    fe_restrict_scratch(const sxu::FEGrid& G, int pass);
 hipError_t fe_restrict(const sxu::FEGrid& G, const double* r, double* rc, const uint8_t* mask, double* t1, double* t2,
-                       hipStream_t s);
+                       const ChebStart& start, hipStream_t s);
 hipError_t fe_prolong_add(const sxu::FEGrid& G, const double* ec, double* z, hipStream_t s);
 // vertex level l <-> l + 1 (trilinear): rc = P^T rf (zero where maskc is set);
 // zf += P ec (skipping entries where maskf is set)
-hipError_t grid_restrict(const double* rf, Grid3 f, double* rc, Grid3 c, const uint8_t* maskc, hipStream_t s);
+hipError_t grid_restrict(const double* rf, Grid3 f, double* rc, Grid3 c, const uint8_t* maskc, const ChebStart& start,
+                         hipStream_t s);
 hipError_t grid_prolong_add(const double* ec, Grid3 c, double* zf, Grid3 f, const uint8_t* maskf, hipStream_t s);
 // y = S x
 hipError_t stencil_apply(const double* S, Grid3 g, const double* x, double* y, hipStream_t s);
+// the smoother's passes over a vertex level, each with one product S x in it:
+//   stencil_cheb_step:    r -= S d; d_new = c1 d + c2 dinv r; x += d_new (both: += d + d_new)
+//   stencil_residual:     r -= S d
+//   stencil_cheb_restart: r = b - S x; d = dinv r / theta (x += d is left to the next step)
+hipError_t stencil_cheb_step(const double* S, Grid3 g, const double* d, double* d_new, double* r, const double* dinv,
+                             double c1, double c2, double* x, bool both, hipStream_t s);
+hipError_t stencil_residual(const double* S, Grid3 g, const double* d, double* r, hipStream_t s);
+hipError_t stencil_cheb_restart(const double* S, Grid3 g, const double* x, const double* b, double* r, double* d,
+                                const double* dinv, double theta, hipStream_t s);
 // probing: e = 1 on component ci of the vertices whose index is c (mod 3) in
 // every direction (and not masked), else 0;  extract writes y (= P^T A P e on
 // the coarse grid) into the stencil entries that colour determines
@@ -54,16 +72,19 @@ hipError_t rows_mask(const int32_t* rows, int64_t nr, uint8_t* mask, hipStream_t
 // vmask of the coarse level: the constraint of the coinciding fine vertex
 hipError_t coarsen_mask(const uint8_t* mf, Grid3 f, uint8_t* mc, Grid3 c, hipStream_t s);
 
-// Chebyshev smoothing (x0 = 0 or not):
-//   cheb_init:  d = dinv b / theta; x = d (x_add = 0) or x += d; r = b (copy_r)
-//   cheb_step:  r -= t; d = c1 d + c2 dinv r; x += d
-//   residual:   r = b - t;  sub_inplace: r -= t
-hipError_t cheb_init(const double* b, const double* dinv, double theta, double* x, double* d, double* r, int x_add,
-                     int copy_r, int64_t n, hipStream_t s);
+// Chebyshev smoothing on level 0 (t is the operator's product; rows with
+// dinv = 0, the essential ones, keep r = 0 whatever t holds there):
+//   cheb_init:     from x = 0: d = dinv b / theta; x = d; r = b
+//   cheb_restart:  from x, t = A x: r = b - t; d = dinv r / theta; x += d
+//   cheb_step:     t = A d: r -= t; d = c1 d + c2 dinv r; x += d
+//   cheb_residual: t = A d: r -= t
+hipError_t cheb_init(const double* b, const double* dinv, double theta, double* x, double* d, double* r, int64_t n,
+                     hipStream_t s);
+hipError_t cheb_restart(const double* b, const double* t, const double* dinv, double theta, double* x, double* d,
+                        double* r, int64_t n, hipStream_t s);
 hipError_t cheb_step(double* r, const double* t, double* d, const double* dinv, double c1, double c2, double* x,
                      int64_t n, hipStream_t s);
-hipError_t residual(const double* b, const double* t, double* r, int64_t n, hipStream_t s);
-hipError_t sub_inplace(double* r, const double* t, int64_t n, hipStream_t s);
+hipError_t cheb_residual(double* r, const double* t, const double* dinv, int64_t n, hipStream_t s);
 // zeroes the masked entries of x
 hipError_t apply_mask(double* x, const uint8_t* mask, int64_t n, hipStream_t s);
 // x = A b for a dense row-major n x n A
@@ -99,20 +120,21 @@ hipError_t vertex_compatible(const sxu::FEGrid& G, const int32_t* rows, int64_t 
 // storage and arithmetic; transfers accumulate in FP64); to_f32 zeroes the
 // masked entries
 hipError_t fe_restrict(const sxu::FEGrid& G, const float* r, double* rc, const uint8_t* mask, double* t1, double* t2,
-                       hipStream_t s);
+                       const ChebStart& start, hipStream_t s);
 hipError_t fe_prolong_add(const sxu::FEGrid& G, const double* ec, float* z, hipStream_t s);
-hipError_t cheb_init(const float* b, const float* dinv, double theta, float* x, float* d, float* r, int x_add,
-                     int copy_r, int64_t n, hipStream_t s);
+hipError_t cheb_init(const float* b, const float* dinv, double theta, float* x, float* d, float* r, int64_t n,
+                     hipStream_t s);
+hipError_t cheb_restart(const float* b, const float* t, const float* dinv, double theta, float* x, float* d, float* r,
+                        int64_t n, hipStream_t s);
 hipError_t cheb_step(float* r, const float* t, float* d, const float* dinv, double c1, double c2, float* x, int64_t n,
                      hipStream_t s);
-hipError_t residual(const float* b, const float* t, float* r, int64_t n, hipStream_t s);
-hipError_t sub_inplace(float* r, const float* t, int64_t n, hipStream_t s);
+hipError_t cheb_residual(float* r, const float* t, const float* dinv, int64_t n, hipStream_t s);
 hipError_t apply_mask(float* x, const uint8_t* mask, int64_t n, hipStream_t s);
 hipError_t to_f32(const double* x, float* y, const uint8_t* mask, int64_t n, hipStream_t s);
 hipError_t to_f64(const float* x, double* y, int64_t n, hipStream_t s);
-// power iteration helpers: v = dinv t / |dinv t| (norms on the host)
+// power iteration helpers: v = dinv t; v /= sqrt(*norm2) (device)
 hipError_t mul_dinv(const double* dinv, const double* t, double* v, int64_t n, hipStream_t s);
-hipError_t scale(double* v, double a, int64_t n, hipStream_t s);
+hipError_t normalize(double* v, const double* norm2, int64_t n, hipStream_t s);
 hipError_t seed_field(double* v, int64_t n, uint64_t seed, const uint8_t* mask, hipStream_t s);
 
 }  // namespace sxm
