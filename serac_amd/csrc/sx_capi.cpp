@@ -887,7 +887,8 @@ void apply_gradient(sx_grad* g, const void* dx, void* df, hipEvent_t* ev = nullp
   bool      set   = !out_zeroed;
   for (auto& I : f->integrals)
     if (depends(*I, g->wrt) && I->has_tangent) {
-      n += run_integral(f, *I, sxk::MODE_JVP, dx, df, set, ev ? ev + 2 * n : nullptr, kprec,
+      // (a node sum that comes first need not read the zeros it would add to)
+      n += run_integral(f, *I, sxk::MODE_JVP, dx, df, set || (n == 0 && I->node_sum), ev ? ev + 2 * n : nullptr, kprec,
                         lo && I->d_tangent_lo.ptr != nullptr, stop);
       set = false;
     }
@@ -2782,7 +2783,7 @@ void mg_pcg(sx_grad* g, sx_multigrid* M, const int32_t* ess, int64_t ness, const
     // a V-cycle costs several J.v, so the host runs at most 4 iterations ahead
     const int chunk = std::min(std::max(it / 8, 1), std::min(4, max_iter - it + 1));
     for (int j = 0; j < chunk; j++, it++) {
-      SX_HIP(sxm::pcg_step_xr(x, r, Ad, d, scal, part, sxk::reduction_blocks(), n, stop, s));
+      SX_HIP(sxm::pcg_step_xr(x, r, Ad, d, scal, part, sxk::reduction_blocks(n), n, stop, s));
       mg_apply(M, g, ess, ness, r, z);
       SX_HIP(sxk::dot_partial(r, z, n, part_rz, s));
       SX_HIP(sxk::cg_step_d(d, z, scal, part_rz, n, goal, it, stop, s));

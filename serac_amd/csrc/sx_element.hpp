@@ -839,9 +839,11 @@ __global__ void __launch_bounds__((jvp_group_lanes<N, T>())) k_jvp(const ElemLau
   __shared__ T   stab[TAB];
   __shared__ int snode[EB * NQ];
 
-  // a Krylov loop that already converged: the whole grid leaves (the flag
-  // was written by an earlier kernel on the stream, so every block reads the same)
-  if (P.stop != nullptr && *P.stop != 0.0) return;
+  // a Krylov loop that already converged: the whole grid leaves (the flag was
+  // written by an earlier kernel on the stream, so every block reads the same),
+  // once the loads below are on their way, so that a running one does not wait
+  // for the flag first
+  const double halt = P.stop != nullptr ? *P.stop : 0.0;
 
   const int     tid    = threadIdx.x;
   const int     el     = tid / NQ;
@@ -873,6 +875,7 @@ __global__ void __launch_bounds__((jvp_group_lanes<N, T>())) k_jvp(const ElemLau
   }
   TangentRegs<T, S, DS, NQ> Dr;
   if (active) Dr.load(static_cast<const char*>(P.D) + size_t(slot) * Lay::stride * sizeof(S), li);
+  if (halt != 0.0) return;
   if (active) {
 #pragma unroll
     for (int c = 0; c < NC; c++) S_[c * NQ + li] = ug[c];

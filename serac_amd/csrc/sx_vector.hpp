@@ -9,7 +9,9 @@ namespace sxk {
 hipError_t vec_fill(double* x, double v, int64_t n, hipStream_t s);
 hipError_t vec_fill_f32(float* x, float v, int64_t n, hipStream_t s);
 hipError_t vec_axpy(double a, const double* x, double* y, int64_t n, hipStream_t s);
-// number of partial sums the reductions use (size of the `part` scratch)
+// number of partial sums the reductions of n entries use, and the most of
+// them (size of the `part` scratch)
+int reduction_blocks(int64_t n);
 int reduction_blocks();
 // scal[slot] = (a, b); op 1 then sets scal[2] = scal[0]/scal[1]
 hipError_t vec_dot_dev(const double* a, const double* b, int64_t n, double* part, double* scal, int slot, int op,
