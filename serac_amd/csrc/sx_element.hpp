@@ -11,10 +11,10 @@
 //
 // Thread mapping: the workgroup has 256 lanes (4 wave64s) and holds EB =
 // floor(256 / Q^3) elements; lane li of element el owns the index triple
-// (i2, i1, i0) = li in every stage (node (z,y,x), partial sums, or quadrature
-// point (qz,qy,qx)), which is possible because every form here uses
-// Q = p + 1 = nodes per direction (fn/functional.hpp:193).  LDS per element is
-// (6 + has_source) * nc * Q^3 values, reused across stages.
+// (i2, i1, i0) = li as a node (z,y,x) or a quadrature point (qz,qy,qx), which is
+// possible because every form here uses Q = p + 1 = nodes per direction
+// (fn/functional.hpp:193).  In the contractions of the residual, the
+// linearization and the diagonal a lane owns rows instead (see Rows).
 //
 // The scatter-add is an FP64/FP32 atomic add, or a plain store of the element's
 // values for a node sum that follows (SCATTER_ELEMENT, reproducible), both in
@@ -481,32 +481,106 @@ __device__ __forceinline__ void store_tangent_entry(void* base, int q, int k, do
 }
 
 // ---------------------------------------------------------------------------
+// contractions by rows
+// ---------------------------------------------------------------------------
+// One direction of a sum factorization on an element's [component][z][y][x]
+// array in LDS: a lane owns whole rows along that direction, so it reads N
+// values, forms all N results (for each table that applies) and writes them
+// back in their place.  The table entries are then the same for every lane and
+// compile-time offsets from a kernel argument: scalar loads and scalar
+// operands, no LDS reads.  With a lane per result instead, each result cost N
+// value reads and N table reads through the one LDS port of a CU.  Neo-Hookean
+// residual p = 2 on 57x48x43: 148 -> 120 us of kernel time; p = 3 on 64^3: 735
+// -> 682, two thirds of which FP64 instructions take (about 680 a point).
+template <int N, int NC>
+struct Rows {
+  static constexpr int NQ = N * N * N, COUNT = NC * N * N, ITER = (COUNT + NQ - 1) / NQ;
+  static constexpr int STRIDE[3] = {1, N, N * N};
+  // first entry of row r along `dir`, stride STRIDE[dir]
+  __device__ __forceinline__ static int base(int dir, int r)
+  {
+    const int c = r / (N * N), k = r % (N * N);
+    return c * NQ + (dir == 0 ? k * N : dir == 1 ? (k / N) * N * N + k % N : k);
+  }
+};
+typedef const __attribute__((address_space(4))) double* ScalarTable;  // read by scalar loads
+
+// f(first entry) for every row along DIR that lane li of an active element owns
+template <int N, int NC, int DIR, class F>
+__device__ __forceinline__ void for_rows(int li, bool active, F&& f)
+{
+  using R = Rows<N, NC>;
+#pragma unroll
+  for (int it = 0; it < R::ITER; it++) {
+    const int r = li + it * R::NQ;
+    if (active && r < R::COUNT) f(R::base(DIR, r));
+  }
+}
+template <int N, int STRIDE>
+__device__ __forceinline__ void read_row(const double* a, double* v)
+{
+#pragma unroll
+  for (int i = 0; i < N; i++) v[i] = a[i * STRIDE];
+}
+// out[q] (+)= sum_i T[q][i] v[i]
+template <int N>
+__device__ __forceinline__ void row_forward(ScalarTable T, const double* v, double* out, bool add = false)
+{
+#pragma unroll
+  for (int q = 0; q < N; q++) {
+    double s = add ? out[q] : 0.0;
+#pragma unroll
+    for (int i = 0; i < N; i++) s += T[q * N + i] * v[i];
+    out[q] = s;
+  }
+}
+// out[i] (+)= sum_q T[q][i] v[q]
+template <int N>
+__device__ __forceinline__ void row_transposed(ScalarTable T, const double* v, double* out, bool add = false)
+{
+#pragma unroll
+  for (int i = 0; i < N; i++) {
+    double s = add ? out[i] : 0.0;
+#pragma unroll
+    for (int q = 0; q < N; q++) s += T[q * N + i] * v[q];
+    out[i] = s;
+  }
+}
+template <int N, int STRIDE>
+__device__ __forceinline__ void write_row(double* a, const double* v)
+{
+#pragma unroll
+  for (int i = 0; i < N; i++) a[i * STRIDE] = v[i];
+}
+
+// ---------------------------------------------------------------------------
 // residual (MODE_RESIDUAL) and linearization (MODE_LINEARIZE, tangent in S)
 // ---------------------------------------------------------------------------
 // Waves per SIMD the register allocation aims at: the J2 linearization would
 // take 278 registers (one wave); held to two waves it spills nothing.
-template <int MODE, class QF>
+template <int NC, int MODE, class QF>
 constexpr int element_waves()
 {
-  return MODE == MODE_LINEARIZE && QF::STATE > 0 ? 2 : 1;
+  if (QF::STATE > 0) return MODE == MODE_LINEARIZE ? 2 : 3;
+  return NC == 1 || MODE != MODE_RESIDUAL ? 4 : 5;
 }
 
 template <int N, int NC, int MODE, class QF, int LAYOUT, typename S>
-__global__ void __launch_bounds__(256, (element_waves<MODE, QF>())) k_element(const ElemLaunch P)
+__global__ void __launch_bounds__(256, (element_waves<NC, MODE, QF>())) k_element(const ElemLaunch P)
 {
   constexpr int  NQ      = N * N * N;
+  constexpr int  NN      = N * N;
   constexpr int  EB      = 256 / NQ;
   using Shape            = TanShape<LAYOUT, NC>;
   constexpr bool HAS_SRC = QF::HAS_SOURCE;
   constexpr int  DS      = Shape::DS;
   constexpr int  NST     = QF::STATE;
   constexpr int  R       = NC * NQ;  // one LDS region
-  constexpr int  PER     = (6 + (HAS_SRC ? 1 : 0)) * R;
-  constexpr int  TAB     = 4 * N * N + N;
+  constexpr int  PER     = (3 + (HAS_SRC || QF::USES_VALUE ? 1 : 0)) * R;
   using Lay              = TangentLayout<S, DS, NQ>;
 
   __shared__ double smem[EB * PER];
-  __shared__ double stab[TAB];
+  __shared__ double sxw[2 * N];  // Gauss points and weights
   __shared__ double sxv[EB * 24];
   __shared__ int    snode[EB * NQ];
 
@@ -515,19 +589,16 @@ __global__ void __launch_bounds__(256, (element_waves<MODE, QF>())) k_element(co
   const int     li     = tid - el * NQ;
   const int     i0     = li % N;
   const int     i1     = (li / N) % N;
-  const int     i2     = li / (N * N);
+  const int     i2     = li / NN;
   const int64_t slot   = P.slot_begin + logical_block(P.xcd_remap) * EB + el;
   const bool    active = (el < EB) && (slot < P.slot_end);
-  double*       S_     = smem + (el < EB ? el : 0) * PER;
-  const double* u      = static_cast<const double*>(P.u);
-  double*       r      = static_cast<double*>(P.r);
+  double*       S0     = smem + (el < EB ? el : 0) * PER;
+  double *      S1 = S0 + R, *S2 = S0 + 2 * R, *S3 = S0 + 3 * R;  // S3 only where PER has it
+  double*       r = static_cast<double*>(P.r);
 
-  for (int k = tid; k < TAB; k += blockDim.x) stab[k] = P.tables[k];
-  const double* tB  = stab;
-  const double* tG  = stab + N * N;
-  const double* tBw = stab + 2 * N * N;
-  const double* tGw = stab + 3 * N * N;
-  const double* txq = stab + 4 * N * N;
+  if (tid < 2 * N) sxw[tid] = P.tables[4 * NN + tid];
+  const ScalarTable tB = (ScalarTable)(uintptr_t)P.tables;
+  const ScalarTable tG = tB + NN;
 
   // ---- quadrature-point state (issued first, consumed at the qfunction)
   double  st[NST > 0 ? NST : 1];
@@ -539,268 +610,191 @@ __global__ void __launch_bounds__(256, (element_waves<MODE, QF>())) k_element(co
       for (int k = 0; k < NST; k++) st[k] = stp[k * NQ];
     }
   }
+  int64_t node = 0;
+  if (active) {
+    node = P.map[size_t(slot) * NQ + li];
+    for (int k = li; k < 24; k += NQ) sxv[el * 24 + k] = P.coords[size_t(slot) * 24 + k];
+  }
 
+  // Parent gradient (and value) at this lane's point of a field on the
+  // element's nodes: gather, then x, y and z in turn.  Every lane calls it; the
+  // regions are free again after it.
+  auto interpolate = [&](const double* field, double* val, double* gp) {
+    if (active) {
+#pragma unroll
+      for (int c = 0; c < NC; c++) S0[c * NQ + li] = field[lidx(node, c, NC, P.nnodes, P.ordering)];
+    }
+    lds_barrier();
+    for_rows<N, NC, 0>(li, active, [&](int o) {  // u -> B u, G u
+      double v[N], a[N], b[N];
+      read_row<N, 1>(S0 + o, v);
+      row_forward<N>(tB, v, a);
+      row_forward<N>(tG, v, b);
+      write_row<N, 1>(S0 + o, a);
+      write_row<N, 1>(S1 + o, b);
+    });
+    lds_barrier();
+    for_rows<N, NC, 1>(li, active, [&](int o) {  // -> BB, BG (y, x), GB
+      double v[N], w[N], a[N];
+      read_row<N, N>(S0 + o, v);
+      read_row<N, N>(S1 + o, w);
+      row_forward<N>(tB, v, a);
+      write_row<N, N>(S0 + o, a);
+      row_forward<N>(tB, w, a);
+      write_row<N, N>(S1 + o, a);
+      row_forward<N>(tG, v, a);
+      write_row<N, N>(S2 + o, a);
+    });
+    lds_barrier();
+    for_rows<N, NC, 2>(li, active, [&](int o) {  // -> d/dx in S1, d/dy in S2, d/dz in S0, value in S3
+      double v[N], a[N];
+      read_row<N, NN>(S1 + o, v);
+      row_forward<N>(tB, v, a);
+      write_row<N, NN>(S1 + o, a);
+      read_row<N, NN>(S2 + o, v);
+      row_forward<N>(tB, v, a);
+      write_row<N, NN>(S2 + o, a);
+      read_row<N, NN>(S0 + o, v);
+      row_forward<N>(tG, v, a);
+      write_row<N, NN>(S0 + o, a);
+      if constexpr (QF::USES_VALUE) {
+        row_forward<N>(tB, v, a);
+        write_row<N, NN>(S3 + o, a);
+      }
+    });
+    lds_barrier();
+    if (active) {
+#pragma unroll
+      for (int c = 0; c < NC; c++) {
+        gp[c * 3 + 0] = S1[c * NQ + li];
+        gp[c * 3 + 1] = S2[c * NQ + li];
+        gp[c * 3 + 2] = S0[c * NQ + li];
+        if constexpr (QF::USES_VALUE) val[c] = S3[c * NQ + li];
+      }
+    }
+    lds_barrier();
+  };
+
+  double val[NC], gp[3 * NC];
+#pragma unroll
+  for (int c = 0; c < NC; c++) val[c] = 0.0;
+  interpolate(static_cast<const double*>(P.u), val, gp);
   // ---- shape displacement (ShapeAwareFunctional, fn/shape_aware_functional.hpp:37-50):
   // the parent gradient of p at this lane's quadrature point, added to the
   // geometric Jacobian below, so dx/dxi = dX/dxi + dp/dxi = (I + dp/dX) dX/dxi.
   // P.shape is the same for every lane, so the barriers inside are uniform.
-  // parent gradient (at this lane's point) of a 3-component field on the
-  // element's nodes, by the interpolation's sum factorization; uses LDS
-  // regions 0..5 before the gather
-  auto parent_grad3 = [&](const double* field, double* out9) {
-    if (active) {
-      const int64_t nd = P.map[size_t(slot) * NQ + li];
-#pragma unroll
-      for (int c = 0; c < 3; c++) S_[c * NQ + li] = field[lidx(nd, c, 3, P.nnodes, P.ordering)];
-    }
-    lds_barrier();
-    if (active) {
-#pragma unroll
-      for (int c = 0; c < 3; c++) {
-        const double* pp = S_ + c * NQ + (i2 * N + i1) * N;
-        double        s0 = 0.0, s1 = 0.0;
-#pragma unroll
-        for (int x = 0; x < N; x++) {
-          s0 += tB[i0 * N + x] * pp[x];
-          s1 += tG[i0 * N + x] * pp[x];
-        }
-        S_[1 * R + c * NQ + li] = s0;
-        S_[2 * R + c * NQ + li] = s1;
-      }
-    }
-    lds_barrier();
-    if (active) {
-#pragma unroll
-      for (int c = 0; c < 3; c++) {
-        const double* a10 = S_ + 1 * R + c * NQ;
-        const double* a11 = S_ + 2 * R + c * NQ;
-        double        s0 = 0.0, s1 = 0.0, s2 = 0.0;
-#pragma unroll
-        for (int y = 0; y < N; y++) {
-          const int    idx = (i2 * N + y) * N + i0;
-          const double b = tB[i1 * N + y], g = tG[i1 * N + y];
-          s0 += b * a10[idx];
-          s1 += b * a11[idx];
-          s2 += g * a10[idx];
-        }
-        S_[3 * R + c * NQ + li] = s0;
-        S_[4 * R + c * NQ + li] = s1;
-        S_[5 * R + c * NQ + li] = s2;
-      }
-    }
-    lds_barrier();
-    if (active) {
-#pragma unroll
-      for (int c = 0; c < 3; c++) {
-        const double* a20 = S_ + 3 * R + c * NQ;
-        const double* a21 = S_ + 4 * R + c * NQ;
-        const double* a22 = S_ + 5 * R + c * NQ;
-#pragma unroll
-        for (int z = 0; z < N; z++) {
-          const int    idx = (z * N + i1) * N + i0;
-          const double b = tB[i2 * N + z], g = tG[i2 * N + z];
-          out9[c * 3 + 0] += b * a21[idx];
-          out9[c * 3 + 1] += b * a22[idx];
-          out9[c * 3 + 2] += g * a20[idx];
-        }
-      }
-    }
-    lds_barrier();  // the next pass / the gather overwrites the regions read above
-  };
   double gps[9], dgps[9];
 #pragma unroll
   for (int k = 0; k < 9; k++) gps[k] = dgps[k] = 0.0;
   if constexpr (NC == 3) {
-    if (P.shape != nullptr) parent_grad3(P.shape, gps);
-    if constexpr (MODE == MODE_SHAPE_JVP) parent_grad3(P.dshape, dgps);
+    double unused[NC];
+    if (P.shape != nullptr) interpolate(P.shape, unused, gps);
+    if constexpr (MODE == MODE_SHAPE_JVP) interpolate(P.dshape, unused, dgps);
   }
 
-  // ---- gather
-  int64_t node = 0;
+  // ---- quadrature point
   if (active) {
-    node = P.map[size_t(slot) * NQ + li];
-#pragma unroll
-    for (int c = 0; c < NC; c++) S_[c * NQ + li] = u[lidx(node, c, NC, P.nnodes, P.ordering)];
-    for (int k = li; k < 24; k += NQ) sxv[el * 24 + k] = P.coords[size_t(slot) * 24 + k];
-  }
-  lds_barrier();
-
-  // ---- interpolate, stage x: (z, y, qx)
-  if (active) {
-#pragma unroll
-    for (int c = 0; c < NC; c++) {
-      const double* uu = S_ + c * NQ + (i2 * N + i1) * N;
-      double        s0 = 0.0, s1 = 0.0;
-#pragma unroll
-      for (int x = 0; x < N; x++) {
-        s0 += tB[i0 * N + x] * uu[x];
-        s1 += tG[i0 * N + x] * uu[x];
-      }
-      S_[1 * R + c * NQ + li] = s0;
-      S_[2 * R + c * NQ + li] = s1;
-    }
-  }
-  lds_barrier();
-
-  // ---- stage y: (z, qy, qx)
-  if (active) {
-#pragma unroll
-    for (int c = 0; c < NC; c++) {
-      const double* a10 = S_ + 1 * R + c * NQ;
-      const double* a11 = S_ + 2 * R + c * NQ;
-      double        s0 = 0.0, s1 = 0.0, s2 = 0.0;
-#pragma unroll
-      for (int y = 0; y < N; y++) {
-        const int    idx = (i2 * N + y) * N + i0;
-        const double b = tB[i1 * N + y], g = tG[i1 * N + y];
-        s0 += b * a10[idx];
-        s1 += b * a11[idx];
-        s2 += g * a10[idx];
-      }
-      S_[3 * R + c * NQ + li] = s0;
-      S_[4 * R + c * NQ + li] = s1;
-      S_[5 * R + c * NQ + li] = s2;
-    }
-  }
-  lds_barrier();
-
-  // ---- stage z + quadrature point: (qz, qy, qx)
-  if (active) {
-    double val[NC], gp[3 * NC];
-#pragma unroll
-    for (int c = 0; c < NC; c++) {
-      const double* a20 = S_ + 3 * R + c * NQ;
-      const double* a21 = S_ + 4 * R + c * NQ;
-      const double* a22 = S_ + 5 * R + c * NQ;
-      double        v = 0.0, g0 = 0.0, g1 = 0.0, g2 = 0.0;
-#pragma unroll
-      for (int z = 0; z < N; z++) {
-        const int    idx = (z * N + i1) * N + i0;
-        const double b = tB[i2 * N + z], g = tG[i2 * N + z];
-        if constexpr (QF::USES_VALUE) v += b * a20[idx];
-        g0 += b * a21[idx];
-        g1 += b * a22[idx];
-        g2 += g * a20[idx];
-      }
-      val[c]        = v;
-      gp[c * 3 + 0] = g0;
-      gp[c * 3 + 1] = g1;
-      gp[c * 3 + 2] = g2;
-    }
-
     double J[9], Ji[9];
-    trilinear_jacobian(sxv + el * 24, txq[i0], txq[i1], txq[i2], J);
+    trilinear_jacobian(sxv + el * 24, sxw[i0], sxw[i1], sxw[i2], J);
 #pragma unroll
     for (int k = 0; k < 9; k++) J[k] += gps[k];
     inv3(J, Ji);
-    const double dJ = det3(J);
-    double       src[NC], fp[3 * NC];
+    const double dJ = det3(J), wq = sxw[N + i0] * sxw[N + i1] * sxw[N + i2];
+    double       src[NC], fp[3 * NC];  // source and flux, times the quadrature weight
     if constexpr (MODE == MODE_SHAPE_JVP) {
       qpoint_shape_dir<QF, NC>(P.params, J, dgps, val, gp, st, src, fp);
+#pragma unroll
+      for (int c = 0; c < NC; c++) src[c] *= wq;
+#pragma unroll
+      for (int k = 0; k < 3 * NC; k++) fp[k] *= wq;
     } else {
-    if constexpr (MODE == MODE_LINEARIZE) {
-      // the entries come in increasing storage order; the state is the one before this call
-      void*                        Dp = static_cast<char*>(P.D) + size_t(slot) * Lay::stride * sizeof(S);
-      typename StoreTraits<S>::raw pend[Lay::VEC];
-      double                       g[3 * NC];
-      physical_gradient<NC>(gp, Ji, g);
-      QF::tangent(P.params, g, Ji, dJ, st, [&](int rr, int s, double v) {
-        store_tangent_entry<S, DS, NQ>(Dp, li, Shape::idx(rr, s), v, pend);
-      });
+      if constexpr (MODE == MODE_LINEARIZE) {
+        // the entries come in increasing storage order; the state is the one before this call
+        void*                        Dp = static_cast<char*>(P.D) + size_t(slot) * Lay::stride * sizeof(S);
+        typename StoreTraits<S>::raw pend[Lay::VEC];
+        double                       g[3 * NC];
+        physical_gradient<NC>(gp, Ji, g);
+        QF::tangent(P.params, g, Ji, dJ, st, [&](int rr, int s, double v) {
+          store_tangent_entry<S, DS, NQ>(Dp, li, Shape::idx(rr, s), v, pend);
+        });
+        if constexpr (NST > 0) {
+          // eval() below starts over from its inputs: sharing the trial state with the tangent kept it in registers
+          // across all 81 entries
+#pragma unroll
+          for (int k = 0; k < 3 * NC; k++) opaque(gp[k]);
+        }
+      }
+      qpoint_eval<QF, NC>(P.params, Ji, dJ * wq, val, gp, src, fp, st);
       if constexpr (NST > 0) {
-        // eval() below starts over from its inputs: sharing the trial state with the tangent kept it in registers
-        // across all 81 entries
+        // batch_apply_qf (fn/domain_integral_kernels.hpp:125-150): commit the
+        // point's updated state only when asked to
+        if (P.update_state) {
 #pragma unroll
-        for (int k = 0; k < 3 * NC; k++) opaque(gp[k]);
+          for (int k = 0; k < NST; k++) stp[k * NQ] = st[k];
+        }
       }
     }
-    qpoint_eval<QF, NC>(P.params, Ji, dJ, val, gp, src, fp, st);
-    if constexpr (NST > 0) {
-      // batch_apply_qf (fn/domain_integral_kernels.hpp:125-150): commit the
-      // point's updated state only when asked to
-      if (P.update_state) {
-#pragma unroll
-        for (int k = 0; k < NST; k++) stp[k * NQ] = st[k];
-      }
-    }
-    }
-    // flux -> regions 0..2 (u and stage-x partials are dead), source -> region 6
 #pragma unroll
     for (int c = 0; c < NC; c++) {
-#pragma unroll
-      for (int d = 0; d < 3; d++) S_[(c * 3 + d) * NQ + li] = fp[c * 3 + d];
-      if constexpr (HAS_SRC) S_[6 * R + c * NQ + li] = src[c];
+      S0[c * NQ + li] = fp[c * 3 + 0];
+      S1[c * NQ + li] = fp[c * 3 + 1];
+      S2[c * NQ + li] = fp[c * 3 + 2];
+      if constexpr (HAS_SRC) S3[c * NQ + li] = src[c];
     }
   }
   lds_barrier();
 
-  // ---- integrate, stage qx: (qz, qy, x)
-  if (active) {
-#pragma unroll
-    for (int c = 0; c < NC; c++) {
-      const double* f0 = S_ + (c * 3 + 0) * NQ;
-      const double* f1 = S_ + (c * 3 + 1) * NQ;
-      const double* f2 = S_ + (c * 3 + 2) * NQ;
-      const double* sr = S_ + 6 * R + c * NQ;
-      double        s0 = 0.0, s1 = 0.0, s2 = 0.0;
-#pragma unroll
-      for (int qx = 0; qx < N; qx++) {
-        const int    q  = (i2 * N + i1) * N + qx;
-        const double bw = tBw[qx * N + i0], gw = tGw[qx * N + i0];
-        if constexpr (HAS_SRC) s0 += sr[q] * bw;
-        s0 += f0[q] * gw;
-        s1 += f1[q] * bw;
-        s2 += f2[q] * bw;
-      }
-      S_[3 * R + c * NQ + li] = s0;
-      S_[4 * R + c * NQ + li] = s1;
-      S_[5 * R + c * NQ + li] = s2;
+  // ---- integrate: x, y, z (the weights are in the flux)
+  for_rows<N, NC, 0>(li, active, [&](int o) {
+    double v[N], a[N];
+    read_row<N, 1>(S0 + o, v);
+    row_transposed<N>(tG, v, a);
+    if constexpr (HAS_SRC) {
+      read_row<N, 1>(S3 + o, v);
+      row_transposed<N>(tB, v, a, true);
     }
-  }
+    write_row<N, 1>(S0 + o, a);
+    read_row<N, 1>(S1 + o, v);
+    row_transposed<N>(tB, v, a);
+    write_row<N, 1>(S1 + o, a);
+    read_row<N, 1>(S2 + o, v);
+    row_transposed<N>(tB, v, a);
+    write_row<N, 1>(S2 + o, a);
+  });
+  lds_barrier();
+  for_rows<N, NC, 1>(li, active, [&](int o) {
+    double v[N], a[N];
+    read_row<N, N>(S0 + o, v);
+    row_transposed<N>(tB, v, a);
+    read_row<N, N>(S1 + o, v);
+    row_transposed<N>(tG, v, a, true);
+    write_row<N, N>(S0 + o, a);
+    read_row<N, N>(S2 + o, v);
+    row_transposed<N>(tB, v, a);
+    write_row<N, N>(S1 + o, a);
+  });
+  lds_barrier();
+  for_rows<N, NC, 2>(li, active, [&](int o) {
+    double v[N], a[N];
+    read_row<N, NN>(S0 + o, v);
+    row_transposed<N>(tB, v, a);
+    read_row<N, NN>(S1 + o, v);
+    row_transposed<N>(tG, v, a, true);
+    write_row<N, NN>(S2 + o, a);
+  });
   lds_barrier();
 
-  // ---- stage qy: (qz, y, x)
-  if (active) {
-#pragma unroll
-    for (int c = 0; c < NC; c++) {
-      const double* a20 = S_ + 3 * R + c * NQ;
-      const double* a21 = S_ + 4 * R + c * NQ;
-      const double* a22 = S_ + 5 * R + c * NQ;
-      double        s0 = 0.0, s1 = 0.0;
-#pragma unroll
-      for (int qy = 0; qy < N; qy++) {
-        const int    idx = (i2 * N + qy) * N + i0;
-        const double bw = tBw[qy * N + i1], gw = tGw[qy * N + i1];
-        s0 += a20[idx] * bw + a21[idx] * gw;
-        s1 += a22[idx] * bw;
-      }
-      S_[0 * R + c * NQ + li] = s0;
-      S_[1 * R + c * NQ + li] = s1;
-    }
-  }
-  lds_barrier();
-
-  // ---- stage qz + scatter-add: (z, y, x)
+  // ---- scatter-add: lane = node
   double acc[NC];
   if (active) {
 #pragma unroll
-    for (int c = 0; c < NC; c++) {
-      const double* a10 = S_ + 0 * R + c * NQ;
-      const double* a11 = S_ + 1 * R + c * NQ;
-      acc[c]            = 0.0;
-#pragma unroll
-      for (int qz = 0; qz < N; qz++) {
-        const int idx = (qz * N + i1) * N + i0;
-        acc[c] += a10[idx] * tBw[qz * N + i2] + a11[idx] * tGw[qz * N + i2];
-      }
-    }
+    for (int c = 0; c < NC; c++) acc[c] = S2[c * NQ + li];
   }
   if (P.scatter == SCATTER_ELEMENT) {
-    store_element<N, NC>(P.E, acc, S_ + 2 * R, slot, li, active);
+    store_element<N, NC>(P.E, acc, S0, slot, li, active);
   } else if (P.ordered) {
-    scatter_element<N, NC, double, double>(r, acc, S_ + 2 * R, smem + (el > 0 && el < EB ? el - 1 : 0) * PER + 2 * R,
-                                           snode, el, EB, node, li, active, P.nnodes, P.ordering, P.scatter,
-                                           P.ordered == 2);
+    scatter_element<N, NC, double, double>(r, acc, S0, smem + (el > 0 && el < EB ? el - 1 : 0) * PER, snode, el, EB,
+                                           node, li, active, P.nnodes, P.ordering, P.scatter, P.ordered == 2);
   } else if (active) {
 #pragma unroll
     for (int c = 0; c < NC; c++) scatter_add(r, lidx(node, c, NC, P.nnodes, P.ordering), acc[c], P.scatter);
@@ -1255,7 +1249,7 @@ __global__ void __launch_bounds__(64 * EB) k_jvp_xy(const ElemLaunch P)
 // (a, b) and (b, a) share their tables and are summed first; the value rows of
 // FULL_SYM add the (value, value) term and the (value, grad) pairs.  Per
 // component this leaves NF fields per point, each contracted over qx, qy, qz in
-// turn through LDS (lane = point, then (jx, qy, qz), (jx, jy, qz), node).
+// turn through LDS.
 template <int LAYOUT, int NC>
 struct DiagFields {
   using Shape                = TanShape<LAYOUT, NC>;
@@ -1271,6 +1265,9 @@ struct DiagFields {
   }
 };
 
+// The contractions go by rows, all components at once and every field in its
+// place.  Neo-Hookean p = 3 on 48x40x44, FP64: 305 -> 248 us, of which the
+// tangent's bytes take 176.
 template <int N, int NC, int LAYOUT, typename S>
 __global__ void __launch_bounds__(256) k_diagonal(const ElemLaunch P)
 {
@@ -1281,25 +1278,18 @@ __global__ void __launch_bounds__(256) k_diagonal(const ElemLaunch P)
   constexpr int NF = F::NF;
   constexpr int VO = Shape::VO;
   constexpr int NN = N * N;
+  constexpr int R  = NC * NQ;  // one field, all components
   using Lay        = TangentLayout<S, Shape::DS, NQ>;
-  static_assert(NF >= NC, "the scatter stages NC x NQ values in the element's field slots");
-  __shared__ double stab[3 * NN];  // [w B B | w G B | w G G][q * N + j]
-  __shared__ double sf[EB * NF * NQ];
+  __shared__ double sf[EB * NF * R];
   __shared__ int    snode[EB * NQ];
 
   const int     tid    = threadIdx.x;
   const int     el     = tid / NQ;
   const int     li     = tid - el * NQ;
-  const int     a0     = li % N, a1 = (li / N) % N, a2 = li / NN;
   const int64_t slot   = P.slot_begin + logical_block(P.xcd_remap) * EB + el;
   const bool    active = (el < EB) && (slot < P.slot_end);  // uniform over the element's lanes
-  double*       sv     = sf + (el < EB ? el : 0) * NF * NQ;
-  for (int k = tid; k < NN; k += blockDim.x) {
-    const double b = P.tables[k], g = P.tables[NN + k], bw = P.tables[2 * NN + k], gw = P.tables[3 * NN + k];
-    stab[k]          = bw * b;
-    stab[NN + k]     = gw * b;
-    stab[2 * NN + k] = gw * g;
-  }
+  double*       sv     = sf + (el < EB ? el : 0) * NF * R;
+  const ScalarTable tab = (ScalarTable)(uintptr_t)P.tables + (4 * NN + 2 * N);  // w B B, w G B, w G G
 
   using raw        = typename StoreTraits<S>::raw;
   const raw* Dbase = reinterpret_cast<const raw*>(static_cast<const char*>(P.D) +
@@ -1311,8 +1301,6 @@ __global__ void __launch_bounds__(256) k_diagonal(const ElemLaunch P)
     else
       return double(v);
   };
-  // the point's fields, all components, loaded up front
-  double fv[NC][NF];
   if (active) {
 #pragma unroll
     for (int c = 0; c < NC; c++) {
@@ -1320,77 +1308,63 @@ __global__ void __launch_bounds__(256) k_diagonal(const ElemLaunch P)
 #pragma unroll
       for (int f = 0; f < 6; f++) {
         const int ra = g0 + F::pa(f), rb = g0 + F::pb(f);
-        fv[c][f]     = ra == rb ? Dat(Shape::idx(ra, rb)) : Dat(Shape::idx(ra, rb)) + Dat(Shape::idx(rb, ra));
+        sv[f * R + c * NQ + li] = ra == rb ? Dat(Shape::idx(ra, rb)) : Dat(Shape::idx(ra, rb)) + Dat(Shape::idx(rb, ra));
       }
       if constexpr (F::FULL) {
-        fv[c][6] = Dat(Shape::idx(c, c));
+        sv[6 * R + c * NQ + li] = Dat(Shape::idx(c, c));
 #pragma unroll
-        for (int d = 0; d < 3; d++) fv[c][7 + d] = Dat(Shape::idx(c, g0 + d)) + Dat(Shape::idx(g0 + d, c));
+        for (int d = 0; d < 3; d++)
+          sv[(7 + d) * R + c * NQ + li] = Dat(Shape::idx(c, g0 + d)) + Dat(Shape::idx(g0 + d, c));
       }
     }
   }
-  const double* tx = stab + 0;  // offset by table * NN below
-  double        acc[NC];
-#pragma unroll
-  for (int c = 0; c < NC; c++) {
-    acc[c] = 0.0;
-    __syncthreads();  // the tables (c = 0); the previous component's z reads (c > 0)
-    if (active) {
-#pragma unroll
-      for (int f = 0; f < NF; f++) sv[f * NQ + li] = fv[c][f];
-    }
-    __syncthreads();
-    double t[NF];
-    if (active) {  // x: lane (jx, qy, qz)
-#pragma unroll
-      for (int f = 0; f < NF; f++) {
-        const double* X = tx + F::table(f, 0) * NN;
-        double        r = 0.0;
-#pragma unroll
-        for (int q = 0; q < N; q++) r += X[q * N + a0] * sv[f * NQ + (a2 * N + a1) * N + q];
-        t[f] = r;
-      }
-    }
-    __syncthreads();
-    if (active) {
-#pragma unroll
-      for (int f = 0; f < NF; f++) sv[f * NQ + li] = t[f];
-    }
-    __syncthreads();
-    if (active) {  // y: lane (jx, jy, qz)
-#pragma unroll
-      for (int f = 0; f < NF; f++) {
-        const double* Y = tx + F::table(f, 1) * NN;
-        double        r = 0.0;
-#pragma unroll
-        for (int q = 0; q < N; q++) r += Y[q * N + a1] * sv[f * NQ + (a2 * N + q) * N + a0];
-        t[f] = r;
-      }
-    }
-    __syncthreads();
-    if (active) {
-#pragma unroll
-      for (int f = 0; f < NF; f++) sv[f * NQ + li] = t[f];
-    }
-    __syncthreads();
-    if (active) {  // z: lane = node (jx, jy, jz)
-#pragma unroll
-      for (int f = 0; f < NF; f++) {
-        const double* Z = tx + F::table(f, 2) * NN;
-#pragma unroll
-        for (int q = 0; q < N; q++) acc[c] += Z[q * N + a2] * sv[f * NQ + (q * N + a1) * N + a0];
-      }
-    }
-  }
-  // scatter in address order (as the J.v's), through the element's field slots
   const int64_t node = active ? int64_t(P.map[size_t(slot) * NQ + li]) : 0;
-  double*       out  = static_cast<double*>(P.r);
-  __syncthreads();  // the last z stage has read the slots
+  lds_barrier();
+  for_rows<N, NC, 0>(li, active, [&](int o) {
+#pragma unroll
+    for (int f = 0; f < NF; f++) {
+      double v[N], a[N];
+      read_row<N, 1>(sv + f * R + o, v);
+      row_transposed<N>(tab + F::table(f, 0) * NN, v, a);
+      write_row<N, 1>(sv + f * R + o, a);
+    }
+  });
+  lds_barrier();
+  for_rows<N, NC, 1>(li, active, [&](int o) {
+#pragma unroll
+    for (int f = 0; f < NF; f++) {
+      double v[N], a[N];
+      read_row<N, N>(sv + f * R + o, v);
+      row_transposed<N>(tab + F::table(f, 1) * NN, v, a);
+      write_row<N, N>(sv + f * R + o, a);
+    }
+  });
+  lds_barrier();
+  for_rows<N, NC, 2>(li, active, [&](int o) {
+    double a[N];
+#pragma unroll
+    for (int i = 0; i < N; i++) a[i] = 0.0;
+#pragma unroll
+    for (int f = 0; f < NF; f++) {
+      double v[N];
+      read_row<N, NN>(sv + f * R + o, v);
+      row_transposed<N>(tab + F::table(f, 2) * NN, v, a, true);
+    }
+    write_row<N, NN>(sv + o, a);
+  });
+  lds_barrier();
+  // scatter (in address order as the J.v's) through the second field's place
+  double acc[NC];
+  if (active) {
+#pragma unroll
+    for (int c = 0; c < NC; c++) acc[c] = sv[c * NQ + li];
+  }
+  double* out = static_cast<double*>(P.r);
   if (P.scatter == SCATTER_ELEMENT) {
-    store_element<N, NC>(P.E, acc, sv, slot, li, active);
+    store_element<N, NC>(P.E, acc, sv + R, slot, li, active);
   } else if (P.ordered) {
-    scatter_element<N, NC, double, double>(out, acc, sv, sf + (el > 0 && el < EB ? el - 1 : 0) * NF * NQ, snode, el,
-                                           EB, node, li, active, P.nnodes, P.ordering, P.scatter, P.ordered == 2);
+    scatter_element<N, NC, double, double>(out, acc, sv + R, sf + (el > 0 && el < EB ? el - 1 : 0) * NF * R + R, snode,
+                                           el, EB, node, li, active, P.nnodes, P.ordering, P.scatter, P.ordered == 2);
   } else if (active) {
 #pragma unroll
     for (int c = 0; c < NC; c++) scatter_add(out, lidx(node, c, NC, P.nnodes, P.ordering), acc[c], P.scatter);

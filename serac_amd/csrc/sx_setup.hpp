@@ -76,11 +76,12 @@ inline void lagrange(const std::vector<double>& pts, double x, double* phi, doub
   }
 }
 
-// Device table for N = Q = p+1: B, G, Bw, Gw as [q][n], then GL points [q].
+// Device table for N = Q = p+1: B, G, Bw, Gw as [q][n], then GL points [q] and
+// weights [q], then the diagonal's w B B, w G B, w G G as [q][n].
 inline std::vector<double> element_tables(int N)
 {
   const int           Q = N;
-  std::vector<double> t(size_t(4 * N * N + N));
+  std::vector<double> t(size_t(7 * N * N + 2 * N));
   double              xq[8], wq[8], phi[8], dphi[8];
   gauss_legendre(Q, xq, wq);
   auto pts = lobatto_points(N);
@@ -92,7 +93,14 @@ inline std::vector<double> element_tables(int N)
       t[2 * N * N + q * N + i] = phi[i] * wq[q];
       t[3 * N * N + q * N + i] = dphi[i] * wq[q];
     }
-    t[4 * N * N + q] = xq[q];
+    t[4 * N * N + q]     = xq[q];
+    t[4 * N * N + N + q] = wq[q];
+    double* d            = &t[4 * N * N + 2 * N];
+    for (int i = 0; i < N; i++) {
+      d[0 * N * N + q * N + i] = phi[i] * wq[q] * phi[i];
+      d[1 * N * N + q * N + i] = dphi[i] * wq[q] * phi[i];
+      d[2 * N * N + q * N + i] = dphi[i] * wq[q] * dphi[i];
+    }
   }
   return t;
 }
