@@ -503,7 +503,9 @@ struct Rows {
     return c * NQ + (dir == 0 ? k * N : dir == 1 ? (k / N) * N * N + k % N : k);
   }
 };
-typedef const __attribute__((address_space(4))) double* ScalarTable;  // read by scalar loads
+template <typename T>
+using ScalarPtr = const __attribute__((address_space(4))) T*;  // read by scalar loads
+using ScalarTable = ScalarPtr<double>;
 
 // f(first entry) for every row along DIR that lane li of an active element owns
 template <int N, int NC, int DIR, class F>
@@ -516,38 +518,50 @@ __device__ __forceinline__ void for_rows(int li, bool active, F&& f)
     if (active && r < R::COUNT) f(R::base(DIR, r));
   }
 }
-template <int N, int STRIDE>
-__device__ __forceinline__ void read_row(const double* a, double* v)
+template <int N, int STRIDE, typename T>
+__device__ __forceinline__ void read_row(const T* a, T* v)
 {
 #pragma unroll
   for (int i = 0; i < N; i++) v[i] = a[i * STRIDE];
 }
-// out[q] (+)= sum_i T[q][i] v[i]
-template <int N>
-__device__ __forceinline__ void row_forward(ScalarTable T, const double* v, double* out, bool add = false)
+// out[q] (+)= sum_i tab[q][i] v[i]
+template <int N, typename T>
+__device__ __forceinline__ void row_forward(ScalarPtr<T> tab, const T* v, T* out, bool add = false)
 {
 #pragma unroll
   for (int q = 0; q < N; q++) {
-    double s = add ? out[q] : 0.0;
+    T s = add ? out[q] : T(0);
 #pragma unroll
-    for (int i = 0; i < N; i++) s += T[q * N + i] * v[i];
+    for (int i = 0; i < N; i++) s += tab[q * N + i] * v[i];
     out[q] = s;
   }
 }
-// out[i] (+)= sum_q T[q][i] v[q]
-template <int N>
-__device__ __forceinline__ void row_transposed(ScalarTable T, const double* v, double* out, bool add = false)
+// out[i] (+)= sum_q tab[q][i] v[q]
+template <int N, typename T>
+__device__ __forceinline__ void row_transposed(ScalarPtr<T> tab, const T* v, T* out, bool add = false)
 {
 #pragma unroll
   for (int i = 0; i < N; i++) {
-    double s = add ? out[i] : 0.0;
+    T s = add ? out[i] : T(0);
 #pragma unroll
-    for (int q = 0; q < N; q++) s += T[q * N + i] * v[q];
+    for (int q = 0; q < N; q++) s += tab[q * N + i] * v[q];
     out[i] = s;
   }
 }
-template <int N, int STRIDE>
-__device__ __forceinline__ void write_row(double* a, const double* v)
+// out[i] = sum_q (ta[q][i] v[q] + tb[q][i] w[q]), a pair at a time
+template <int N, typename T>
+__device__ __forceinline__ void row_transposed_pair(ScalarPtr<T> ta, const T* v, ScalarPtr<T> tb, const T* w, T* out)
+{
+#pragma unroll
+  for (int i = 0; i < N; i++) {
+    T s = T(0);
+#pragma unroll
+    for (int q = 0; q < N; q++) s += v[q] * ta[q * N + i] + w[q] * tb[q * N + i];
+    out[i] = s;
+  }
+}
+template <int N, int STRIDE, typename T>
+__device__ __forceinline__ void write_row(T* a, const T* v)
 {
 #pragma unroll
   for (int i = 0; i < N; i++) a[i * STRIDE] = v[i];
@@ -1018,6 +1032,190 @@ __global__ void __launch_bounds__((jvp_group_lanes<N, T>())) k_jvp(const ElemLau
   } else if (P.ordered) {
     scatter_element<N, NC, T, V>(r, acc, S_ + 2 * R, smem + (el > 0 && el < EB ? el - 1 : 0) * PER + 2 * R, snode,
                                  el, EB, node, li, active, P.nnodes, P.ordering, P.scatter, P.ordered == 2);
+  } else if (active) {
+#pragma unroll
+    for (int c = 0; c < NC; c++) scatter_add(r, lidx(node, c, NC, P.nnodes, P.ordering), V(acc[c]), P.scatter);
+  }
+}
+
+// J.v in FP32 arithmetic with the contractions by rows (see Rows), the stages
+// otherwise those of k_jvp (and its pairs of products where two fields meet):
+// half the LDS traffic, which bounds the BF16 tangent.  Three components and
+// p = 2, 4 (use_jvp_rows): Neo-Hookean, BF16 tangent, p = 4 36^3 188 -> 163 us,
+// p = 2 64^3 188 -> 168; FP32 tangents are bound by memory and stay within 1 %
+// (p = 2 64^3 268 -> 260).  With one component the rows fill a fifth to a third
+// of the lanes (heat p = 4: 104 -> 109), at p = 1 they take two turns
+// (mass-diffusion 105 -> 115): k_jvp there.
+template <int N, int NC>
+constexpr bool use_jvp_rows()
+{
+  return NC == 3 && N != 2;
+}
+
+template <int N, int NC, int LAYOUT, typename S, typename V>
+__global__ void __launch_bounds__((jvp_group_lanes<N, float>())) k_jvp_rows(const ElemLaunch P)
+{
+  using T             = float;
+  constexpr int  NQ   = N * N * N;
+  constexpr int  NN   = N * N;
+  constexpr int  EB   = jvp_group_lanes<N, T>() / NQ;
+  using Shape         = TanShape<LAYOUT, NC>;
+  constexpr bool FULL = Shape::VAL;
+  constexpr int  M    = Shape::M;
+  constexpr int  DS   = Shape::DS;
+  constexpr int  VO   = Shape::VO;
+  constexpr int  R    = NC * NQ;
+  constexpr int  PER  = (3 + (FULL ? 1 : 0)) * R;
+  using Lay           = TangentLayout<S, DS, NQ>;
+
+  __shared__ T   smem[EB * PER];
+  __shared__ int snode[EB * NQ];
+
+  const double  halt   = P.stop != nullptr ? *P.stop : 0.0;  // as in k_jvp
+  const int     tid    = threadIdx.x;
+  const int     el     = tid / NQ;
+  const int     li     = tid - el * NQ;
+  const int64_t slot   = P.slot_begin + logical_block(P.xcd_remap) * EB + el;
+  const bool    active = (el < EB) && (slot < P.slot_end);
+  T*            S0     = smem + (el < EB ? el : 0) * PER;
+  T *           S1 = S0 + R, *S2 = S0 + 2 * R, *S3 = S0 + 3 * R;  // S3 only where PER has it
+  const V*      u      = static_cast<const V*>(P.u);
+  V*            r      = static_cast<V*>(P.r);
+
+  const ScalarPtr<T> tB  = (ScalarPtr<T>)(uintptr_t)(P.tables + 7 * NN + 2 * N);
+  const ScalarPtr<T> tG  = tB + NN;
+  const ScalarPtr<T> tBw = tB + 2 * NN;
+  const ScalarPtr<T> tGw = tB + 3 * NN;
+
+  int64_t node = 0;
+  T       ug[NC];
+  if (active) {
+    node = P.map[size_t(slot) * NQ + li];
+#pragma unroll
+    for (int c = 0; c < NC; c++) ug[c] = T(u[lidx(node, c, NC, P.nnodes, P.ordering)]);
+  }
+  TangentRegs<T, S, DS, NQ> Dr;
+  if (active) Dr.load(static_cast<const char*>(P.D) + size_t(slot) * Lay::stride * sizeof(S), li);
+  if (halt != 0.0) return;
+  if (active) {
+#pragma unroll
+    for (int c = 0; c < NC; c++) S0[c * NQ + li] = ug[c];
+  }
+  lds_barrier();
+  for_rows<N, NC, 0>(li, active, [&](int o) {
+    T v[N], a[N], b[N];
+    read_row<N, 1>(S0 + o, v);
+    row_forward<N>(tB, v, a);
+    row_forward<N>(tG, v, b);
+    write_row<N, 1>(S0 + o, a);
+    write_row<N, 1>(S1 + o, b);
+  });
+  lds_barrier();
+  for_rows<N, NC, 1>(li, active, [&](int o) {
+    T v[N], w[N], a[N];
+    read_row<N, N>(S0 + o, v);
+    read_row<N, N>(S1 + o, w);
+    row_forward<N>(tB, v, a);
+    write_row<N, N>(S0 + o, a);
+    row_forward<N>(tB, w, a);
+    write_row<N, N>(S1 + o, a);
+    row_forward<N>(tG, v, a);
+    write_row<N, N>(S2 + o, a);
+  });
+  lds_barrier();
+  for_rows<N, NC, 2>(li, active, [&](int o) {
+    T v[N], a[N];
+    read_row<N, NN>(S1 + o, v);
+    row_forward<N>(tB, v, a);
+    write_row<N, NN>(S1 + o, a);
+    read_row<N, NN>(S2 + o, v);
+    row_forward<N>(tB, v, a);
+    write_row<N, NN>(S2 + o, a);
+    read_row<N, NN>(S0 + o, v);
+    row_forward<N>(tG, v, a);
+    write_row<N, NN>(S0 + o, a);
+    if constexpr (FULL) {
+      row_forward<N>(tB, v, a);
+      write_row<N, NN>(S3 + o, a);
+    }
+  });
+  lds_barrier();
+  if (active) {
+    T in[M], out[M];
+#pragma unroll
+    for (int c = 0; c < NC; c++) {
+      if constexpr (FULL) in[c] = S3[c * NQ + li];
+      in[VO + c * 3 + 0] = S1[c * NQ + li];
+      in[VO + c * 3 + 1] = S2[c * NQ + li];
+      in[VO + c * 3 + 2] = S0[c * NQ + li];
+    }
+#pragma unroll
+    for (int k = 0; k < M; k++) out[k] = T(0);
+#pragma unroll
+    for (int s = 0; s < M; s++)
+#pragma unroll
+      for (int rr = 0; rr < Shape::rows(s); rr++) {
+        const T Dk = Dr.get(Shape::idx(rr, s));
+        out[rr] += Dk * in[s];
+        if (Shape::SYM && rr != s) out[s] += Dk * in[rr];
+      }
+#pragma unroll
+    for (int c = 0; c < NC; c++) {
+      S0[c * NQ + li] = out[VO + c * 3 + 0];
+      S1[c * NQ + li] = out[VO + c * 3 + 1];
+      S2[c * NQ + li] = out[VO + c * 3 + 2];
+      if constexpr (FULL) S3[c * NQ + li] = out[c];
+    }
+  }
+  lds_barrier();
+  for_rows<N, NC, 0>(li, active, [&](int o) {
+    T v[N], a[N];
+    read_row<N, 1>(S0 + o, v);
+    if constexpr (FULL) {
+      T w[N];
+      read_row<N, 1>(S3 + o, w);
+      row_transposed_pair<N>(tBw, w, tGw, v, a);
+    } else {
+      row_transposed<N>(tGw, v, a);
+    }
+    write_row<N, 1>(S0 + o, a);
+    read_row<N, 1>(S1 + o, v);
+    row_transposed<N>(tBw, v, a);
+    write_row<N, 1>(S1 + o, a);
+    read_row<N, 1>(S2 + o, v);
+    row_transposed<N>(tBw, v, a);
+    write_row<N, 1>(S2 + o, a);
+  });
+  lds_barrier();
+  for_rows<N, NC, 1>(li, active, [&](int o) {
+    T v[N], w[N], a[N];
+    read_row<N, N>(S0 + o, v);
+    read_row<N, N>(S1 + o, w);
+    row_transposed_pair<N>(tBw, v, tGw, w, a);
+    write_row<N, N>(S0 + o, a);
+    read_row<N, N>(S2 + o, v);
+    row_transposed<N>(tBw, v, a);
+    write_row<N, N>(S1 + o, a);
+  });
+  lds_barrier();
+  for_rows<N, NC, 2>(li, active, [&](int o) {
+    T v[N], w[N], a[N];
+    read_row<N, NN>(S0 + o, v);
+    read_row<N, NN>(S1 + o, w);
+    row_transposed_pair<N>(tBw, v, tGw, w, a);
+    write_row<N, NN>(S2 + o, a);
+  });
+  lds_barrier();
+  T acc[NC];
+  if (active) {
+#pragma unroll
+    for (int c = 0; c < NC; c++) acc[c] = S2[c * NQ + li];
+  }
+  if (P.scatter == SCATTER_ELEMENT) {
+    store_element<N, NC>(P.E, acc, S0, slot, li, active);
+  } else if (P.ordered) {
+    scatter_element<N, NC, T, V>(r, acc, S0, smem + (el > 0 && el < EB ? el - 1 : 0) * PER, snode, el, EB, node, li,
+                                 active, P.nnodes, P.ordering, P.scatter, P.ordered == 2);
   } else if (active) {
 #pragma unroll
     for (int c = 0; c < NC; c++) scatter_add(r, lidx(node, c, NC, P.nnodes, P.ordering), V(acc[c]), P.scatter);
@@ -1616,6 +1814,8 @@ inline int dispatch_gradient(const ElemLaunch& P, hipError_t* err)
   if (P.vprec == PREC_F32) {
     if constexpr (N == 4)
       *err = launch_grid_xy<xy_elems_per_group<S>()>(P, k_jvp_xy<float, NC, LAYOUT, S, float, xy_elems_per_group<S>()>);
+    else if constexpr (use_jvp_rows<N, NC>())
+      *err = launch_grid_jvp<N, float>(P, k_jvp_rows<N, NC, LAYOUT, S, float>);
     else
       *err = launch_grid_jvp<N, float>(P, k_jvp<N, NC, LAYOUT, float, S, float>);
     return 1;
@@ -1623,6 +1823,8 @@ inline int dispatch_gradient(const ElemLaunch& P, hipError_t* err)
   if (P.vprec == PREC_MIXED) {
     if constexpr (N == 4)
       *err = launch_grid_xy<xy_elems_per_group<S>()>(P, k_jvp_xy<float, NC, LAYOUT, S, double, xy_elems_per_group<S>()>);
+    else if constexpr (use_jvp_rows<N, NC>())
+      *err = launch_grid_jvp<N, float>(P, k_jvp_rows<N, NC, LAYOUT, S, double>);
     else
       *err = launch_grid_jvp<N, float>(P, k_jvp<N, NC, LAYOUT, float, S, double>);
     return 1;

@@ -6,6 +6,7 @@
 
 #include <cmath>
 #include <cstdint>
+#include <cstring>
 #include <sstream>
 #include <stdexcept>
 #include <string>
@@ -77,11 +78,12 @@ inline void lagrange(const std::vector<double>& pts, double x, double* phi, doub
 }
 
 // Device table for N = Q = p+1: B, G, Bw, Gw as [q][n], then GL points [q] and
-// weights [q], then the diagonal's w B B, w G B, w G G as [q][n].
+// weights [q], then the diagonal's w B B, w G B, w G G as [q][n], then B, G, Bw,
+// Gw again as floats.
 inline std::vector<double> element_tables(int N)
 {
   const int           Q = N;
-  std::vector<double> t(size_t(7 * N * N + 2 * N));
+  std::vector<double> t(size_t(9 * N * N + 2 * N));
   double              xq[8], wq[8], phi[8], dphi[8];
   gauss_legendre(Q, xq, wq);
   auto pts = lobatto_points(N);
@@ -102,6 +104,9 @@ inline std::vector<double> element_tables(int N)
       d[2 * N * N + q * N + i] = dphi[i] * wq[q] * dphi[i];
     }
   }
+  float f[4 * 8 * 8];
+  for (int k = 0; k < 4 * N * N; k++) f[k] = float(t[size_t(k)]);
+  std::memcpy(&t[size_t(7 * N * N + 2 * N)], f, sizeof(float) * size_t(4 * N * N));
   return t;
 }
 
