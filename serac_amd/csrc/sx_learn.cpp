@@ -220,7 +220,7 @@ void weight_grad(sx_unet* N, int k, const void* xa, const void* xb, const float*
 }
 
 // The gradients of layer k from g = dL/d(its output) on the matrix cores: weights and bias into G, the data gradient
-// of the parts of a stride-1 layer's input into da (channels cin_a) and db (channels cin_b) where not null
+// of the input's parts into da (channels cin_a) and db (channels cin_b) where not null
 void backward_layer_mfma(sx_unet* N, int k, const void* xa, const void* xb, const float* g, float* da, float* db)
 {
   const LayerDef&    L  = kLayers[k];
@@ -239,12 +239,15 @@ void backward_layer_mfma(sx_unet* N, int k, const void* xa, const void* xb, cons
     UN_HIP(sxu::wgrad_mfma(N->xcm.as<uint16_t>(), cs[i], int(N->cin(k)), first, N->gcm.as<uint16_t>(), L.cout, P, dw, s));
   }
   if (!da && !db) return;
-  UN_HIP(sxu::planes_cl(g, y, L.cout, P, N->gcl.as<uint16_t>(), s));
+  const sxu::PadGrid Pg   = sxu::pad_grid(N->dims[L.lout]);
+  const sxu::Dims3*  fine = up == 2 ? &N->dims[L.lin] : nullptr;
+  UN_HIP(sxu::planes_cl(g, y, L.cout, Pg, N->gcl.as<uint16_t>(), s));
   if (da)
-    UN_HIP(sxu::dgrad_mfma(N->gcl.as<uint16_t>(), w, int(N->cin(k)), L.cout, 0, L.cin_a, P, N->wpl.as<uint16_t>(), da, s));
+    UN_HIP(sxu::dgrad_mfma(N->gcl.as<uint16_t>(), w, int(N->cin(k)), L.cout, 0, L.cin_a, Pg, fine, N->wpl.as<uint16_t>(),
+                           da, s));
   if (db)
-    UN_HIP(sxu::dgrad_mfma(N->gcl.as<uint16_t>(), w, int(N->cin(k)), L.cout, L.cin_a, L.cin_b, P, N->wpl.as<uint16_t>(),
-                           db, s));
+    UN_HIP(sxu::dgrad_mfma(N->gcl.as<uint16_t>(), w, int(N->cin(k)), L.cout, L.cin_a, L.cin_b, Pg, fine,
+                           N->wpl.as<uint16_t>(), db, s));
 }
 
 // backward from dL/dy (in gact[11]); gradients accumulate into G
@@ -257,11 +260,12 @@ void backward(sx_unet* N)
   auto layer = [&](int k, const void* xa, const void* xb, float* da, float* db) {
     const LayerDef& L = kLayers[k];
     float*          g = N->gact[k].as<float>();
-    const bool      strided = L.mode == 1;
-    if (N->use_mfma) backward_layer_mfma(N, k, xa, xb, g, strided ? nullptr : da, strided ? nullptr : db);
-    if (N->use_mfma && !strided) return;
+    if (N->use_mfma) {
+      backward_layer_mfma(N, k, xa, xb, g, da, db);
+      return;
+    }
     if (L.relu && !N->identity) UN_HIP(sxu::relu_bwd(g, N->act[k].as<uint16_t>(), nel(k), s));
-    if (!N->use_mfma) weight_grad(N, k, xa, xb, g);
+    weight_grad(N, k, xa, xb, g);
     if (da) data_grad(N, k, g, 0, L.cin_a, da);
     if (db) data_grad(N, k, g, L.cin_a, L.cin_b, db);
   };
@@ -379,7 +383,7 @@ void init(sx_unet* N, int nx, int ny, int nz, uint64_t seed)
   for (int k = 0; k < 12; k++) {
     const LayerDef&    L = kLayers[k];
     const sxu::PadGrid P = sxu::pad_grid(N->dims[L.lin]);
-    if (L.mode == 0) gcl = std::max(gcl, sxu::planes_cl_elems(P, L.cout));
+    gcl = std::max(gcl, sxu::planes_cl_elems(sxu::pad_grid(N->dims[L.lout]), L.cout));
     gcm = std::max(gcm, size_t(P.row) * size_t(3 * L.cout));
     xcm = std::max(xcm, size_t(P.row) * size_t(std::max(L.cin_a, L.cin_b)));
     wpl = std::max(wpl, size_t(std::max(L.cin_a, L.cin_b)) * size_t(sxu::plane_kpad(L.cout)));

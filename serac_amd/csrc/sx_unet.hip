@@ -493,31 +493,83 @@ __global__ void __launch_bounds__(kThreads) k_to_cm(const void* src, const uint1
   }
 }
 
-// wt[ci][tap'][plane][co] = w[26 - tap'][c0 + ci][co], three times over, for
-// ci < cpart: the data gradient's weights along its K, padded with zeros
-__global__ void k_weights_planes(const uint16_t* w, int cin, int cout, int c0, int cpart, int CP, int kpad, uint16_t* wt)
+// A data gradient's taps in the order of its K.  Stride 1: place t reads g at
+// the neighbour (t % 3 - 1, ...) and the forward weight 26 - t.  Stride 2: the
+// input node s = 2 i + parity takes, per direction, g at i through the middle
+// weight where it is even, and g at i and i + 1 through the weights 2 and 0
+// where it is odd; the 27 taps are grouped by the parity class (bit d: odd in
+// direction d) they belong to, 1 to 8 each.
+struct DgradTap {
+  int d[3];    // offset of the g node
+  int weight;  // tap of the forward weights
+};
+__host__ __device__ inline int dgrad_class_first(int cls)
+{
+  int n = 0;
+  for (int c = 0; c < cls; c++) n += (c & 1 ? 2 : 1) * (c & 2 ? 2 : 1) * (c & 4 ? 2 : 1);
+  return n;
+}
+__device__ inline DgradTap dgrad_tap(int t, bool strided)
+{
+  DgradTap T;
+  if (!strided) {
+    T.d[0] = t % 3 - 1, T.d[1] = (t / 3) % 3 - 1, T.d[2] = t / 9 - 1;
+    T.weight = 26 - t;
+    return T;
+  }
+  int cls = 0;
+  while (cls < 7 && dgrad_class_first(cls + 1) <= t) cls++;
+  int r = t - dgrad_class_first(cls), scale = 1;
+  T.weight = 0;
+  for (int k = 0; k < 3; k++) {
+    int tap = 1;
+    T.d[k]  = 0;
+    if ((cls >> k) & 1) {
+      T.d[k] = r & 1;
+      tap    = T.d[k] ? 0 : 2;
+      r >>= 1;
+    }
+    T.weight += tap * scale;
+    scale *= 3;
+  }
+  return T;
+}
+
+// wt[ci][place][plane][co] = w[the place's tap][c0 + ci][co], three times over,
+// for ci < cpart: the data gradient's weights along its K, padded with zeros
+__global__ void k_weights_planes(const uint16_t* w, int cin, int cout, int c0, int cpart, int CP, int kpad, int strided,
+                                 uint16_t* wt)
 {
   const int64_t n = int64_t(cpart) * kpad;
   for (int64_t t = int64_t(blockIdx.x) * kThreads + threadIdx.x; t < n; t += int64_t(gridDim.x) * kThreads) {
     const int ci = int(t / kpad), k = int(t % kpad), tap = k / CP, pc = k % CP;
-    wt[t] = tap < 27 && pc < 3 * cout ? w[(int64_t(26 - tap) * cin + c0 + ci) * cout + pc % cout] : uint16_t(0);
+    wt[t] = tap < 27 && pc < 3 * cout
+                ? w[(int64_t(dgrad_tap(tap, strided).weight) * cin + c0 + ci) * cout + pc % cout]
+                : uint16_t(0);
   }
 }
 
 // Data gradient: out[node][co] (FP32, unpadded) = sum_k planes[node + tap][plane, channel] wt[co][k], an implicit
 // GEMM of 16-node row tiles by 16-channel column tiles on mfma_f32_16x16x32_bf16.  KS = 1: a wave owns RT row tiles
 // and NT column tiles, all of K.  KS = 4 (coarse levels, where that leaves most of the GPU idle): the workgroup's
-// four waves share one row tile's K and add their parts in LDS.
+// four waves share one row tile's K and add their parts in LDS.  Stride 2 (fine
+// set): blockIdx.z is the parity class of the output nodes 2 i + parity, K its
+// taps, and i runs over the padded grid of g.
 // 65^3 grid, 16 <- 32 channels: 105 us where the vector units took 304; 17^3, 64 <- 64: 66 us (107).
 template <int NT, int RT, int KS>
-__global__ void __launch_bounds__(kThreads) k_dgrad(const uint16_t* planes, int CP, const uint16_t* wt, int kpad, int K,
-                                                    PadGrid P, float* out, int cout)
+__global__ void __launch_bounds__(kThreads) k_dgrad(const uint16_t* planes, int CP, const uint16_t* wt, int kpad,
+                                                    PadGrid P, float* out, int cout, Dims3 fine)
 {
   extern __shared__ int soff[];  // element offset of every 8-channel group of K
-  for (int t = threadIdx.x; t < kpad / 8; t += kThreads) {
-    const int k = 8 * t, tap = k / CP;
-    const int d = (tap % 3 - 1) + P.px * ((tap / 3) % 3 - 1) + P.px * P.py * (tap / 9 - 1);
-    soff[t]     = k < K ? d * CP + (k - tap * CP) : 0;  // past K the weights are zero
+  const bool strided = fine.n[0] > 0;
+  const int  cls     = int(blockIdx.z);
+  // this launch's part of K: a class's taps (whole K steps, its CP is a multiple of 32), or all of it
+  const int kbeg = strided ? dgrad_class_first(cls) * CP : 0, kend = strided ? dgrad_class_first(cls + 1) * CP : kpad;
+  for (int t = threadIdx.x; t < (kend - kbeg) / 8; t += kThreads) {
+    const int      k = kbeg + 8 * t, tap = k / CP;
+    const DgradTap T = dgrad_tap(tap < 27 ? tap : 0, strided);
+    soff[t]          = tap < 27 ? (T.d[0] + P.px * T.d[1] + P.px * P.py * T.d[2]) * CP + (k - tap * CP)
+                                : 0;  // past K the weights are zero
   }
   __syncthreads();
   const int lane = int(threadIdx.x) & 63, wave = int(threadIdx.x) >> 6;
@@ -532,8 +584,8 @@ __global__ void __launch_bounds__(kThreads) k_dgrad(const uint16_t* planes, int 
   const uint16_t* pa[RT];
 #pragma unroll
   for (int rt = 0; rt < RT; rt++) pa[rt] = planes + (int64_t(P.guard) + min(base + rt * 16 + m, P.nodes - 1)) * CP;
-  const uint16_t* pb = wt + int64_t(ct0 * 16 + m) * kpad;
-  const int       steps = kpad / 32;
+  const uint16_t* pb = wt + int64_t(ct0 * 16 + m) * kpad + kbeg;
+  const int       steps = (kend - kbeg) / 32;
   const int       s0 = KS == 1 ? 0 : steps * wave / KS, s1 = KS == 1 ? steps : steps * (wave + 1) / KS;
 #pragma unroll 4
   for (int s = s0; s < s1; s++) {
@@ -568,7 +620,16 @@ __global__ void __launch_bounds__(kThreads) k_dgrad(const uint16_t* planes, int 
       const int v = base + rt * 16 + 4 * kg + r;
       int       ix, iy, iz;
       if (v >= P.nodes || !pad_interior(v, P, ix, iy, iz)) continue;
-      float* o = out + ((int64_t(iz) * (P.py - 2) + iy) * (P.px - 2) + ix) * cout + ct0 * 16 + m;
+      int nx = P.px - 2, ny = P.py - 2;
+      if (strided) {
+        ix = 2 * ix + (cls & 1);
+        iy = 2 * iy + ((cls >> 1) & 1);
+        iz = 2 * iz + (cls >> 2);
+        nx = fine.n[0];
+        ny = fine.n[1];
+        if (ix >= nx || iy >= ny || iz >= fine.n[2]) continue;
+      }
+      float* o = out + ((int64_t(iz) * ny + iy) * nx + ix) * cout + ct0 * 16 + m;
 #pragma unroll
       for (int ct = 0; ct < NT; ct++) o[ct * 16] = acc[rt][ct][r];
     }
@@ -580,7 +641,7 @@ __global__ void __launch_bounds__(kThreads) k_dgrad(const uint16_t* planes, int 
 // each wave every fourth tap; the parts are added with FP32 atomics.  x at
 // o + tap is 16 bytes at any 2-byte address, read straight from memory (the
 // rows of a tile stay in the caches across taps).
-// 65^3 grid, 32 x 16 channels: 192 us where the vector units took 880.  Bound by the latency of the loads.
+// 65^3 grid, 32 x 16 channels: 198 us where the vector units took 880.  Bound by the latency of the loads.
 __global__ void __launch_bounds__(kThreads) k_wgrad(const uint16_t* x, int cin, const uint16_t* g, int cout, PadGrid P,
                                                     int steps_per_run, float* dw, int cin_all, int ci_first)
 {
@@ -1045,28 +1106,28 @@ hipError_t input_cm(const uint16_t* x, int cin, Dims3 d, const PadGrid& P, uint1
 }
 
 hipError_t dgrad_mfma(const uint16_t* planes, const uint16_t* w, int cin, int cout, int c0, int cpart, const PadGrid& P,
-                      uint16_t* wt, float* out, hipStream_t s)
+                      const Dims3* fine, uint16_t* wt, float* out, hipStream_t s)
 {
-  if (cpart % 16) return hipErrorInvalidValue;
-  const int CP = plane_channels(cout), kpad = plane_kpad(cout), K = 27 * CP;
+  const int CP = plane_channels(cout), kpad = plane_kpad(cout);
+  if (cpart % 16 || (fine && CP % 32)) return hipErrorInvalidValue;
   hipLaunchKernelGGL(k_weights_planes, dim3(std::min<unsigned>(blocks_for(int64_t(cpart) * kpad), 2048)), dim3(kThreads),
-                     0, s, w, cin, cout, c0, cpart, CP, kpad, wt);
-  const size_t shmem = size_t(kpad / 8) * sizeof(int);
-  const dim3   block{unsigned(kThreads)};
+                     0, s, w, cin, cout, c0, cpart, CP, kpad, fine ? 1 : 0, wt);
+  const size_t   shmem = size_t((fine ? 8 * CP : kpad) / 8) * sizeof(int);
+  const dim3     block{unsigned(kThreads)};
+  const unsigned tiles = unsigned((P.nodes + 15) / 16), cls = fine ? 8u : 1u;
+  const Dims3    f     = fine ? *fine : Dims3{{0, 0, 0}};
   if (P.nodes < kChannelParallelBelow) {
-    const dim3 g{unsigned((P.nodes + 15) / 16), unsigned(cpart / 16)};
-    hipLaunchKernelGGL((k_dgrad<1, 1, 4>), g, block, shmem, s, planes, CP, wt, kpad, K, P, out, cpart);
+    hipLaunchKernelGGL((k_dgrad<1, 1, 4>), dim3(tiles, unsigned(cpart / 16), cls), block, shmem, s, planes, CP, wt, kpad, P,
+                       out, cpart, f);
+  } else if (cpart % 64 == 0) {
+    hipLaunchKernelGGL((k_dgrad<4, 1, 1>), dim3((tiles + 3) / 4, unsigned(cpart / 64), cls), block, shmem, s, planes, CP,
+                       wt, kpad, P, out, cpart, f);
+  } else if (cpart % 32 == 0) {
+    hipLaunchKernelGGL((k_dgrad<2, 2, 1>), dim3((tiles + 7) / 8, unsigned(cpart / 32), cls), block, shmem, s, planes, CP,
+                       wt, kpad, P, out, cpart, f);
   } else {
-    const unsigned tiles = unsigned((P.nodes + 15) / 16);
-    if (cpart % 64 == 0)
-      hipLaunchKernelGGL((k_dgrad<4, 1, 1>), dim3((tiles + 3) / 4, unsigned(cpart / 64)), block, shmem, s, planes, CP, wt,
-                         kpad, K, P, out, cpart);
-    else if (cpart % 32 == 0)
-      hipLaunchKernelGGL((k_dgrad<2, 2, 1>), dim3((tiles + 7) / 8, unsigned(cpart / 32)), block, shmem, s, planes, CP, wt,
-                         kpad, K, P, out, cpart);
-    else
-      hipLaunchKernelGGL((k_dgrad<1, 2, 1>), dim3((tiles + 7) / 8, unsigned(cpart / 16)), block, shmem, s, planes, CP, wt,
-                         kpad, K, P, out, cpart);
+    hipLaunchKernelGGL((k_dgrad<1, 2, 1>), dim3((tiles + 7) / 8, unsigned(cpart / 16), cls), block, shmem, s, planes, CP,
+                       wt, kpad, P, out, cpart, f);
   }
   return hipGetLastError();
 }
@@ -1075,8 +1136,8 @@ hipError_t wgrad_mfma(const uint16_t* x_cm, int cin, int cin_all, int ci_first, 
                       const PadGrid& P, float* dw, hipStream_t s)
 {
   const int tiles = (cin + 15) / 16 * ((cout + 15) / 16), steps = (P.nodes + 31) / 32;
-  // about 768 workgroups, at least 8 steps each
-  const int runs = std::max(1, std::min(steps / 8, (768 + tiles - 1) / tiles));
+  // about 256 workgroups, at least 8 steps each
+  const int runs = std::max(1, std::min(steps / 8, (256 + tiles - 1) / tiles));
   const int per  = (steps + runs - 1) / runs;
   hipLaunchKernelGGL(k_wgrad, dim3(unsigned((steps + per - 1) / per), unsigned(tiles)), dim3(kThreads), 0, s, x_cm, cin,
                      g_cm, cout, P, per, dw, cin_all, ci_first);

@@ -54,8 +54,7 @@ bool       conv_mfma_supported(const ConvArgs& A, int cout, bool in_f32, bool ou
 hipError_t weights_kmajor(const uint16_t* w, int cin, int cout, uint16_t* wt, hipStream_t s);
 hipError_t conv_mfma(const ConvArgs& A, int cout, const uint16_t* wt, hipStream_t s);
 hipError_t conv_wgrad(const WGradArgs& A, int cout, bool in_f32, hipStream_t s);
-// Backward convolutions of stride-1 layers (and the weight gradient of the
-// stride-2 ones) on the matrix cores.  The FP32 gradient is split into three
+// Backward convolutions on the matrix cores.  The FP32 gradient is split into three
 // BF16 planes, over a grid padded by one node on each side:
 struct PadGrid {
   int     px, py, pz, nodes;  // padded dims and their product
@@ -72,10 +71,11 @@ hipError_t planes_cl(const float* g, const uint16_t* y, int cout, const PadGrid&
 hipError_t planes_cm(const float* g, const uint16_t* y, int cout, int up, Dims3 d, const PadGrid& P, uint16_t* out,
                      hipStream_t s);
 hipError_t input_cm(const uint16_t* x, int cin, Dims3 d, const PadGrid& P, uint16_t* out, hipStream_t s);
-// out [node][cpart] = the gradient of input channels c0 .. c0 + cpart - 1 (cpart a multiple of 16); wt: scratch of
-// cpart * plane_kpad(cout)
+// out [node][cpart] = the gradient of input channels c0 .. c0 + cpart - 1 (cpart a multiple of 16); planes: planes_cl of
+// g on its own grid P; fine: the input's grid where the layer has stride 2 (cout then a multiple of 32), or null; wt:
+// scratch of cpart * plane_kpad(cout)
 hipError_t dgrad_mfma(const uint16_t* planes, const uint16_t* w, int cin, int cout, int c0, int cpart, const PadGrid& P,
-                      uint16_t* wt, float* out, hipStream_t s);
+                      const Dims3* fine, uint16_t* wt, float* out, hipStream_t s);
 // dw[tap][ci_first + ci][co] += for the cin channels of x_cm
 hipError_t wgrad_mfma(const uint16_t* x_cm, int cin, int cin_all, int ci_first, const uint16_t* g_cm, int cout,
                       const PadGrid& P, float* dw, hipStream_t s);
