@@ -88,7 +88,7 @@ def unet_bench(sx, n, steps, warmup):
         "forward_tflops": round(fl / t_fwd / 1e12, 2),
         "train_tflops": round(3 * fl / t_train / 1e12, 2),
         "flops_note": "2 x multiply-adds of the 3x3x3 convolutions; a training step counts 3x the forward",
-        "kernels": "direct convolution on FP32 FMA units (BF16 weights and activations, FP32 accumulation)",
+        "kernels": "matrix-core implicit GEMM (BF16 weights and activations, FP32 gradients as three BF16 planes, FP32 accumulation)",
         "peak_tflops_fp32_vector": 157.3,
         "peak_tflops_bf16_mfma_dense": 2500.0,
     }
