@@ -2217,7 +2217,7 @@ double read_scalar(sx_form* f, int slot)
 }
 
 struct Workspace {
-  DeviceBuffer r, z, d, Ad, diag, ess, t, part2;
+  DeviceBuffer r, z, d, Ad, diag, ess, t, part2, mask;
   DeviceBuffer V, hb, gpart;  // GMRES basis, coefficients, partial dots
   DeviceBuffer Zb;            // flexible GMRES: the preconditioned directions
   DeviceBuffer gs;            // GMRES least-squares state (sxk::gmres_state_doubles)
@@ -2247,9 +2247,12 @@ void compute_diag(sx_grad* g, const int32_t* ess_dev, int64_t ness, double* diag
 }
 
 // The device vectors of one Jacobi-CG solve: five of ndof doubles and the
-// reduction_blocks() partials of (r, z).
+// reduction_blocks() partials of (r, z).  With a mask (a byte an entry, room
+// for the essential rows) the copy of these rows goes with the scalar product;
+// a caller's own work memory has none, and there it is a launch.
 struct CgVectors {
-  double *r, *z, *d, *Ad, *diag, *part_rz;
+  double * r, *z, *d, *Ad, *diag, *part_rz;
+  uint8_t* mask;
 };
 
 CgVectors cg_vectors(Workspace& w, int64_t n)
@@ -2260,8 +2263,9 @@ CgVectors cg_vectors(Workspace& w, int64_t n)
   w.Ad.allocate(size_t(n) * 8);
   w.diag.allocate(size_t(n) * 8);
   w.part2.allocate(size_t(sxk::reduction_blocks()) * 8);
+  w.mask.allocate(size_t(n));
   return {w.r.as<double>(), w.z.as<double>(), w.d.as<double>(), w.Ad.as<double>(), w.diag.as<double>(),
-          w.part2.as<double>()};
+          w.part2.as<double>(), w.mask.as<uint8_t>()};
 }
 
 void cg_core(sx_grad* g, const int32_t* ess_dev, int64_t ness, const double* b, double* x, double rel,
@@ -2292,12 +2296,22 @@ void cg_core(sx_grad* g, const int32_t* ess_dev, int64_t ness, const double* b, 
   // unconverged with x = 0
   if (rep->converged || nom0 < 0.0) return;
 
-  auto apply_bc = [&](const double* in, double* outv) {
-    apply_gradient(g, in, outv);
-    SX_HIP(sxk::copy_rows(outv, in, ess_dev, ness, s));
+  uint8_t* mask = ness > 0 ? v.mask : nullptr;
+  if (mask) {
+    SX_HIP(hipMemsetAsync(mask, 0, size_t(n), s));
+    SX_HIP(sxm::rows_mask(ess_dev, ness, mask, s));
+  }
+  // the essential rows of Ad, then the partials of (d, Ad)
+  auto rows_and_dot = [&] {
+    if (mask) {
+      SX_HIP(sxk::dot_rows(d, Ad, mask, n, part, s));
+    } else {
+      SX_HIP(sxk::copy_rows(Ad, d, ess_dev, ness, s));
+      SX_HIP(sxk::dot_partial(d, Ad, n, part, s));
+    }
   };
-  // One iteration is five launches: the J.v (into the Ad that cg_step_x
-  // zeroed), the essential rows, the partials of (d, Ad), then cg_step_x and
+  // One iteration is the J.v (into the Ad that cg_step_x zeroed), the
+  // essential rows with the partials of (d, Ad), then cg_step_x and
   // cg_step_d, which reduce the partials themselves.  The convergence test
   // runs on the device (scal[8] = stop flag, scal[9] = the iteration that set
   // it): once (r, z) <= goal the step kernels leave x, r, z, d and the scalars
@@ -2309,8 +2323,8 @@ void cg_core(sx_grad* g, const int32_t* ess_dev, int64_t ness, const double* b, 
   double* part_rz = v.part_rz;
   double* stop    = scal + 8;
   SX_HIP(sxk::vec_fill(stop, 0.0, 2, s));
-  apply_bc(d, Ad);
-  SX_HIP(sxk::dot_partial(d, Ad, n, part, s));
+  apply_gradient(g, d, Ad);
+  rows_and_dot();
   int it = 1;
   while (it <= max_iter) {
     const int chunk = hook ? 1 : std::min(std::max(it / 4, 1), std::min(32, max_iter - it + 1));
@@ -2319,8 +2333,7 @@ void cg_core(sx_grad* g, const int32_t* ess_dev, int64_t ness, const double* b, 
       if (hook) (*hook)(it, x, r);
       SX_HIP(sxk::cg_step_d(d, z, scal, part_rz, n, goal, it, stop, s));
       apply_gradient(g, d, Ad, nullptr, nullptr, sxk::PREC_F64, true, false, stop);
-      SX_HIP(sxk::copy_rows(Ad, d, ess_dev, ness, s));
-      SX_HIP(sxk::dot_partial(d, Ad, n, part, s));
+      rows_and_dot();
     }
     double st[7];  // scal[3..9]
     SX_HIP(hipMemcpyAsync(st, scal + 3, sizeof(st), hipMemcpyDeviceToHost, s));

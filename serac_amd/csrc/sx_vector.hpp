@@ -20,6 +20,7 @@ hipError_t vec_dot_dev(const double* a, const double* b, int64_t n, double* part
 // kernel's reduction_blocks() partials itself (in the fixed order of
 // k_reduce_final's sum):
 //   dot_partial: part = partials of (a, b)
+//   dot_rows:    b = a where mask is set, then part = partials of (a, b)
 //   cg_step_x:   alpha = scal[0] / sum(part_den); x += alpha d; r -= alpha Ad;
 //                z = r/diag; Ad = 0; part_rz = partials of (r, z);
 //                scal[1] = den, scal[2] = alpha, scal[5] = scal[0]
@@ -30,6 +31,7 @@ hipError_t vec_dot_dev(const double* a, const double* b, int64_t n, double* part
 //                (betanom not a number)
 // Both leave everything alone once stop[0] is set (stop: device {code, iteration}).
 hipError_t dot_partial(const double* a, const double* b, int64_t n, double* part, hipStream_t s);
+hipError_t dot_rows(const double* a, double* b, const uint8_t* mask, int64_t n, double* part, hipStream_t s);
 hipError_t cg_step_x(double* x, double* r, double* z, double* Ad, const double* d, const double* diag, double* scal,
                      const double* part_den, double* part_rz, int64_t n, const double* stop, hipStream_t s);
 hipError_t cg_step_d(double* d, const double* z, double* scal, const double* part_rz, int64_t n, double goal, int it,
