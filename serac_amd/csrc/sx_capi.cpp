@@ -234,7 +234,7 @@ struct Integral {
   double               params[SX_MAX_PARAMS] = {0};
   std::vector<int>     depends_on;
   int64_t              nslots = 0;
-  std::vector<int64_t> color_off;  // [ncolors + 1] slot ranges (of `d_order` where node_sum)
+  std::vector<int64_t> color_off;  // [launches + 1] slot ranges (of `d_order` where node_sum)
   // reproducible scatter: the element kernels store their values (sx_form::E)
   // and a node sum follows; otherwise one launch per colour (one range in all
   // with atomics)
@@ -451,9 +451,9 @@ sxk::ElemLaunch base_launch(const sx_form* f, const Integral& I, int mode)
 // filled GPU each time.  Before -> after: a Jacobi-CG iteration p = 2 on 16x5x4
 // elements 60 -> 25 us, Neo-Hookean residual p = 2 on 57x48x43 214 -> 180 us,
 // FP64 J.v p = 3 on 40^3 364 -> 306 us, with a BF16 tangent 174 -> 125 us.
-// Colours remain for domains that list an element twice and for values beyond
-// kNodeSumBytes (J.v p = 3 on 64^3, 403 MB: 1.35 ms with colours, 1.39 with
-// the sum; BF16 tangent 0.52 and 0.54).
+// Colours remain for domains that list an element twice (a range per repetition
+// and colour) and for values beyond kNodeSumBytes (J.v p = 3 on 64^3, 403 MB:
+// 1.35 ms with colours, 1.39 with the sum; BF16 tangent 0.52 and 0.54).
 int run_slots(const sx_form* f_, const Integral& I, sxk::ElemLaunch& P, void* r, bool set, hipEvent_t* ev)
 {
   sx_form*   f = const_cast<sx_form*>(f_);
@@ -1362,19 +1362,29 @@ int sx_form_add_domain_integral(sx_form* f, int qfunc_id, const double* params, 
   return sx_form_add_domain_integral_qdata(f, qfunc_id, params, nparams, depends_on, ndep, elems, nelem, nullptr);
 }
 
+}  // extern "C"
+
 namespace {
 
-// One domain integral of qfunction qfunc_id in trial argument `trial`
-// (companion: the mass part of a two-argument integral).
-// positions sorted by colour (stable) and the colours' ranges
-std::vector<int> by_color(const std::vector<int>& color, int ncolors, std::vector<int64_t>& off)
+// Positions of `domain` sorted by launch (stable) and the launches' ranges: no
+// two elements of a launch share a node.  The k-th listing of an element goes
+// with its colour's k-th launch: two listings of one element in one launch
+// would update the same nodes at the same time.
+std::vector<int> by_color(const sx_space* s, const std::vector<int>& domain, std::vector<int64_t>& off)
 {
-  off.assign(size_t(ncolors) + 1, 0);
-  for (int c : color) off[size_t(c) + 1]++;
-  for (int c = 0; c < ncolors; c++) off[size_t(c) + 1] += off[size_t(c)];
+  std::vector<int> listed(size_t(s->mesh->m.ne), 0), launch(domain.size());
+  int              n = s->ncolors;
+  for (size_t i = 0; i < domain.size(); i++) {
+    const size_t e = size_t(domain[i]);
+    launch[i]      = listed[e]++ * s->ncolors + s->color[e];
+    n              = std::max(n, listed[e] * s->ncolors);
+  }
+  off.assign(size_t(n) + 1, 0);
+  for (int l : launch) off[size_t(l) + 1]++;
+  for (int l = 0; l < n; l++) off[size_t(l) + 1] += off[size_t(l)];
   std::vector<int64_t> at(off.begin(), off.end() - 1);
-  std::vector<int>     pos(color.size());
-  for (size_t i = 0; i < color.size(); i++) pos[size_t(at[size_t(color[i])]++)] = int(i);
+  std::vector<int>     pos(domain.size());
+  for (size_t i = 0; i < domain.size(); i++) pos[size_t(at[size_t(launch[i])]++)] = int(i);
   return pos;
 }
 
@@ -1420,15 +1430,14 @@ bool prepare_node_sum(sx_form* f, Integral& I, const std::vector<int>& domain)
 void assembly_order(sx_form* f, Integral& I)
 {
   std::lock_guard<std::mutex> lk(f->e_mu);
-  const sx_space*             vs = f->test;
   if (!I.node_sum || I.elems.empty()) return;
-  std::vector<int> color(I.elems.size());
-  for (size_t i = 0; i < color.size(); i++) color[i] = vs->color[size_t(I.elems[i])];
-  I.d_order.upload(by_color(color, vs->ncolors, I.color_off));
+  I.d_order.upload(by_color(f->test, I.elems, I.color_off));
   I.elems.clear();
   I.elems.shrink_to_fit();
 }
 
+// One domain integral of qfunction qfunc_id in trial argument `trial`
+// (companion: the mass part of a two-argument integral).
 void add_domain_integral_one(sx_form* f, int qfunc_id, const double* params, int nparams, int trial, const int* elems,
                              int nelem, sx_qdata* qdata, bool companion)
 {
@@ -1480,11 +1489,7 @@ void add_domain_integral_one(sx_form* f, int qfunc_id, const double* params, int
   I->color_off = {0, int64_t(pos.size())};
   if (f->scatter != SX_SCATTER_ATOMIC) {
     I->node_sum = prepare_node_sum(f, *I, domain);
-    if (!I->node_sum) {
-      std::vector<int> elem_color(domain.size());
-      for (size_t i = 0; i < domain.size(); i++) elem_color[i] = vs->color[size_t(domain[i])];
-      pos = by_color(elem_color, vs->ncolors, I->color_off);
-    }
+    if (!I->node_sum) pos = by_color(vs, domain, I->color_off);
   }
   std::vector<int> slots(pos.size());
   for (size_t k = 0; k < pos.size(); k++) slots[k] = domain[size_t(pos[k])];
@@ -1530,6 +1535,8 @@ bool rate_coefficient(int qf, const double* params, int nparams, double* coef)
 }
 
 }  // namespace
+
+extern "C" {
 
 int sx_form_add_domain_integral_qdata(sx_form* f, int qfunc_id, const double* params, int nparams,
                                       const int* depends_on, int ndep, const int* elems, int nelem, sx_qdata* qdata)
