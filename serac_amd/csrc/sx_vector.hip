@@ -601,68 +601,54 @@ hipError_t scatter_e(const int64_t* offs, const int32_t* ents, const double* E, 
   return hipGetLastError();
 }
 
-// r (+)= sum of the element values E of each node, in increasing element order
-// (reproducible).  E holds npe * NC values per domain position, node-major; pos
-// maps an element to its domain position, -1 outside (null: the same).  A
-// thread per node and component: the nodes of an element row are neighbours in
-// r and in E, so a wave reads runs of both.  What it waits for is the chain
-// offsets -> entries -> values, so four entries go side by side.
+// r (+)= sum of the element values E of each listed node, in the order of its
+// entries (node_sum in sx_vector.hpp).  E holds npe * NC values per domain
+// position, node-major.  A thread per node and component: the nodes of an
+// element row are neighbours in r and in E, so a wave reads runs of both.  What
+// it waits for is the chain offsets -> entries -> values, so four entries go
+// side by side.
 // J.v p = 1 on 96^3: 54 us (84 with a thread per node, whose 24-byte strides
 // cost three times the cache accesses); p = 3 on 64^3: 211 us.
 template <typename T, typename V, int NC>
-__global__ void __launch_bounds__(kThreads) k_node_sum(const int64_t* offs, const int32_t* ents, const int32_t* pos,
-                                                        const T* E, V* r, unsigned nnodes, unsigned npe, int vdim,
+__global__ void __launch_bounds__(kThreads) k_node_sum(const int32_t* nodes, const int64_t* offs, const int32_t* ents,
+                                                        const T* E, V* r, unsigned n, unsigned nnodes, int vdim,
                                                         int add, const double* stop)
 {
   const double halt = stop != nullptr ? *stop : 0.0;  // looked at before the store: no wait of its own
   // each XCD takes a contiguous run of nodes: the lines of E that neighbouring node rows share meet in one L2
-  const unsigned per  = gridDim.x / 8;
-  const unsigned blk  = blockIdx.x < per * 8 ? (blockIdx.x % 8) * per + blockIdx.x / 8 : blockIdx.x;
-  const unsigned i    = blk * kThreads + threadIdx.x;
-  const unsigned node = i / NC, c = i - node * NC;
-  if (node >= nnodes) return;
-  int       k   = int(offs[node]);  // entries are numbered in int32
-  const int k1  = int(offs[node + 1]);
-  V*        out = r + (vdim ? i : c * nnodes + node);
-  V         acc = add ? *out : V(0);
+  const unsigned per = gridDim.x / 8;
+  const unsigned blk = blockIdx.x < per * 8 ? (blockIdx.x % 8) * per + blockIdx.x / 8 : blockIdx.x;
+  const unsigned i   = blk * kThreads + threadIdx.x;
+  const unsigned t   = i / NC, c = i - t * NC;
+  if (t >= n) return;
+  int            k    = int(offs[t]);  // entries are numbered in int32
+  const int      k1   = int(offs[t + 1]);
+  const unsigned node = nodes != nullptr ? unsigned(nodes[t]) : t;
+  V*             out  = r + (vdim ? node * NC + c : c * nnodes + node);
+  V              acc  = add ? *out : V(0);
   for (; k < k1; k += 4) {
-    int at[4];  // the entry's value, -1: no entry
-#pragma unroll
-    for (int m = 0; m < 4; m++) {
-      at[m] = -1;
-      if (k + m < k1) {
-        unsigned ej = unsigned(ents[k + m]);
-        if (pos == nullptr) {
-          at[m] = int(ej * NC + c);
-        } else {
-          const unsigned e = ej / npe;
-          const int      q = pos[e];
-          if (q >= 0) at[m] = int((unsigned(q) * npe + (ej - e * npe)) * NC + c);
-        }
-      }
-    }
     T v[4];
 #pragma unroll
-    for (int m = 0; m < 4; m++) v[m] = at[m] >= 0 ? E[at[m]] : T(0);
+    for (int m = 0; m < 4; m++) v[m] = k + m < k1 ? E[ents[k + m] * NC + int(c)] : T(0);
 #pragma unroll
     for (int m = 0; m < 4; m++)
-      if (at[m] >= 0) acc += V(v[m]);
+      if (k + m < k1) acc += V(v[m]);
   }
   if (halt == 0.0) *out = acc;
 }
 
 template <typename T, typename V>
-hipError_t launch_node_sum(const int64_t* offs, const int32_t* ents, const int32_t* pos, const void* E, void* r,
-                           unsigned nnodes, unsigned npe, int nc, int ordering, int add, const double* stop,
+hipError_t launch_node_sum(const int32_t* nodes, const int64_t* offs, const int32_t* ents, const void* E, void* r,
+                           unsigned n, unsigned nnodes, int nc, int ordering, int add, const double* stop,
                            hipStream_t s)
 {
-  const dim3 g((nnodes * unsigned(nc) + kThreads - 1) / kThreads), b(kThreads);
+  const dim3 g((n * unsigned(nc) + kThreads - 1) / kThreads), b(kThreads);
   const T*   e = static_cast<const T*>(E);
   V*         o = static_cast<V*>(r);
   if (nc == 1)
-    hipLaunchKernelGGL((k_node_sum<T, V, 1>), g, b, 0, s, offs, ents, pos, e, o, nnodes, npe, ordering, add, stop);
+    hipLaunchKernelGGL((k_node_sum<T, V, 1>), g, b, 0, s, nodes, offs, ents, e, o, n, nnodes, ordering, add, stop);
   else
-    hipLaunchKernelGGL((k_node_sum<T, V, 3>), g, b, 0, s, offs, ents, pos, e, o, nnodes, npe, ordering, add, stop);
+    hipLaunchKernelGGL((k_node_sum<T, V, 3>), g, b, 0, s, nodes, offs, ents, e, o, n, nnodes, ordering, add, stop);
   return hipGetLastError();
 }
 
@@ -689,16 +675,16 @@ hipError_t e_transpose(const double* in, double* out, int64_t ne, int nc, int np
   return hipGetLastError();
 }
 
-hipError_t node_sum(const int64_t* offs, const int32_t* ents, const int32_t* pos, const void* E, bool e_f32, void* r,
-                    bool r_f32, int64_t nnodes, int npe, int nc, int ordering, bool add, const double* stop,
-                    hipStream_t s)
+hipError_t node_sum(const int32_t* nodes, const int64_t* offs, const int32_t* ents, int64_t n, const void* E,
+                    bool e_f32, void* r, bool r_f32, int64_t nnodes, int nc, int ordering, bool add,
+                    const double* stop, hipStream_t s)
 {
-  if (nnodes <= 0) return hipSuccess;
-  if (nnodes * nc > INT32_MAX || (nc != 1 && nc != 3)) return hipErrorInvalidValue;
-  const unsigned n = unsigned(nnodes);
-  if (r_f32) return launch_node_sum<float, float>(offs, ents, pos, E, r, n, unsigned(npe), nc, ordering, int(add), stop, s);
-  if (e_f32) return launch_node_sum<float, double>(offs, ents, pos, E, r, n, unsigned(npe), nc, ordering, int(add), stop, s);
-  return launch_node_sum<double, double>(offs, ents, pos, E, r, n, unsigned(npe), nc, ordering, int(add), stop, s);
+  if (n <= 0) return hipSuccess;
+  if (nnodes * nc > INT32_MAX || n > nnodes || (nc != 1 && nc != 3)) return hipErrorInvalidValue;
+  const unsigned m = unsigned(n), nn = unsigned(nnodes);
+  if (r_f32) return launch_node_sum<float, float>(nodes, offs, ents, E, r, m, nn, nc, ordering, int(add), stop, s);
+  if (e_f32) return launch_node_sum<float, double>(nodes, offs, ents, E, r, m, nn, nc, ordering, int(add), stop, s);
+  return launch_node_sum<double, double>(nodes, offs, ents, E, r, m, nn, nc, ordering, int(add), stop, s);
 }
 
 hipError_t csr_spmv(const int64_t* rp, const int32_t* col, const double* val, const double* x, double* y,

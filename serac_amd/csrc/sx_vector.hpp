@@ -77,14 +77,15 @@ hipError_t gather_e(const int* map, const double* L, double* E, int64_t ne, int 
 hipError_t scatter_e(const int64_t* offs, const int32_t* ents, const double* E, double* L, int64_t nnodes, int npe,
                      int nc, int ordering, hipStream_t s);
 
-// r (+)= per node, the sum of its element values E in increasing element order
-// (the layout SCATTER_ELEMENT kernels write; pos: element -> domain position,
-// -1 outside, or null); e_f32 / r_f32: E / r in FP32 (an FP32 r has an FP32 E).
+// r (+)= per listed node, the sum of its element values E (the layout that
+// SCATTER_ELEMENT kernels write).  The lists: node t of n is nodes[t] (null: t),
+// its values, at their place's number in E / nc (domain position * npe + local
+// node), are ents[offs[t]] .. ents[offs[t + 1] - 1], added in that order; E has
+// at most 2^31 values.  e_f32 / r_f32: E / r in FP32 (an FP32 r has an FP32 E).
 // Leaves r alone when *stop is set.
-hipError_t node_sum(const int64_t* offs, const int32_t* ents, const int32_t* pos, const void* E, bool e_f32, void* r,
-                    bool r_f32, int64_t nnodes, int npe, int nc, int ordering, bool add, const double* stop,
-                    hipStream_t s);
-
+hipError_t node_sum(const int32_t* nodes, const int64_t* offs, const int32_t* ents, int64_t n, const void* E,
+                    bool e_f32, void* r, bool r_f32, int64_t nnodes, int nc, int ordering, bool add,
+                    const double* stop, hipStream_t s);
 // E-vector layouts: dir 0 copies the reference layout [e][c][j] into the
 // component-major [c][e][j], dir 1 back
 hipError_t e_transpose(const double* in, double* out, int64_t ne, int nc, int npe, int dir, hipStream_t s);

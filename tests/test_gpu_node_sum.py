@@ -89,3 +89,26 @@ def test_two_threads_on_one_form(gpu_lib):
     f.synchronize()
     for k in range(2):
         assert all(np.array_equal(o.numpy(), want[k]) for o in outs[k])
+
+
+@pytest.mark.parametrize("which", ["one", "few", "all out of order"])
+@pytest.mark.parametrize("ordering", [0, 1])
+def test_lists_of_a_part(gpu_lib, which, ordering):
+    """A domain's own node lists: a part below and one above a sixteenth of the nodes, and every node."""
+    space = sx.Space(sx.Mesh.cuboid(9, 8, 7), 2, 3, ordering)
+    elems = np.random.default_rng(6).permutation(space.ne)[: {"one": 1, "few": 60}.get(which)]
+    U = sx.DeviceVector.from_numpy(W.nodal_field(space.nnodes, 3, 3, 2000, -1e-3, 1e-3, ordering))
+    v = sx.DeviceVector.from_numpy(W.nodal_field(space.nnodes, 3, 4, 3000, -1.0, 1.0, ordering))
+    got = []
+    for scatter in (capi.SX_SCATTER_COLORED, capi.SX_SCATTER_ATOMIC):
+        f = form_on(space, scatter, [elems])
+        r = f(0.0, U).numpy()  # its first call: the output holds what the allocation held
+        _, grad = f(0.0, U, wrt=0)
+        jv = sx.DeviceVector.from_numpy(np.full(space.ndof, np.nan))
+        grad.mult(v, jv)
+        ess = space.boundary_dofs(0b1)
+        x = sx.DeviceVector(space.ndof)
+        rep = grad.cg(ess, v, x, rel_tol=1e-9, max_iter=3, raise_on_noconv=False)
+        got.append((r, jv.numpy(), grad.diagonal().numpy(), rep["linear_iterations"]))
+    for a, b in zip(*got):
+        assert np.isfinite(a).all() and np.abs(a - b).max() <= 1e-14 * np.abs(b).max()
