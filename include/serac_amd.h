@@ -240,9 +240,11 @@ int sx_form_eval(sx_form* f, double t, const double* const* inputs, double* out,
 /* Form options (no reference counterpart: the reference runs serially).
  *   SX_OPT_SCATTER: SX_SCATTER_COLORED (default) gives bitwise reproducible
  *     results: the element kernel stores its values and a second kernel adds
- *     them per node in element order (the form keeps up to 192 MB of element
- *     values), or, on larger meshes, one kernel per element colour adds with
- *     plain read-modify-writes.  SX_SCATTER_ATOMIC adds with FP64 atomics:
+ *     them per node (the form keeps up to 192 MB of element values), or, on
+ *     larger meshes, where that memory is not there and for domains that list
+ *     an element twice, one kernel per element colour adds with plain
+ *     read-modify-writes.  Both add a node's values in the order of its
+ *     elements' colours: the bits do not depend on which one runs.  SX_SCATTER_ATOMIC adds with FP64 atomics:
  *     one pass, last-bit rounding depends on the order the hardware applies
  *     them.
  *     Must be set before the first AddDomainIntegral.

@@ -194,10 +194,12 @@ struct sx_space {
   int              ncolors = 0;
   DeviceBuffer     d_emap;  // element order (E-vector gather)
   DeviceBuffer     d_offs, d_ents;  // node -> (e*npe + j), increasing e
-  // DOF-level sparsity of forms on this space, on the device (built on first
-  // assembly; the matrices share it)
+  // Built when first needed, under lazy_mu: the DOF-level sparsity of forms on
+  // this space, on the device (the matrices share it), and d_ents with each
+  // node's entries in the order of their elements' colours (the node sum's)
   std::shared_ptr<const struct CsrPattern> csr;
-  std::mutex                               csr_mu;
+  DeviceBuffer                             d_ents_by_color;
+  std::mutex                               lazy_mu;
   // numbering: native = the library's own (lexicographic node grid on cuboid
   // meshes); otherwise node_of_own[own node] = the caller's node id
   bool                 native = true;
@@ -448,14 +450,15 @@ sxk::ElemLaunch base_launch(const sx_form* f, const Integral& I, int mode)
 // number of event pairs recorded.
 //
 // The reproducible scatter stores every element's values and sums them per
-// node in element order, two launches in all, where one launch per element
-// colour (8 on cuboids, 17 on a shuffled numbering) pays a launch and a partly
+// node, two launches in all, where one launch per element colour (8 on cuboids, 17 on a shuffled numbering) pays a launch and a partly
 // filled GPU each time.  Before -> after: a Jacobi-CG iteration p = 2 on 16x5x4
 // elements 60 -> 25 us, Neo-Hookean residual p = 2 on 57x48x43 214 -> 180 us,
 // FP64 J.v p = 3 on 40^3 364 -> 306 us, with a BF16 tangent 174 -> 125 us.
 // Colours remain for domains that list an element twice (a range per repetition
 // and colour) and for values beyond kNodeSumBytes (J.v p = 3 on 64^3, 403 MB:
-// 1.35 ms with colours, 1.39 with the sum; BF16 tangent 0.52 and 0.54).
+// 1.35 ms with colours, 1.39 with the sum; BF16 tangent 0.52 and 0.54).  Both
+// add a node's values in the same order, so results have the same bits whichever
+// runs.
 int run_slots(const sx_form* f_, const Integral& I, sxk::ElemLaunch& P, void* r, bool set, hipEvent_t* ev)
 {
   sx_form*   f = const_cast<sx_form*>(f_);
@@ -482,7 +485,7 @@ int run_slots(const sx_form* f_, const Integral& I, sxk::ElemLaunch& P, void* r,
     P.E                           = f->E.ptr;
     P.slot_begin                  = 0;
     P.slot_end                    = I.nslots;
-    const DeviceBuffer &offs = I.own_lists ? I.d_noffs : s->d_offs, &ents = I.own_lists ? I.d_nents : s->d_ents;
+    const DeviceBuffer &offs = I.own_lists ? I.d_noffs : s->d_offs, &ents = I.own_lists ? I.d_nents : s->d_ents_by_color;
     const bool          all  = I.d_nodes.ptr == nullptr;
     if (set && !all) fill();
     if (ev) SX_HIP(hipEventRecord(ev[0], f->stream));
@@ -529,7 +532,7 @@ int run_integral(const sx_form* f, const Integral& I, int mode, const void* u, v
 // assembly (Neo-Hookean p = 2, 14x12x13 elements, 11 M entries).
 std::shared_ptr<const CsrPattern> csr_pattern(sx_space* s)
 {
-  std::lock_guard<std::mutex> lk(s->csr_mu);
+  std::lock_guard<std::mutex> lk(s->lazy_mu);
   if (s->csr) return s->csr;
   const int64_t nn = s->nnodes, npe = s->npe, ne = int64_t(s->emap.size()) / npe;
   const int     nc = s->nc;
@@ -1400,10 +1403,11 @@ std::vector<int> by_color(const sx_space* s, const std::vector<int>& domain, std
 constexpr size_t kNodeSumBytes = size_t(192) << 20;
 
 // The node sum's lists over `domain`: the nodes of its elements, ascending, and
-// each one's places in the element values.  A sum over the whole mesh visits
-// every node and entry, which on a part of it costs more than the part (J.v on
-// one of 48 layers, p = 3: 74 us with the whole mesh's lists, 49 with colours,
-// 33 with the layer's own; sixteen integrals over three layers each 1547, 1441, 650).
+// each one's places in the element values, in the order of the colour launches.
+// A sum over the whole mesh visits every node and entry, which on a part of it
+// costs more than the part (J.v on one of 48 layers, p = 3: 74 us with the whole
+// mesh's lists, 49 with colours, 33 with the layer's own; sixteen integrals over
+// three layers each 1547, 1441, 650).
 void node_lists(const sx_space* s, Integral& I, const std::vector<int>& domain)
 {
   const size_t         npe = size_t(s->npe);
@@ -1430,14 +1434,45 @@ void node_lists(const sx_space* s, Integral& I, const std::vector<int>& domain)
   for (size_t t = 0; t < nodes.size(); t++) offs[t + 1] += offs[t];
   std::vector<int32_t> ents(domain.size() * npe);
   std::vector<int64_t> next(offs.begin(), offs.end() - 1);
-  for (size_t i = 0; i < domain.size(); i++)
+  std::vector<int64_t> launches;
+  for (int i : by_color(s, domain, launches))
     for (size_t j = 0; j < npe; j++)
-      ents[size_t(next[size_t(at[size_t(s->emap[size_t(domain[i]) * npe + j])])]++)] = int32_t(i * npe + j);
+      ents[size_t(next[size_t(at[size_t(s->emap[size_t(domain[size_t(i)]) * npe + j])])]++)] = int32_t(size_t(i) * npe + j);
   I.nsum = int64_t(nodes.size());
   if (I.nsum < s->nnodes) I.d_nodes.upload(nodes);
   I.d_noffs.upload(offs);
   I.d_nents.upload(ents);
   I.own_lists = true;
+}
+
+// Device memory, or false where there is not enough (what was there stays).
+bool try_allocate(DeviceBuffer& b, size_t bytes)
+{
+  void* p = nullptr;
+  if (hipMalloc(&p, bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  b.release();
+  b.ptr   = p;
+  b.bytes = bytes;
+  return true;
+}
+
+// The entries of all the space's nodes in the order of the colour launches.
+bool entries_by_color(sx_space* s)
+{
+  std::lock_guard<std::mutex> lk(s->lazy_mu);
+  if (s->d_ents_by_color.ptr) return true;
+  DeviceBuffer out, color;
+  if (!try_allocate(out, s->d_ents.bytes) || !try_allocate(color, s->color.size() * sizeof(int))) return false;
+  color.upload(s->color);
+  SX_HIP(sxk::entries_by_color(s->d_offs.as<const int64_t>(), s->d_ents.as<const int32_t>(), color.as<const int32_t>(),
+                               s->npe, s->nnodes, out.as<int32_t>(), nullptr));
+  SX_HIP(hipStreamSynchronize(nullptr));
+  std::swap(s->d_ents_by_color.ptr, out.ptr);
+  std::swap(s->d_ents_by_color.bytes, out.bytes);
+  return true;
 }
 
 // Memory and lists for the node sum of an integral over `domain`; false where
@@ -1457,18 +1492,14 @@ bool prepare_node_sum(sx_form* f, Integral& I, const std::vector<int>& domain)
     whole                   = whole && domain[i] == int(i);
   }
   if (f->E.bytes < bytes) {
-    void* p = nullptr;
     SX_HIP(hipStreamSynchronize(f->stream));
-    if (hipMalloc(&p, bytes) != hipSuccess) {
-      (void)hipGetLastError();
-      return false;
-    }
-    f->E.release();
-    f->E.ptr   = p;
-    f->E.bytes = bytes;
+    if (!try_allocate(f->E, bytes)) return false;
   }
   I.nsum = vs->nnodes;
-  if (!whole) node_lists(vs, I, domain);
+  if (!whole)
+    node_lists(vs, I, domain);
+  else if (!entries_by_color(const_cast<sx_space*>(vs)))
+    return false;
   I.elems = domain;
   return true;
 }

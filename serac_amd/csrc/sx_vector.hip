@@ -627,12 +627,18 @@ __global__ void __launch_bounds__(kThreads) k_node_sum(const int32_t* nodes, con
   V*             out  = r + (vdim ? node * NC + c : c * nnodes + node);
   V              acc  = add ? *out : V(0);
   for (; k < k1; k += 4) {
+    int at[4];  // the entry's value, -1: no entry
+#pragma unroll
+    for (int m = 0; m < 4; m++) {
+      at[m] = -1;
+      if (k + m < k1) at[m] = ents[k + m] * NC + int(c);
+    }
     T v[4];
 #pragma unroll
-    for (int m = 0; m < 4; m++) v[m] = k + m < k1 ? E[ents[k + m] * NC + int(c)] : T(0);
+    for (int m = 0; m < 4; m++) v[m] = at[m] >= 0 ? E[at[m]] : T(0);
 #pragma unroll
     for (int m = 0; m < 4; m++)
-      if (k + m < k1) acc += V(v[m]);
+      if (at[m] >= 0) acc += V(v[m]);
   }
   if (halt == 0.0) *out = acc;
 }
@@ -650,6 +656,22 @@ hipError_t launch_node_sum(const int32_t* nodes, const int64_t* offs, const int3
   else
     hipLaunchKernelGGL((k_node_sum<T, V, 3>), g, b, 0, s, nodes, offs, ents, e, o, n, nnodes, ordering, add, stop);
   return hipGetLastError();
+}
+
+// the entries of each node sorted by their elements' colour (equal colours keep their order)
+__global__ void __launch_bounds__(kThreads) k_entries_by_color(const int64_t* offs, const int32_t* ents,
+                                                                const int32_t* color, int npe, int64_t nnodes,
+                                                                int32_t* out)
+{
+  const int64_t v = int64_t(blockIdx.x) * kThreads + threadIdx.x;
+  if (v >= nnodes) return;
+  const int64_t k0 = offs[v], k1 = offs[v + 1];
+  for (int64_t k = k0; k < k1; k++) {
+    const int32_t ej = ents[k], c = color[ej / npe];
+    int64_t       at = k;
+    for (; at > k0 && color[out[at - 1] / npe] > c; at--) out[at] = out[at - 1];
+    out[at] = ej;
+  }
 }
 
 __global__ void __launch_bounds__(kThreads) k_e_transpose(const double* in, double* out, int64_t ne, int nc, int npe,
@@ -685,6 +707,15 @@ hipError_t node_sum(const int32_t* nodes, const int64_t* offs, const int32_t* en
   if (r_f32) return launch_node_sum<float, float>(nodes, offs, ents, E, r, m, nn, nc, ordering, int(add), stop, s);
   if (e_f32) return launch_node_sum<float, double>(nodes, offs, ents, E, r, m, nn, nc, ordering, int(add), stop, s);
   return launch_node_sum<double, double>(nodes, offs, ents, E, r, m, nn, nc, ordering, int(add), stop, s);
+}
+
+hipError_t entries_by_color(const int64_t* offs, const int32_t* ents, const int32_t* color, int npe, int64_t nnodes,
+                            int32_t* out, hipStream_t s)
+{
+  if (nnodes <= 0) return hipSuccess;
+  hipLaunchKernelGGL(k_entries_by_color, dim3(unsigned((nnodes + kThreads - 1) / kThreads)), dim3(kThreads), 0, s, offs,
+                     ents, color, npe, nnodes, out);
+  return hipGetLastError();
 }
 
 hipError_t csr_spmv(const int64_t* rp, const int32_t* col, const double* val, const double* x, double* y,

@@ -86,6 +86,11 @@ hipError_t scatter_e(const int64_t* offs, const int32_t* ents, const double* E, 
 hipError_t node_sum(const int32_t* nodes, const int64_t* offs, const int32_t* ents, int64_t n, const void* E,
                     bool e_f32, void* r, bool r_f32, int64_t nnodes, int nc, int ordering, bool add,
                     const double* stop, hipStream_t s);
+// out = ents (node -> e * npe + j) with each node's sorted by color[e] (equal
+// colours keep their order)
+hipError_t entries_by_color(const int64_t* offs, const int32_t* ents, const int32_t* color, int npe, int64_t nnodes,
+                            int32_t* out, hipStream_t s);
+
 // E-vector layouts: dir 0 copies the reference layout [e][c][j] into the
 // component-major [c][e][j], dir 1 back
 hipError_t e_transpose(const double* in, double* out, int64_t ne, int nc, int npe, int dir, hipStream_t s);

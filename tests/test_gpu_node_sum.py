@@ -112,3 +112,19 @@ def test_lists_of_a_part(gpu_lib, which, ordering):
         got.append((r, jv.numpy(), grad.diagonal().numpy(), rep["linear_iterations"]))
     for a, b in zip(*got):
         assert np.isfinite(a).all() and np.abs(a - b).max() <= 1e-14 * np.abs(b).max()
+
+
+@pytest.mark.parametrize("nz", [67, 68])
+def test_at_the_limit_of_the_element_values(gpu_lib, nz):
+    """Meshes just below and just above 192 MB of element values: the sum, and the colours that large meshes take."""
+    space = sx.Space(sx.Mesh.cuboid(68, 68, nz), 2, 3)
+    assert (space.ne * space.npe * 3 * 8 <= 192 << 20) == (nz == 67)
+    U = sx.DeviceVector.from_numpy(W.nodal_field(space.nnodes, 3, 3, 2000, -1e-4, 1e-4))
+    v = sx.DeviceVector.from_numpy(W.nodal_field(space.nnodes, 3, 4, 3000, -1.0, 1.0))
+    got = []
+    for scatter in (capi.SX_SCATTER_COLORED, capi.SX_SCATTER_ATOMIC):
+        f = form_on(space, scatter, [None])
+        r, grad = f(0.0, U, wrt=0)
+        got.append((r.numpy(), grad(v).numpy(), grad.diagonal().numpy()))
+    for a, b in zip(*got):
+        assert np.abs(a - b).max() <= 1e-14 * np.abs(b).max()

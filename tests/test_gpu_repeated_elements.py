@@ -1,8 +1,8 @@
 """Domains that list elements more than once: every listing counts.  They run
 one launch per element colour and listing with plain read-modify-writes (as
-large meshes do per colour), and have to equal a form whose integrals list an
-element once each: sums of the same element values, at most 8 elements by 3
-listings at a node, in another order (24 roundings; FP32 vectors add in FP32).
+large meshes do per colour), and have to equal, bit for bit, a form whose
+integrals list an element once each, which take the node sum: both add a
+node's values colour by colour, listing by listing.
 Cuboids with their 8 colours and meshes from arrays with greedy ones, every
 order, precision and scatter order, the assembly, the shape gradient, and
 plastic state against the oracle."""
@@ -79,9 +79,8 @@ def test_every_listing_counts(gpu_lib, kind, p, material):
             got = results(space, material, [repeated], tangent, arithmetic, dtype, order)
             want = results(space, material, once, tangent, arithmetic, dtype, order)
             for k, b in want.items():
-                tol = 24 * 6e-8 if got[k].dtype == np.float32 else 24 * 1.2e-16
-                assert np.isfinite(got[k]).all() and np.abs(b).max() > 0, k
-                assert np.abs(got[k] - b).max() <= tol * np.abs(b).max(), (k, tangent, arithmetic, dtype)
+                assert np.isfinite(b).all() and np.abs(b).max() > 0, k
+                assert np.array_equal(got[k], b), (k, tangent, arithmetic, dtype, order)
 
 
 @pytest.mark.parametrize("p", [1, 2])
