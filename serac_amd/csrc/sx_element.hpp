@@ -571,12 +571,13 @@ __device__ __forceinline__ void write_row(T* a, const T* v)
 // residual (MODE_RESIDUAL) and linearization (MODE_LINEARIZE, tangent in S)
 // ---------------------------------------------------------------------------
 // Waves per SIMD the register allocation aims at: the J2 linearization would
-// take 278 registers (one wave); held to two waves it spills nothing.
+// take 278 registers (one wave); held to two waves it spills nothing.  A vector
+// residual spills 6 to 9 at five waves, 20 where it also carries the value.
 template <int NC, int MODE, class QF>
 constexpr int element_waves()
 {
   if (QF::STATE > 0) return MODE == MODE_LINEARIZE ? 2 : 3;
-  return NC == 1 || MODE != MODE_RESIDUAL ? 4 : 5;
+  return NC == 1 || MODE != MODE_RESIDUAL || QF::USES_VALUE ? 4 : 5;
 }
 
 template <int N, int NC, int MODE, class QF, int LAYOUT, typename S>
@@ -590,7 +591,9 @@ __global__ void __launch_bounds__(256, (element_waves<NC, MODE, QF>())) k_elemen
   constexpr int  DS      = Shape::DS;
   constexpr int  NST     = QF::STATE;
   constexpr int  R       = NC * NQ;  // one LDS region
-  constexpr int  PER     = (3 + (HAS_SRC || QF::USES_VALUE ? 1 : 0)) * R;
+  constexpr int  REGIONS = 3 + (HAS_SRC || QF::USES_VALUE ? 1 : 0);
+  // elements of a wave (eight at p = 1) start in different LDS banks
+  constexpr int  PER     = REGIONS * R + (REGIONS * R % 32 == 0 ? 8 : 0);
   using Lay              = TangentLayout<S, DS, NQ>;
 
   __shared__ double smem[EB * PER];

@@ -57,7 +57,7 @@ def test_mixed_operator_against_oracle(gpu_lib, tprec, tol, scatter):
 # p = 2 starts from the loaded face, moved so little (0.2 %) that its tangent
 # stays definite.  From 2 % the mixed solve broke down for 7, 11 and 18 of 24
 # displacements one last bit apart, with three orders of adding a node's element
-# values (FP64: none); from 0.2 % none of 192 did, in 1047 to 1100 CG iterations.
+# values (FP64: none); from 0.2 % none of 96 did, in 1047 to 1100 CG iterations.
 @pytest.mark.parametrize("tprec", [sx.capi.SX_PREC_F32])
 @pytest.mark.parametrize("p", [2, 4])
 def test_mixed_newton_reaches_fp64_solution(gpu_lib, tprec, p):
