@@ -459,7 +459,13 @@ struct TangentRegs<T, bf16, DS, NQ> {
 };
 
 // Stores tangent entry k (FP64 value) of quadrature point q: entries arrive in
-// increasing k; whole 16-byte groups are stored at once from `pend`.
+// increasing k; whole 16-byte groups are stored at once from `pend`.  The stores
+// bypass the caches, except where a long tangent (78 entries) meets groups that
+// fill no whole cache lines (p = 2, 4).  Bypassing and not, mass-diffusion of
+// three components: FP64 p = 2 on 48x47x49 elements 718 and 507 us, p = 4 on
+// 28x27x29 445 and 416; FP32 p = 2 339 and 270, but p = 4 229 and 254; BF16
+// p = 2 164 and 219.  Shorter tangents: Neo-Hookean p = 3 on 36x35x37 244 and
+// 328, p = 2 328 and 355.
 template <typename S, int DS, int NQ>
 __device__ __forceinline__ void store_tangent_entry(void* base, int q, int k, double v,
                                                     typename StoreTraits<S>::raw* pend)
@@ -467,16 +473,22 @@ __device__ __forceinline__ void store_tangent_entry(void* base, int q, int k, do
   using L   = TangentLayout<S, DS, NQ>;
   using raw = typename StoreTraits<S>::raw;
   raw* Dp   = static_cast<raw*>(base);
+  auto put  = [](auto x, auto* at) {
+    if constexpr (DS == 78 && ((sizeof(S) == 8 && NQ % 2 == 1) || (sizeof(S) == 4 && NQ == 27)))
+      *at = x;
+    else
+      __builtin_nontemporal_store(x, at);
+  };
   if (k < L::G * L::VEC) {
     pend[k % L::VEC] = raw(to_store(v, static_cast<S*>(nullptr)));
     if (k % L::VEC == L::VEC - 1) {
       typedef unsigned int u4 __attribute__((ext_vector_type(4)));
       u4 w;
       __builtin_memcpy(&w, pend, 16);
-      __builtin_nontemporal_store(w, reinterpret_cast<u4*>(Dp + (k / L::VEC) * L::VEC * NQ + q * L::VEC));
+      put(w, reinterpret_cast<u4*>(Dp + (k / L::VEC) * L::VEC * NQ + q * L::VEC));
     }
   } else {
-    __builtin_nontemporal_store(raw(to_store(v, static_cast<S*>(nullptr))), Dp + L::offset(k, q));
+    put(raw(to_store(v, static_cast<S*>(nullptr))), Dp + L::offset(k, q));
   }
 }
 
@@ -570,18 +582,35 @@ __device__ __forceinline__ void write_row(T* a, const T* v)
 // ---------------------------------------------------------------------------
 // residual (MODE_RESIDUAL) and linearization (MODE_LINEARIZE, tangent in S)
 // ---------------------------------------------------------------------------
-// Waves per SIMD the register allocation aims at: the J2 linearization would
-// take 278 registers (one wave); held to two waves it spills nothing.  A vector
-// residual spills 6 to 9 at five waves, 20 where it also carries the value.
-template <int NC, int MODE, class QF>
-constexpr int element_waves()
+// Waves per SIMD that the register allocation aims at, and the most of them.
+// The J2 linearization would take 278 registers (one wave); held to two waves it
+// spills nothing.  A vector residual spills 6 to 9 at five waves, 20 where it
+// also carries the value.  The linearization of a constant tangent does little
+// but store it, and at p = 1, 2, where an element's groups are short, it stores
+// faster with fewer waves in flight: linear elasticity p = 1 on 80x79x81
+// elements 358 us of kernel time at four waves, 300 at two; p = 2 on 48x47x49
+// 320 and, at three, 305; mass-diffusion p = 2 490 and 425.  At p = 3, 4 four
+// waves are faster (p = 3 on 36x35x37 elastic 200 us against 235).
+template <int N, int NC, int MODE, class QF, typename S>
+constexpr int element_max_waves()
 {
+  if (MODE == MODE_LINEARIZE && NC == 3 && N <= 3 && QF::CONSTANT_TANGENT) return N;
+  return 8;
+}
+template <int N, int NC, int MODE, class QF, typename S>
+constexpr int element_min_waves()
+{
+  constexpr int most = element_max_waves<N, NC, MODE, QF, S>();
+  if (most < 8) return most;
   if (QF::STATE > 0) return MODE == MODE_LINEARIZE ? 2 : 3;
   return NC == 1 || MODE != MODE_RESIDUAL || QF::USES_VALUE ? 4 : 5;
 }
 
 template <int N, int NC, int MODE, class QF, int LAYOUT, typename S>
-__global__ void __launch_bounds__(256, (element_waves<NC, MODE, QF>())) k_element(const ElemLaunch P)
+__global__ void __launch_bounds__(256)
+    __attribute__((amdgpu_waves_per_eu((element_min_waves<N, NC, MODE, QF, S>()),
+                                       (element_max_waves<N, NC, MODE, QF, S>()))))
+    k_element(const ElemLaunch P)
 {
   constexpr int  NQ      = N * N * N;
   constexpr int  NN      = N * N;

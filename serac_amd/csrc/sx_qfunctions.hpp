@@ -130,7 +130,9 @@ __device__ __forceinline__ void gram(const double* Ji, double f, double* M)
 // dual per column, 9 (12) times the work of the values, and made the
 // linearization compute-bound (Neo-Hookean p = 3 on 48x40x44 elements: 1196
 // us of kernel time with the passes, 505 with the closed form, 330 for the
-// tangent's bytes alone; J2 p = 2 on 56x48x50: 1463, 672 and 400).  HAS_SOURCE: the source output is nonzero; USES_VALUE: the
+// tangent's bytes alone; J2 p = 2 on 56x48x50: 1463, 672 and 400).
+// CONSTANT_TANGENT: it does not depend on the field.
+// HAS_SOURCE: the source output is nonzero; USES_VALUE: the
 // outputs depend on the field value (not only its gradient); SYMMETRIC: the
 // tangent is major-symmetric, so half of it is stored.
 // ---------------------------------------------------------------------------
@@ -143,6 +145,7 @@ struct QFHeat {
   static constexpr bool HAS_SOURCE = true;
   static constexpr bool USES_VALUE = false;
   static constexpr int  STATE      = 0;
+  static constexpr bool CONSTANT_TANGENT = true;
   template <typename T>
   __device__ __forceinline__ static void eval(const double* p, const T*, const T* g, T* src, T* flux)
   {
@@ -171,6 +174,7 @@ struct QFMassDiffusion {
   static constexpr bool HAS_SOURCE = true;
   static constexpr bool USES_VALUE = true;
   static constexpr int  STATE      = 0;
+  static constexpr bool CONSTANT_TANGENT = true;
   template <typename T>
   __device__ __forceinline__ static void eval(const double* p, const T* v, const T* g, T* src, T* flux)
   {
@@ -209,6 +213,7 @@ struct QFNeoHookean {
   static constexpr bool HAS_SOURCE = false;
   static constexpr bool USES_VALUE = false;
   static constexpr int  STATE      = 0;
+  static constexpr bool CONSTANT_TANGENT = false;
   template <typename T>
   __device__ __forceinline__ static void eval(const double* p, const T*, const T* H, T*, T* flux)
   {
@@ -281,6 +286,7 @@ struct QFQoiValue {
   static constexpr bool HAS_SOURCE = true;
   static constexpr bool USES_VALUE = false;
   static constexpr int  STATE      = 0;
+  static constexpr bool CONSTANT_TANGENT = true;
   template <typename T>
   __device__ __forceinline__ static void eval(const double* p, const T*, const T*, T* src, T* flux)
   {
@@ -300,6 +306,7 @@ struct QFLinearElastic {
   static constexpr bool HAS_SOURCE = false;
   static constexpr bool USES_VALUE = false;
   static constexpr int  STATE      = 0;
+  static constexpr bool CONSTANT_TANGENT = true;
   template <typename T>
   __device__ __forceinline__ static void eval(const double* p, const T*, const T* g, T*, T* flux)
   {
@@ -366,6 +373,7 @@ struct QFJ2 {
   static constexpr bool   HAS_SOURCE = false;
   static constexpr bool   USES_VALUE = false;
   static constexpr int    STATE      = 10;
+  static constexpr bool CONSTANT_TANGENT = false;
   static constexpr double TOL        = 1e-10;
 
   __device__ __forceinline__ static double solve(double q, double a, double sy, double Hi, double e0, double hi,
