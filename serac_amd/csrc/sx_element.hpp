@@ -504,6 +504,9 @@ __device__ __forceinline__ void store_tangent_entry(void* base, int q, int k, do
 // value reads and N table reads through the one LDS port of a CU.  Neo-Hookean
 // residual p = 2 on 57x48x43: 148 -> 120 us of kernel time; p = 3 on 64^3: 735
 // -> 682, two thirds of which FP64 instructions take (about 680 a point).
+// One component has N * N rows for N^3 lanes and stays with a lane per result
+// (use_rows): heat residual p = 3 on 36x35x37 elements 84 us by rows and 67 so,
+// p = 1 on 80x79x81 91 and 73 (both with the fill of the output).
 template <int N, int NC>
 struct Rows {
   static constexpr int NQ = N * N * N, COUNT = NC * N * N, ITER = (COUNT + NQ - 1) / NQ;
@@ -578,6 +581,22 @@ __device__ __forceinline__ void write_row(T* a, const T* v)
 #pragma unroll
   for (int i = 0; i < N; i++) a[i * STRIDE] = v[i];
 }
+template <int NC>
+constexpr bool use_rows()
+{
+  return NC > 1;
+}
+
+// A lane per result: sum_i tab[i * TS] a[i * AS], N table entries and N values
+// from LDS
+template <int N, int TS, int AS, typename T>
+__device__ __forceinline__ T dot_result(const T* tab, const T* a)
+{
+  T s = T(0);
+#pragma unroll
+  for (int i = 0; i < N; i++) s += tab[i * TS] * a[i * AS];
+  return s;
+}
 
 // ---------------------------------------------------------------------------
 // residual (MODE_RESIDUAL) and linearization (MODE_LINEARIZE, tangent in S)
@@ -603,7 +622,8 @@ constexpr int element_min_waves()
   constexpr int most = element_max_waves<N, NC, MODE, QF, S>();
   if (most < 8) return most;
   if (QF::STATE > 0) return MODE == MODE_LINEARIZE ? 2 : 3;
-  return NC == 1 || MODE != MODE_RESIDUAL || QF::USES_VALUE ? 4 : 5;
+  if (NC == 1) return MODE == MODE_LINEARIZE && sizeof(S) == 2 ? 4 : 7;
+  return MODE != MODE_RESIDUAL || QF::USES_VALUE ? 4 : 5;
 }
 
 template <int N, int NC, int MODE, class QF, int LAYOUT, typename S>
@@ -619,14 +639,16 @@ __global__ void __launch_bounds__(256)
   constexpr bool HAS_SRC = QF::HAS_SOURCE;
   constexpr int  DS      = Shape::DS;
   constexpr int  NST     = QF::STATE;
+  constexpr bool ROWS    = use_rows<NC>();
   constexpr int  R       = NC * NQ;  // one LDS region
-  constexpr int  REGIONS = 3 + (HAS_SRC || QF::USES_VALUE ? 1 : 0);
+  constexpr int  REGIONS = ROWS ? 3 + (HAS_SRC || QF::USES_VALUE ? 1 : 0) : 6 + (HAS_SRC ? 1 : 0);
   // elements of a wave (eight at p = 1) start in different LDS banks
   constexpr int  PER     = REGIONS * R + (REGIONS * R % 32 == 0 ? 8 : 0);
   using Lay              = TangentLayout<S, DS, NQ>;
 
   __shared__ double smem[EB * PER];
-  __shared__ double sxw[2 * N];  // Gauss points and weights
+  __shared__ double stab[ROWS ? 1 : 4 * NN];  // B, G, and both times the weights
+  __shared__ double sxw[2 * N];               // Gauss points and weights
   __shared__ double sxv[EB * 24];
   __shared__ int    snode[EB * NQ];
 
@@ -642,6 +664,8 @@ __global__ void __launch_bounds__(256)
   double *      S1 = S0 + R, *S2 = S0 + 2 * R, *S3 = S0 + 3 * R;  // S3 only where PER has it
   double*       r = static_cast<double*>(P.r);
 
+  if constexpr (!ROWS)
+    for (int k = tid; k < 4 * NN; k += blockDim.x) stab[k] = P.tables[k];
   if (tid < 2 * N) sxw[tid] = P.tables[4 * NN + tid];
   const ScalarTable tB = (ScalarTable)(uintptr_t)P.tables;
   const ScalarTable tG = tB + NN;
@@ -656,75 +680,109 @@ __global__ void __launch_bounds__(256)
       for (int k = 0; k < NST; k++) st[k] = stp[k * NQ];
     }
   }
-  int64_t node = 0;
-  if (active) {
-    node = P.map[size_t(slot) * NQ + li];
+  int64_t node = active ? P.map[size_t(slot) * NQ + li] : 0;
+  double  nodal[NC];  // this lane's node
+  auto    gather = [&](const double* field) {
+    if (active) {
+#pragma unroll
+      for (int c = 0; c < NC; c++) nodal[c] = field[lidx(node, c, NC, P.nnodes, P.ordering)];
+    }
+  };
+  gather(static_cast<const double*>(P.u));
+  if (active)
     for (int k = li; k < 24; k += NQ) sxv[el * 24 + k] = P.coords[size_t(slot) * 24 + k];
-  }
 
-  // Parent gradient (and value) at this lane's point of a field on the
-  // element's nodes: gather, then x, y and z in turn.  Every lane calls it; the
-  // regions are free again after it.
-  auto interpolate = [&](const double* field, double* val, double* gp) {
+  // Parent gradient (and value) at this lane's point of the gathered field:
+  // x, y and z in turn.  Every lane calls it; the regions (with a lane per
+  // result, the first three) are free again after it.
+  auto interpolate = [&](double* val, double* gp) {
     if (active) {
 #pragma unroll
-      for (int c = 0; c < NC; c++) S0[c * NQ + li] = field[lidx(node, c, NC, P.nnodes, P.ordering)];
+      for (int c = 0; c < NC; c++) S0[c * NQ + li] = nodal[c];
     }
     lds_barrier();
-    for_rows<N, NC, 0>(li, active, [&](int o) {  // u -> B u, G u
-      double v[N], a[N], b[N];
-      read_row<N, 1>(S0 + o, v);
-      row_forward<N>(tB, v, a);
-      row_forward<N>(tG, v, b);
-      write_row<N, 1>(S0 + o, a);
-      write_row<N, 1>(S1 + o, b);
-    });
-    lds_barrier();
-    for_rows<N, NC, 1>(li, active, [&](int o) {  // -> BB, BG (y, x), GB
-      double v[N], w[N], a[N];
-      read_row<N, N>(S0 + o, v);
-      read_row<N, N>(S1 + o, w);
-      row_forward<N>(tB, v, a);
-      write_row<N, N>(S0 + o, a);
-      row_forward<N>(tB, w, a);
-      write_row<N, N>(S1 + o, a);
-      row_forward<N>(tG, v, a);
-      write_row<N, N>(S2 + o, a);
-    });
-    lds_barrier();
-    for_rows<N, NC, 2>(li, active, [&](int o) {  // -> d/dx in S1, d/dy in S2, d/dz in S0, value in S3
-      double v[N], a[N];
-      read_row<N, NN>(S1 + o, v);
-      row_forward<N>(tB, v, a);
-      write_row<N, NN>(S1 + o, a);
-      read_row<N, NN>(S2 + o, v);
-      row_forward<N>(tB, v, a);
-      write_row<N, NN>(S2 + o, a);
-      read_row<N, NN>(S0 + o, v);
-      row_forward<N>(tG, v, a);
-      write_row<N, NN>(S0 + o, a);
-      if constexpr (QF::USES_VALUE) {
+    if constexpr (!ROWS) {
+      const int     oy = i2 * NN + i0, oz = i1 * N + i0;  // first entries of the lane's lines along y and z
+      const double *sB = stab, *sG = stab + NN;
+      // (results first, stores after: a line and a table row are then read once)
+      if (active) {
+        const double b = dot_result<N, 1, 1>(sB + i0 * N, S0 + li - i0);
+        const double g = dot_result<N, 1, 1>(sG + i0 * N, S0 + li - i0);
+        S1[li]         = b;
+        S2[li]         = g;
+      }
+      lds_barrier();
+      if (active) {
+        const double bb = dot_result<N, 1, N>(sB + i1 * N, S1 + oy);
+        const double bg = dot_result<N, 1, N>(sB + i1 * N, S2 + oy);
+        const double gb = dot_result<N, 1, N>(sG + i1 * N, S1 + oy);
+        S3[li]          = bb;
+        S3[NQ + li]     = bg;
+        S3[2 * NQ + li] = gb;
+      }
+      lds_barrier();
+      if (active) {
+        gp[0] = dot_result<N, 1, NN>(sB + i2 * N, S3 + NQ + oz);
+        gp[1] = dot_result<N, 1, NN>(sB + i2 * N, S3 + 2 * NQ + oz);
+        gp[2] = dot_result<N, 1, NN>(sG + i2 * N, S3 + oz);
+        if constexpr (QF::USES_VALUE) val[0] = dot_result<N, 1, NN>(sB + i2 * N, S3 + oz);
+      }
+    } else {
+      for_rows<N, NC, 0>(li, active, [&](int o) {  // u -> B u, G u
+        double v[N], a[N], b[N];
+        read_row<N, 1>(S0 + o, v);
         row_forward<N>(tB, v, a);
-        write_row<N, NN>(S3 + o, a);
-      }
-    });
-    lds_barrier();
-    if (active) {
+        row_forward<N>(tG, v, b);
+        write_row<N, 1>(S0 + o, a);
+        write_row<N, 1>(S1 + o, b);
+      });
+      lds_barrier();
+      for_rows<N, NC, 1>(li, active, [&](int o) {  // -> BB, BG (y, x), GB
+        double v[N], w[N], a[N];
+        read_row<N, N>(S0 + o, v);
+        read_row<N, N>(S1 + o, w);
+        row_forward<N>(tB, v, a);
+        write_row<N, N>(S0 + o, a);
+        row_forward<N>(tB, w, a);
+        write_row<N, N>(S1 + o, a);
+        row_forward<N>(tG, v, a);
+        write_row<N, N>(S2 + o, a);
+      });
+      lds_barrier();
+      for_rows<N, NC, 2>(li, active, [&](int o) {  // -> d/dx in S1, d/dy in S2, d/dz in S0, value in S3
+        double v[N], a[N];
+        read_row<N, NN>(S1 + o, v);
+        row_forward<N>(tB, v, a);
+        write_row<N, NN>(S1 + o, a);
+        read_row<N, NN>(S2 + o, v);
+        row_forward<N>(tB, v, a);
+        write_row<N, NN>(S2 + o, a);
+        read_row<N, NN>(S0 + o, v);
+        row_forward<N>(tG, v, a);
+        write_row<N, NN>(S0 + o, a);
+        if constexpr (QF::USES_VALUE) {
+          row_forward<N>(tB, v, a);
+          write_row<N, NN>(S3 + o, a);
+        }
+      });
+      lds_barrier();
+      if (active) {
 #pragma unroll
-      for (int c = 0; c < NC; c++) {
-        gp[c * 3 + 0] = S1[c * NQ + li];
-        gp[c * 3 + 1] = S2[c * NQ + li];
-        gp[c * 3 + 2] = S0[c * NQ + li];
-        if constexpr (QF::USES_VALUE) val[c] = S3[c * NQ + li];
+        for (int c = 0; c < NC; c++) {
+          gp[c * 3 + 0] = S1[c * NQ + li];
+          gp[c * 3 + 1] = S2[c * NQ + li];
+          gp[c * 3 + 2] = S0[c * NQ + li];
+          if constexpr (QF::USES_VALUE) val[c] = S3[c * NQ + li];
+        }
       }
+      lds_barrier();
     }
-    lds_barrier();
   };
 
   double val[NC], gp[3 * NC];
 #pragma unroll
   for (int c = 0; c < NC; c++) val[c] = 0.0;
-  interpolate(static_cast<const double*>(P.u), val, gp);
+  interpolate(val, gp);
   // ---- shape displacement (ShapeAwareFunctional, fn/shape_aware_functional.hpp:37-50):
   // the parent gradient of p at this lane's quadrature point, added to the
   // geometric Jacobian below, so dx/dxi = dX/dxi + dp/dxi = (I + dp/dX) dX/dxi.
@@ -734,19 +792,28 @@ __global__ void __launch_bounds__(256)
   for (int k = 0; k < 9; k++) gps[k] = dgps[k] = 0.0;
   if constexpr (NC == 3) {
     double unused[NC];
-    if (P.shape != nullptr) interpolate(P.shape, unused, gps);
-    if constexpr (MODE == MODE_SHAPE_JVP) interpolate(P.dshape, unused, dgps);
+    if (P.shape != nullptr) {
+      gather(P.shape);
+      interpolate(unused, gps);
+    }
+    if constexpr (MODE == MODE_SHAPE_JVP) {
+      gather(P.dshape);
+      interpolate(unused, dgps);
+    }
   }
 
   // ---- quadrature point
   if (active) {
     double J[9], Ji[9];
     trilinear_jacobian(sxv + el * 24, sxw[i0], sxw[i1], sxw[i2], J);
+    if constexpr (NC == 3) {
 #pragma unroll
-    for (int k = 0; k < 9; k++) J[k] += gps[k];
+      for (int k = 0; k < 9; k++) J[k] += gps[k];
+    }
     inv3(J, Ji);
-    const double dJ = det3(J), wq = sxw[N + i0] * sxw[N + i1] * sxw[N + i2];
-    double       src[NC], fp[3 * NC];  // source and flux, times the quadrature weight
+    // rows carry the quadrature weight in the flux, a lane per result in its tables
+    const double dJ = det3(J), wq = ROWS ? sxw[N + i0] * sxw[N + i1] * sxw[N + i2] : 1.0;
+    double       src[NC], fp[3 * NC];  // source and flux
     if constexpr (MODE == MODE_SHAPE_JVP) {
       qpoint_shape_dir<QF, NC>(P.params, J, dgps, val, gp, st, src, fp);
 #pragma unroll
@@ -785,62 +852,87 @@ __global__ void __launch_bounds__(256)
       S0[c * NQ + li] = fp[c * 3 + 0];
       S1[c * NQ + li] = fp[c * 3 + 1];
       S2[c * NQ + li] = fp[c * 3 + 2];
-      if constexpr (HAS_SRC) S3[c * NQ + li] = src[c];
+      if constexpr (HAS_SRC) S0[(ROWS ? 3 : 6) * R + c * NQ + li] = src[c];
     }
   }
   lds_barrier();
 
-  // ---- integrate: x, y, z (the weights are in the flux)
-  for_rows<N, NC, 0>(li, active, [&](int o) {
-    double v[N], a[N];
-    read_row<N, 1>(S0 + o, v);
-    row_transposed<N>(tG, v, a);
-    if constexpr (HAS_SRC) {
-      read_row<N, 1>(S3 + o, v);
-      row_transposed<N>(tB, v, a, true);
-    }
-    write_row<N, 1>(S0 + o, a);
-    read_row<N, 1>(S1 + o, v);
-    row_transposed<N>(tB, v, a);
-    write_row<N, 1>(S1 + o, a);
-    read_row<N, 1>(S2 + o, v);
-    row_transposed<N>(tB, v, a);
-    write_row<N, 1>(S2 + o, a);
-  });
-  lds_barrier();
-  for_rows<N, NC, 1>(li, active, [&](int o) {
-    double v[N], a[N];
-    read_row<N, N>(S0 + o, v);
-    row_transposed<N>(tB, v, a);
-    read_row<N, N>(S1 + o, v);
-    row_transposed<N>(tG, v, a, true);
-    write_row<N, N>(S0 + o, a);
-    read_row<N, N>(S2 + o, v);
-    row_transposed<N>(tB, v, a);
-    write_row<N, N>(S1 + o, a);
-  });
-  lds_barrier();
-  for_rows<N, NC, 2>(li, active, [&](int o) {
-    double v[N], a[N];
-    read_row<N, NN>(S0 + o, v);
-    row_transposed<N>(tB, v, a);
-    read_row<N, NN>(S1 + o, v);
-    row_transposed<N>(tG, v, a, true);
-    write_row<N, NN>(S2 + o, a);
-  });
-  lds_barrier();
-
-  // ---- scatter-add: lane = node
+  // ---- integrate: x, y, z; lane = node in the end
   double acc[NC];
-  if (active) {
+  if constexpr (!ROWS) {
+    const int     oy = i2 * NN + i0, oz = i1 * N + i0;
+    const double *sB = stab + 2 * NN, *sG = stab + 3 * NN;
+    if (active) {
+      const double* row = S0 + li - i0;
+      double        a   = dot_result<N, N, 1>(sG + i0, row);
+      const double  b = dot_result<N, N, 1>(sB + i0, row + R), c = dot_result<N, N, 1>(sB + i0, row + 2 * R);
+      if constexpr (HAS_SRC) a += dot_result<N, N, 1>(sB + i0, row + 6 * R);
+      S3[li]          = a;
+      S3[NQ + li]     = b;
+      S3[2 * NQ + li] = c;
+    }
+    lds_barrier();
+    if (active) {
+      const double a = dot_result<N, N, N>(sB + i1, S3 + oy) + dot_result<N, N, N>(sG + i1, S3 + NQ + oy);
+      const double b = dot_result<N, N, N>(sB + i1, S3 + 2 * NQ + oy);
+      S0[li]         = a;
+      S1[li]         = b;
+    }
+    lds_barrier();
+    if (active) acc[0] = dot_result<N, N, NN>(sB + i2, S0 + oz) + dot_result<N, N, NN>(sG + i2, S1 + oz);
+  } else {
+    for_rows<N, NC, 0>(li, active, [&](int o) {
+      double v[N], a[N];
+      read_row<N, 1>(S0 + o, v);
+      row_transposed<N>(tG, v, a);
+      if constexpr (HAS_SRC) {
+        read_row<N, 1>(S3 + o, v);
+        row_transposed<N>(tB, v, a, true);
+      }
+      write_row<N, 1>(S0 + o, a);
+      read_row<N, 1>(S1 + o, v);
+      row_transposed<N>(tB, v, a);
+      write_row<N, 1>(S1 + o, a);
+      read_row<N, 1>(S2 + o, v);
+      row_transposed<N>(tB, v, a);
+      write_row<N, 1>(S2 + o, a);
+    });
+    lds_barrier();
+    for_rows<N, NC, 1>(li, active, [&](int o) {
+      double v[N], a[N];
+      read_row<N, N>(S0 + o, v);
+      row_transposed<N>(tB, v, a);
+      read_row<N, N>(S1 + o, v);
+      row_transposed<N>(tG, v, a, true);
+      write_row<N, N>(S0 + o, a);
+      read_row<N, N>(S2 + o, v);
+      row_transposed<N>(tB, v, a);
+      write_row<N, N>(S1 + o, a);
+    });
+    lds_barrier();
+    for_rows<N, NC, 2>(li, active, [&](int o) {
+      double v[N], a[N];
+      read_row<N, NN>(S0 + o, v);
+      row_transposed<N>(tB, v, a);
+      read_row<N, NN>(S1 + o, v);
+      row_transposed<N>(tG, v, a, true);
+      write_row<N, NN>(S2 + o, a);
+    });
+    lds_barrier();
+
+    if (active) {
 #pragma unroll
-    for (int c = 0; c < NC; c++) acc[c] = S2[c * NQ + li];
+      for (int c = 0; c < NC; c++) acc[c] = S2[c * NQ + li];
+    }
   }
+
+  // ---- scatter-add, through a region that the last stage did not read
+  constexpr int SV = ROWS ? 0 : 2 * R;
   if (P.scatter == SCATTER_ELEMENT) {
-    store_element<N, NC>(P.E, acc, S0, slot, li, active);
+    store_element<N, NC>(P.E, acc, S0 + SV, slot, li, active);
   } else if (P.ordered) {
-    scatter_element<N, NC, double, double>(r, acc, S0, smem + (el > 0 && el < EB ? el - 1 : 0) * PER, snode, el, EB,
-                                           node, li, active, P.nnodes, P.ordering, P.scatter, P.ordered == 2);
+    scatter_element<N, NC, double, double>(r, acc, S0 + SV, smem + (el > 0 && el < EB ? el - 1 : 0) * PER + SV, snode,
+                                           el, EB, node, li, active, P.nnodes, P.ordering, P.scatter, P.ordered == 2);
   } else if (active) {
 #pragma unroll
     for (int c = 0; c < NC; c++) scatter_add(r, lidx(node, c, NC, P.nnodes, P.ordering), acc[c], P.scatter);
@@ -1498,6 +1590,16 @@ struct DiagFields {
 // The contractions go by rows, all components at once and every field in its
 // place.  Neo-Hookean p = 3 on 48x40x44, FP64: 305 -> 248 us, of which the
 // tangent's bytes take 176.
+// One component has rows for some of the lanes only.  Rows and a lane per
+// result: heat p = 1 (80x79x81 elements) 62 and 69 us, p = 2 (48x47x49) 57 and
+// 61, p = 3 (36x35x37) 68 and 58, p = 4 (28x27x29) 62 and 69; mass-diffusion
+// with its ten fields 93 and 101, 84 and 76, 103 and 78, 101 and 97.
+template <int N, int NC, int NF>
+constexpr bool use_diag_rows()
+{
+  return NC > 1 || (N != 4 && (NF == 6 || N == 2));
+}
+
 template <int N, int NC, int LAYOUT, typename S>
 __global__ void __launch_bounds__(256) k_diagonal(const ElemLaunch P)
 {
@@ -1510,7 +1612,9 @@ __global__ void __launch_bounds__(256) k_diagonal(const ElemLaunch P)
   constexpr int NN = N * N;
   constexpr int R  = NC * NQ;  // one field, all components
   using Lay        = TangentLayout<S, Shape::DS, NQ>;
+  constexpr bool ROWS = use_diag_rows<N, NC, NF>();
   __shared__ double sf[EB * NF * R];
+  __shared__ double stab[ROWS ? 1 : 3 * NN];  // w B B, w G B, w G G
   __shared__ int    snode[EB * NQ];
 
   const int     tid    = threadIdx.x;
@@ -1519,6 +1623,8 @@ __global__ void __launch_bounds__(256) k_diagonal(const ElemLaunch P)
   const int64_t slot   = P.slot_begin + logical_block(P.xcd_remap) * EB + el;
   const bool    active = (el < EB) && (slot < P.slot_end);  // uniform over the element's lanes
   double*       sv     = sf + (el < EB ? el : 0) * NF * R;
+  if constexpr (!ROWS)
+    for (int k = tid; k < 3 * NN; k += blockDim.x) stab[k] = P.tables[4 * NN + 2 * N + k];
   const ScalarTable tab = (ScalarTable)(uintptr_t)P.tables + (4 * NN + 2 * N);  // w B B, w G B, w G G
 
   using raw        = typename StoreTraits<S>::raw;
@@ -1550,45 +1656,77 @@ __global__ void __launch_bounds__(256) k_diagonal(const ElemLaunch P)
   }
   const int64_t node = active ? int64_t(P.map[size_t(slot) * NQ + li]) : 0;
   lds_barrier();
-  for_rows<N, NC, 0>(li, active, [&](int o) {
-#pragma unroll
-    for (int f = 0; f < NF; f++) {
-      double v[N], a[N];
-      read_row<N, 1>(sv + f * R + o, v);
-      row_transposed<N>(tab + F::table(f, 0) * NN, v, a);
-      write_row<N, 1>(sv + f * R + o, a);
-    }
-  });
-  lds_barrier();
-  for_rows<N, NC, 1>(li, active, [&](int o) {
-#pragma unroll
-    for (int f = 0; f < NF; f++) {
-      double v[N], a[N];
-      read_row<N, N>(sv + f * R + o, v);
-      row_transposed<N>(tab + F::table(f, 1) * NN, v, a);
-      write_row<N, N>(sv + f * R + o, a);
-    }
-  });
-  lds_barrier();
-  for_rows<N, NC, 2>(li, active, [&](int o) {
-    double a[N];
-#pragma unroll
-    for (int i = 0; i < N; i++) a[i] = 0.0;
-#pragma unroll
-    for (int f = 0; f < NF; f++) {
-      double v[N];
-      read_row<N, NN>(sv + f * R + o, v);
-      row_transposed<N>(tab + F::table(f, 2) * NN, v, a, true);
-    }
-    write_row<N, NN>(sv + o, a);
-  });
-  lds_barrier();
-  // scatter (in address order as the J.v's) through the second field's place
   double acc[NC];
-  if (active) {
+  if constexpr (!ROWS) {
+    const int a0 = li % N, a1 = (li / N) % N, a2 = li / NN;
+    double    t[NF];
+    // a field's results take the place of its values once every lane has read them
+    auto put = [&] {
+      lds_barrier();
+      if (active) {
 #pragma unroll
-    for (int c = 0; c < NC; c++) acc[c] = sv[c * NQ + li];
+        for (int f = 0; f < NF; f++) sv[f * NQ + li] = t[f];
+      }
+      lds_barrier();
+    };
+    if (active) {
+#pragma unroll
+      for (int f = 0; f < NF; f++) t[f] = dot_result<N, N, 1>(stab + F::table(f, 0) * NN + a0, sv + f * NQ + li - a0);
+    }
+    put();
+    if (active) {
+#pragma unroll
+      for (int f = 0; f < NF; f++)
+        t[f] = dot_result<N, N, N>(stab + F::table(f, 1) * NN + a1, sv + f * NQ + a2 * NN + a0);
+    }
+    put();
+    if (active) {
+      acc[0] = 0.0;
+#pragma unroll
+      for (int f = 0; f < NF; f++)
+        acc[0] += dot_result<N, N, NN>(stab + F::table(f, 2) * NN + a2, sv + f * NQ + a1 * N + a0);
+    }
+    lds_barrier();  // the scatter below reuses the second field's place
+  } else {
+    for_rows<N, NC, 0>(li, active, [&](int o) {
+#pragma unroll
+      for (int f = 0; f < NF; f++) {
+        double v[N], a[N];
+        read_row<N, 1>(sv + f * R + o, v);
+        row_transposed<N>(tab + F::table(f, 0) * NN, v, a);
+        write_row<N, 1>(sv + f * R + o, a);
+      }
+    });
+    lds_barrier();
+    for_rows<N, NC, 1>(li, active, [&](int o) {
+#pragma unroll
+      for (int f = 0; f < NF; f++) {
+        double v[N], a[N];
+        read_row<N, N>(sv + f * R + o, v);
+        row_transposed<N>(tab + F::table(f, 1) * NN, v, a);
+        write_row<N, N>(sv + f * R + o, a);
+      }
+    });
+    lds_barrier();
+    for_rows<N, NC, 2>(li, active, [&](int o) {
+      double a[N];
+#pragma unroll
+      for (int i = 0; i < N; i++) a[i] = 0.0;
+#pragma unroll
+      for (int f = 0; f < NF; f++) {
+        double v[N];
+        read_row<N, NN>(sv + f * R + o, v);
+        row_transposed<N>(tab + F::table(f, 2) * NN, v, a, true);
+      }
+      write_row<N, NN>(sv + o, a);
+    });
+    lds_barrier();
+    if (active) {
+#pragma unroll
+      for (int c = 0; c < NC; c++) acc[c] = sv[c * NQ + li];
+    }
   }
+  // scatter (in address order as the J.v's) through the second field's place
   double* out = static_cast<double*>(P.r);
   if (P.scatter == SCATTER_ELEMENT) {
     store_element<N, NC>(P.E, acc, sv + R, slot, li, active);
