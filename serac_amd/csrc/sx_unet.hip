@@ -391,10 +391,11 @@ __global__ void __launch_bounds__(kThreads) k_conv_wgrad(WGradArgs A, int chunks
 // backward convolutions on the matrix cores
 // ---------------------------------------------------------------------------
 // The gradient g that arrives at a layer is FP32 and stays so: it is split into
-// three BF16 planes, g = hi + mid + lo (each the rounding of what the previous
-// ones leave, 8 significant bits a plane, so the sum is exact), and every
-// product of an activation or weight (BF16) with g becomes three BF16 products
-// accumulated in FP32.
+// three BF16 planes, g = hi + mid + lo, each the leading 8 significant bits of
+// what the previous ones leave, and every product of an activation or weight
+// (BF16) with g becomes three BF16 products accumulated in FP32.  The sum is g
+// itself for 2^-110 <= |g|, up to the largest float; below that the bits under
+// 2^-133, BF16's smallest number, are dropped.
 //
 // Both convolutions of the backward pass then run over a zero-padded grid,
 // flattened: with px = nx + 2 nodes in a padded row, the neighbour at tap
@@ -406,12 +407,17 @@ __global__ void __launch_bounds__(kThreads) k_conv_wgrad(WGradArgs A, int chunks
 // The channel-major arrays have kPadGuard(px, py) zeros before and after each
 // row, since o of a padding node reaches past the grid (its g is zero).
 
+// (cut off, not rounded: the planes of a number near the largest float stay
+// finite; an infinity or NaN is in the first plane alone, and NaN where the
+// padding's zeros meet it)
 __device__ __forceinline__ void split3(float g, uint16_t* out)
 {
-  out[0]         = f2bf(g);
-  const float r1 = g - bf2f(out[0]);
-  out[1]         = f2bf(r1);
-  out[2]         = f2bf(r1 - bf2f(out[1]));
+  const float hi = __uint_as_float(__float_as_uint(g) & 0xffff0000u), r1 = g - hi;
+  const float mid = __uint_as_float(__float_as_uint(r1) & 0xffff0000u), lo = r1 - mid;
+  const bool  finite = (__float_as_uint(g) & 0x7f800000u) != 0x7f800000u;
+  out[0] = finite ? uint16_t(__float_as_uint(hi) >> 16) : f2bf(g);
+  out[1] = finite ? uint16_t(__float_as_uint(mid) >> 16) : uint16_t(0);
+  out[2] = finite ? uint16_t(__float_as_uint(lo) >> 16) : uint16_t(0);
 }
 
 // padded coordinates of padded node v; false on the padding

@@ -77,3 +77,34 @@ def test_gradients_at_fp32_precision(gpu_lib, dims, relu, mfma):
             a, b = g[off:off + n], ref[off:off + n]
             assert np.linalg.norm(a - b) <= 2e-5 * np.linalg.norm(b), (k, n)
             off += n
+
+
+@pytest.mark.parametrize("mfma", [True, False])
+@pytest.mark.parametrize("through", ["weights", "data"])
+@pytest.mark.parametrize("g", [1e-33, 3e-20, 0.7, 3.39e38, 3.4e38])
+def test_one_gradient_value_over_the_float_range(gpu_lib, mfma, through, g):
+    """dL/dy is one number of FP32's range (the planes' sum is exact from 2^-110 up), everything else small powers of
+    two or zero: the head's weight gradients are that number at its 27 taps, or half of it reaches the layer below."""
+    dims = (9, 9, 9)
+    net = sx.UNet(*dims, seed=1)
+    net.set_activation(sx.capi.SX_UNET_IDENTITY, seed=1)
+    net.set_mfma(mfma)
+    offs = np.cumsum([0] + [n for ca, cb, co in sx.UNet.LAYERS for n in (27 * (ca + cb) * co, co)])
+    p = np.zeros(net.nparam, dtype=np.float32)
+    if through == "weights":
+        p[offs[21]] = 1.0  # layer 10's bias, channel 0: the head's input is 1, its output 0
+    else:
+        p[offs[22] + (13 * 16) * 3 + 1] = -0.5  # the head's centre weight, channel 0 -> 1; its input is 0
+    net.set_params(p)
+    t = np.zeros((net.nvox, 3), dtype=np.float32)
+    t[4 * 81 + 4 * 9 + 4, 1] = v = np.float32(2.0 / g)
+    net.backward(np.zeros((net.nvox, 3), dtype=np.float32), t)
+    want = np.float32(-np.float64(v) * (2.0 / (np.float64(v) * np.float64(v))))
+    assert abs(want / g + 1.0) < 1e-5
+    ref = np.zeros(net.nparam, dtype=np.float32)
+    ref[offs[23] + 1] = want
+    if through == "weights":
+        ref[offs[22]:offs[23]].reshape(27, 16, 3)[:, 0, 1] = want
+    else:
+        ref[offs[21]] = np.float32(-0.5) * want
+    assert np.array_equal(net.grads(), ref)
