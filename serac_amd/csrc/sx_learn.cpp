@@ -59,6 +59,18 @@ struct Buf {
     bytes = n;
     if (n) UN_HIP(hipMalloc(&p, n));
   }
+  // false where there is not enough memory
+  bool try_alloc(size_t n)
+  {
+    alloc(0);
+    if (hipMalloc(&p, n) != hipSuccess) {
+      (void)hipGetLastError();
+      p = nullptr;
+      return false;
+    }
+    bytes = n;
+    return true;
+  }
   template <typename T>
   T* as() const
   {
@@ -102,8 +114,9 @@ struct sx_unet {
   Buf xin;       // BF16 input [n0][3]
   Buf yout;      // FP32 output [n0][3]
   Buf wflip, tmp, sums;
-  // backward pass on the matrix cores: BF16 planes of a layer's gradient
-  // (channel-last and channel-major), its input channel-major, its weights
+  // backward pass on the matrix cores, allocated by the first one: BF16 planes
+  // of a layer's gradient (channel-last and channel-major), its input
+  // channel-major, its weights
   Buf gcl, gcm, xcm, wpl;
 
   int64_t cin(int k) const { return kLayers[k].cin_a + kLayers[k].cin_b; }
@@ -219,6 +232,31 @@ void weight_grad(sx_unet* N, int k, const void* xa, const void* xb, const float*
   UN_HIP(sxu::conv_wgrad(A, L.cout, false, N->stream));
 }
 
+// The work memory of the matrix-core backward pass (about 400 bytes per node of
+// the finest grid), which networks that are only evaluated do without; false
+// where there is not enough.
+bool backward_memory(sx_unet* N)
+{
+  if (N->wpl.p) return true;
+  size_t gcl = 0, gcm = 0, xcm = 0, wpl = 0;
+  for (int k = 0; k < 12; k++) {
+    const LayerDef&    L = kLayers[k];
+    const sxu::PadGrid P = sxu::pad_grid(N->dims[L.lin]);
+    gcl = std::max(gcl, sxu::planes_cl_elems(sxu::pad_grid(N->dims[L.lout]), L.cout));
+    gcm = std::max(gcm, size_t(P.row) * size_t(3 * L.cout));
+    xcm = std::max(xcm, size_t(P.row) * size_t(std::max(L.cin_a, L.cin_b)));
+    wpl = std::max(wpl, size_t(std::max(L.cin_a, L.cin_b)) * size_t(sxu::plane_kpad(L.cout)));
+  }
+  Buf* const   bufs[4]  = {&N->gcl, &N->gcm, &N->xcm, &N->wpl};
+  const size_t bytes[4] = {gcl * 2, gcm * 2, xcm * 2, wpl * 2};
+  for (int i = 0; i < 4; i++)
+    if (!bufs[i]->try_alloc(bytes[i])) {
+      for (Buf* b : bufs) b->alloc(0);
+      return false;
+    }
+  return true;
+}
+
 // The gradients of layer k from g = dL/d(its output) on the matrix cores: weights and bias into G, the data gradient
 // of the input's parts into da (channels cin_a) and db (channels cin_b) where not null
 void backward_layer_mfma(sx_unet* N, int k, const void* xa, const void* xb, const float* g, float* da, float* db)
@@ -250,17 +288,20 @@ void backward_layer_mfma(sx_unet* N, int k, const void* xa, const void* xb, cons
                            N->wpl.as<uint16_t>(), db, s));
 }
 
-// backward from dL/dy (in gact[11]); gradients accumulate into G
+// backward from dL/dy (in gact[11]); gradients accumulate into G.  On the matrix
+// cores where they are on and their work memory is there, on the vector units
+// otherwise.
 void backward(sx_unet* N)
 {
   hipStream_t s   = N->stream;
+  const bool mfma = N->use_mfma && backward_memory(N);
   auto        nel = [&](int k) { return N->nvox[kLayers[k].lout] * kLayers[k].cout; };
   // layer k: weight gradients, and the data gradients of its input parts into
   // da and db (null: none)
   auto layer = [&](int k, const void* xa, const void* xb, float* da, float* db) {
     const LayerDef& L = kLayers[k];
     float*          g = N->gact[k].as<float>();
-    if (N->use_mfma) {
+    if (mfma) {
       backward_layer_mfma(N, k, xa, xb, g, da, db);
       return;
     }
@@ -379,19 +420,6 @@ void init(sx_unet* N, int nx, int ny, int nz, uint64_t seed)
   N->wflip.alloc(size_t(wmax) * 2);
   N->tmp.alloc(size_t(tmax) * 4);
   N->sums.alloc(2 * sizeof(double));
-  size_t gcl = 0, gcm = 0, xcm = 0, wpl = 0;
-  for (int k = 0; k < 12; k++) {
-    const LayerDef&    L = kLayers[k];
-    const sxu::PadGrid P = sxu::pad_grid(N->dims[L.lin]);
-    gcl = std::max(gcl, sxu::planes_cl_elems(sxu::pad_grid(N->dims[L.lout]), L.cout));
-    gcm = std::max(gcm, size_t(P.row) * size_t(3 * L.cout));
-    xcm = std::max(xcm, size_t(P.row) * size_t(std::max(L.cin_a, L.cin_b)));
-    wpl = std::max(wpl, size_t(std::max(L.cin_a, L.cin_b)) * size_t(sxu::plane_kpad(L.cout)));
-  }
-  N->gcl.alloc(gcl * 2);
-  N->gcm.alloc(gcm * 2);
-  N->xcm.alloc(xcm * 2);
-  N->wpl.alloc(wpl * 2);
   UN_HIP(hipStreamCreateWithFlags(&N->stream, hipStreamNonBlocking));
 }
 

@@ -108,3 +108,22 @@ def test_one_gradient_value_over_the_float_range(gpu_lib, mfma, through, g):
     else:
         ref[offs[21]] = np.float32(-0.5) * want
     assert np.array_equal(net.grads(), ref)
+
+
+def test_work_memory_comes_with_the_first_matrix_core_backward(gpu_lib):
+    """65^3 nodes: networks that are evaluated, or trained on the vector units, go without its 109 MB."""
+    rng = np.random.default_rng(3)
+    net = sx.UNet(65, 65, 65, seed=1)
+    x = sx.DeviceVector.from_numpy(rng.standard_normal(net.nvox * 3), dtype=np.float32)
+    t = sx.DeviceVector.from_numpy(rng.standard_normal(net.nvox * 3), dtype=np.float32)
+    net.set_mfma(False)
+    free = []
+    for mfma in (False, True, True):
+        net.set_mfma(mfma)
+        net.forward(x)
+        free.append(torch.cuda.mem_get_info()[0])
+        net.backward(x, t)
+        free.append(torch.cuda.mem_get_info()[0])
+    assert abs(free[1] - free[0]) < 16 << 20 and abs(free[2] - free[1]) < 16 << 20
+    assert free[2] - free[3] > 80 << 20
+    assert abs(free[5] - free[3]) < 16 << 20
