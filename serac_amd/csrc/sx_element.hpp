@@ -1764,6 +1764,7 @@ struct AssembleTiles {
   static constexpr int T      = (N * N * N + 15) / 16;           // tiles per direction of the node pairs
   static constexpr int WAVES  = T * T < 4 ? T * T : 4;           // waves (tiles) per workgroup
   static constexpr int GROUPS = (T * T + WAVES - 1) / WAVES;     // workgroups per element
+  static constexpr int POINTS = (N * N * N + 3) / 4 * 4;         // four to a product
 };
 
 template <int N, int NC, int LAYOUT, typename S, bool STAGE>
@@ -1801,6 +1802,8 @@ __global__ void __launch_bounds__(64 * AssembleTiles<N>::WAVES, 2) k_assemble(co
       const int     q  = t < Lay::G * V * NQ ? gq % NQ : (t - Lay::G * V * NQ) % NQ;
       sD[q * DS + k]   = Dat(k, q);
     }
+    // the last group of four points: zeros in the place of points that are not there
+    for (int t = NQ * DS + threadIdx.x; t < Tiles::POINTS * DS; t += blockDim.x) sD[t] = 0.0;
   }
   for (int k = threadIdx.x; k < TAB; k += blockDim.x) stab[k] = P.tables[k];
   __syncthreads();
@@ -1833,15 +1836,11 @@ __global__ void __launch_bounds__(64 * AssembleTiles<N>::WAVES, 2) k_assemble(co
     double    tf[NS], uf[NS];
     basis(stab + 2 * N * N, stab + 3 * N * N, ic, qc, tf);
     basis(stab, stab + N * N, jc, qc, uf);
-    if (q >= NQ) {  // no such point: its products vanish whatever the tangent read in its place holds
-#pragma unroll
-      for (int a = 0; a < NS; a++) tf[a] = uf[a] = 0.0;
-    }
     auto D = [&](int row, int col) -> double {
       if constexpr (STAGE)
-        return sD[qc * DS + Shape::idx(row, col)];
+        return sD[q * DS + Shape::idx(row, col)];
       else
-        return Dat(Shape::idx(row, col), qc);
+        return q < NQ ? Dat(Shape::idx(row, col), q) : 0.0;
     };
     // input / output number of slot a of component c
     auto slot_of = [](int c, int a) { return VAL ? (a == 0 ? c : NC + c * 3 + a - 1) : c * 3 + a; };
@@ -1966,7 +1965,7 @@ inline int dispatch_gradient(const ElemLaunch& P, hipError_t* err)
     const int64_t n = P.slot_end - P.slot_begin;
     if (n <= 0) return 1;
     using Tiles            = AssembleTiles<N>;
-    constexpr size_t bytes = size_t(N * N * N) * TanShape<LAYOUT, NC>::DS * sizeof(double);
+    constexpr size_t bytes = size_t(Tiles::POINTS) * TanShape<LAYOUT, NC>::DS * sizeof(double);
     constexpr bool   stage = bytes <= 48 * 1024;
     hipLaunchKernelGGL((k_assemble<N, NC, LAYOUT, S, stage>), dim3(unsigned(n * Tiles::GROUPS)),
                        dim3(64 * Tiles::WAVES), stage ? bytes : 0, P.stream, P);

@@ -55,3 +55,15 @@ def test_assembled_entries(gpu_lib, name, p, ordering, scatter, tangent):
         d = np.concatenate([emap[e] * nc + c if ordering == 1 else c * gs.nnodes + emap[e] for c in range(nc)])
         K[np.ix_(d, d)] += of.element_matrix(0, e)
     assert np.abs(A.to_scipy().toarray() - K).max() < 1e-12 * np.abs(K).max()
+
+
+@pytest.mark.parametrize("p", [2, 4])
+def test_infinite_tangent_entries_stay_infinite(gpu_lib, p):
+    """27 and 125 points fill the last group of four with a point that is not there: its tangent must not count.  An
+    infinite mass: the middle node's function is positive at every point."""
+    space = sx.Space(sx.Mesh.cuboid(1, 1, 1), p, 1)
+    f = sx.Functional(space, [space])
+    f.add_domain_integral(sx.SX_QF_MASS_DIFFUSION, (np.inf, 0.0))
+    _, grad = f(0.0, sx.DeviceVector(space.ndof), wrt=0)
+    middle = space.element_nodes()[0, space.npe // 2]
+    assert grad.assemble().to_scipy()[middle, middle] == np.inf
