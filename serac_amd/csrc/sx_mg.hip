@@ -324,7 +324,9 @@ __global__ void __launch_bounds__(kThreads) k_coarsen_mask(const uint8_t* mf, Gr
 }
 
 // Level-0 smoothing steps.  t = J d has values on the essential rows, where
-// dinv is zero: r stays zero there.
+// dinv is zero: r stays zero there.  Elsewhere dinv = 1 / diag(J) is not zero,
+// also rounded to FP32, whose products overflow for a diagonal (7e44) that would
+// round it to zero: it stands for the mask that these steps then need not read.
 template <typename T>
 __global__ void __launch_bounds__(kThreads) k_cheb_init(const T* b, const T* dinv, double inv_theta, T* x, T* d, T* r,
                                                         int64_t n)

@@ -177,6 +177,25 @@ def test_levels_are_galerkin_products_and_the_vcycle_matches_numpy(gpu_lib, n, p
     assert np.abs(z.numpy() - zref).max() <= 1e-10 * np.abs(zref).max()
 
 
+@pytest.mark.parametrize("degrees", [(1, 1), (1, 2), (2, 1), (4, 3)])
+@pytest.mark.parametrize("n,p", [(4, 2), (8, 1)])
+def test_smoothing_degrees_match_numpy(gpu_lib, degrees, n, p):
+    """Degree 1 has no step after the first, which vertex levels otherwise leave half of to the step that follows."""
+    m, s, f, ess, grad = linearized(n, p)
+    mg = sx.Multigrid(s, fine_degree=degrees[0], coarse_degree=degrees[1], smoothing_range=10.0)
+    r = W.nodal_field(s.nnodes, 3, 7, 3000, -1.0, 1.0, 1)
+    # FP32 level-0 vectors: a few hundred roundings of 6e-8 on the way through
+    for vectors, tol in ((sx.capi.SX_PREC_F64, 1e-10), (sx.capi.SX_PREC_F32, 1e-4)):
+        mg.set_smoother_vectors(vectors)
+        mg.setup(grad, ess)
+        info = mg.info()
+        z = sx.DeviceVector(s.ndof)
+        mg.apply(sx.DeviceVector.from_numpy(r), z)
+        zref = vcycle_numpy(hierarchy(n, p, grad, ess, info), info, *degrees, 10.0, r, ess)
+        assert np.abs(z.numpy() - zref).max() <= tol * np.abs(zref).max()
+        assert np.array_equal(z.numpy()[ess], r[ess])
+
+
 @pytest.mark.parametrize("p,tprec", [(1, "f64"), (2, "f64"), (3, "f64"), (4, "f64"), (3, "f32"), (2, "f32")])
 def test_elementwise_vertex_operator_equals_the_probed_one(gpu_lib, p, tprec):
     n = 4
