@@ -88,15 +88,14 @@ struct TangentLayout {
   }
 };
 
-// packed index of the symmetric tangent: upper triangle, column-major, so a
-// forward-mode pass seeded at input s produces entries s(s+1)/2 .. s(s+1)/2+s
+// packed index of the symmetric tangent: upper triangle, column-major, the order
+// in which an integrand's tangent() emits: column s is s(s+1)/2 .. s(s+1)/2+s
 __host__ __device__ constexpr int packed_index(int r, int s) { return r <= s ? s * (s + 1) / 2 + r : r * (r + 1) / 2 + s; }
 
 // Shape of the stored tangent for a layout: M inputs/outputs per point
 // (VAL: the field value is an input and the source an output), DS stored
-// entries, and where entry D(r, s) = d out_r / d in_s lives.  Column s of a
-// forward-mode pass holds entries idx(r, s) for r < rows(s), in increasing
-// storage order.
+// entries, and where entry D(r, s) = d out_r / d in_s lives.  Column s holds
+// entries idx(r, s) for r < rows(s), in increasing storage order.
 template <int LAYOUT, int NC>
 struct TanShape {
   static constexpr bool VAL = (LAYOUT == LAYOUT_FULL_SYM);
@@ -503,7 +502,8 @@ __device__ __forceinline__ void store_tangent_entry(void* base, int q, int k, do
 // operands, no LDS reads.  With a lane per result instead, each result cost N
 // value reads and N table reads through the one LDS port of a CU.  Neo-Hookean
 // residual p = 2 on 57x48x43: 148 -> 120 us of kernel time; p = 3 on 64^3: 735
-// -> 682, two thirds of which FP64 instructions take (about 680 a point).
+// -> 682; its vector instructions (891 a point, 684 of them FP64) fill two thirds
+// of the cycles.
 // One component has N * N rows for N^3 lanes and stays with a lane per result
 // (use_rows): heat residual p = 3 on 36x35x37 elements 84 us by rows and 67 so,
 // p = 1 on 80x79x81 91 and 73 (both with the fill of the output).

@@ -131,10 +131,9 @@ __device__ __forceinline__ void gram(const double* Ji, double f, double* M)
 // linearization compute-bound (Neo-Hookean p = 3 on 48x40x44 elements: 1196
 // us of kernel time with the passes, 505 with the closed form, 330 for the
 // tangent's bytes alone; J2 p = 2 on 56x48x50: 1463, 672 and 400).
-// CONSTANT_TANGENT: it does not depend on the field.
-// HAS_SOURCE: the source output is nonzero; USES_VALUE: the
-// outputs depend on the field value (not only its gradient); SYMMETRIC: the
-// tangent is major-symmetric, so half of it is stored.
+// CONSTANT_TANGENT: it does not depend on the field.  HAS_SOURCE: the source
+// output is nonzero; USES_VALUE: the outputs depend on the field value (not only
+// its gradient).
 // ---------------------------------------------------------------------------
 
 // steady heat conduction: ThermalMaterialIntegrand<LinearIsotropicConductor>
