@@ -128,8 +128,9 @@ def test_j2_state_commit_matches_oracle(gpu_lib, scatter):
 
 
 def test_j2_domain_subset_state_rows_follow_domain_order(gpu_lib):
-    # a domain listed out of element order, with coloured scatter (slots are
-    # permuted by colour): state rows must stay in domain order
+    # a domain listed out of element order: state rows must stay in domain order
+    # (the node sum keeps slots in that order too; slots that launches permute by
+    # colour are those of test_j2_state_of_repeated_elements)
     elems = [13, 2, 7, 26, 0, 14, 5, 20, 9]
     pr = J2Pair(3, 2, J2_PARAMS["c4"], elems=elems, state_seed=8)
     U = pr.shear_field(0.015, 1e-3, 14)
